@@ -165,7 +165,8 @@ def nsm_run(spec, seed: int, replicate: int, budget_s: float):
 
 # Kernels of the default whole-cell step, by rocprofv3 kernel name prefix.
 TRAFFIC_KERNELS = {"sweep_x": "void lmx::sweep_x4_kernel<2>", "sweep_y": "void lmx::sweep_tile_kernel<2, false>",
-                   "sweep_z": "void lmx::sweep_tile_kernel<2, true>", "reaction": "void lmx::reaction_list_kernel<2>"}
+                   "sweep_z": "void lmx::sweep_tile_kernel<2, true>", "reaction": "void lmx::reaction_list_kernel<2>",
+                   "fused": "void lmx::box_step_kernel<lmx::ByteSites<2>, 768, true"}
 
 
 def counter_means(path: str, counter: str) -> dict:
@@ -541,8 +542,10 @@ def main() -> int:
     N, P, K = spec.N, spec.P, args.steps
     value = N * K / (total_ms / 1e3)
     tile_list = tuned is None or (tuned["path"] == 0 and tuned["yz_kernel"] == 0 and tuned["fuse_reaction"])
-    listed = args.path == "sweeps" and uses_reaction_list(spec) and tile_list
-    path = "fused" if args.path == "fused" or (tuned and tuned["path"] == 1) else "sweeps"
+    # the default step: one launch over boxes, the reactions of the few candidate sites, the resolver
+    boxed = "fused" in per and args.path != "fused" and not (tuned and tuned["path"] == 1)
+    listed = args.path == "sweeps" and uses_reaction_list(spec) and tile_list and not boxed
+    path = "boxes" if boxed else ("fused" if "fused" in per else "sweeps")
     list_bytes = occupied * list_entry_bytes(P) if listed else 0
     # per-kernel averages and algorithmic bytes per launch (with the reaction
     # list, the z sweep also writes one entry per occupied site and the
@@ -551,7 +554,7 @@ def main() -> int:
     for name, (ms, launches) in per.items():
         if name.startswith("sweep") or name == "fused":
             b = sweep_bytes_per_site(P) * N + (list_bytes if name == "sweep_z" else 0)
-        elif name == "reaction":
+        elif name == "reaction" and not boxed:
             b = list_bytes if listed else reaction_bytes_per_site(P) * N
         else:
             b = 0
@@ -573,10 +576,12 @@ def main() -> int:
                 # algorithmic rate where the kernels skip the zero upper planes of packed sites
                 "traffic_GBps": (traffic / (dk["avg_us"] / 1e6) / 1e9) if traffic else None,
                 "traffic_source": traffic_note}
-    # Bytes of the step as run: three sweeps plus the reaction list (written
-    # and read once), or plus the full reaction read.
+    # Bytes of the step as run: the lattice once (boxes), or three sweeps plus
+    # the reaction list (written and read once), or plus the full reaction read.
     unfused_alg = (3 * sweep_bytes_per_site(P) + (reaction_bytes_per_site(P) if spec.R else 0)) * N
     step_alg = 3 * sweep_bytes_per_site(P) * N + 2 * list_bytes if listed else unfused_alg
+    if path != "sweeps":
+        step_alg = sweep_bytes_per_site(P) * N
     step_ms = total_ms / K
     out = {
         "metric": "site-steps/s & % HBM roofline; ensemble sims/hr, p50/p99 latency vs plain",
@@ -595,7 +600,7 @@ def main() -> int:
                    "sites": N, "slots_per_site": P, "species": spec.nS, "reactions": spec.R,
                    "site_types": spec.nST, "particles": int(spec.initial_counts().sum()),
                    "lambda_m": spec.spacing, "tau_s": spec.tau, "path": path,
-                   "reaction_phase": "list" if listed else "full pass", "occupied_sites_end": occupied},
+                   "reaction_phase": "candidates" if boxed else ("list" if listed else "full pass"), "occupied_sites_end": occupied},
         "roofline": roofline,
         "step_roofline": {"alg_bytes_per_step": step_alg, "achieved_GBps": step_alg / (step_ms / 1e3) / 1e9,
                           "frac": step_alg / (step_ms / 1e3) / 1e9 / HBM_PEAK_GBS,

@@ -53,7 +53,8 @@ enum lmx_boundary { LMX_BOUNDARY_PERIODIC = 0, LMX_BOUNDARY_REFLECTING = 1 };
 
 /* Step implementations.  Every one gives bit-identical lattices. */
 enum lmx_path {
-    LMX_PATH_SWEEPS = 0,   /* x, y, z sweep kernels + reaction kernel + resolver */
+    LMX_PATH_SWEEPS = 0,   /* the boxed step (LMX_OPT_BOXES), or x, y, z sweep kernels + reaction
+                            * kernel, + resolver */
     LMX_PATH_FUSED = 1     /* one fused diffuse+react kernel per step + resolver */
 };
 
@@ -147,10 +148,16 @@ int lmx_set_path(lmx_solver *s, int path);
  *                          words, and the reaction phase evaluates only the
  *                          listed sites (models without zero-order
  *                          reactions; a full list falls back to the full
- *                          pass); 0 = full reaction kernel */
+ *                          pass); 0 = full reaction kernel
+ *   LMX_OPT_BOXES          1 (default) = on the sweeps path, with the other
+ *                          options at their defaults, a step is one launch
+ *                          over boxes of the lattice, whose work goes with
+ *                          the particles instead of the sites, wherever the
+ *                          particles of a box fit a block (up to about one
+ *                          per site); 0 = the separate sweeps */
 enum lmx_option {
     LMX_OPT_MARCH_SEGMENT = 1, LMX_OPT_FORCE_GENERIC = 2, LMX_OPT_YZ_KERNEL = 3, LMX_OPT_FUSED_ZSEG = 4,
-    LMX_OPT_FUSE_REACTION = 5
+    LMX_OPT_FUSE_REACTION = 5, LMX_OPT_BOXES = 6
 };
 int lmx_set_launch_option(lmx_solver *s, int option, int value);
 

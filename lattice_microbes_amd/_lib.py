@@ -34,6 +34,7 @@ OPT_FORCE_GENERIC = 2
 OPT_YZ_KERNEL = 3
 OPT_FUSED_ZSEG = 4
 OPT_FUSE_REACTION = 5
+OPT_BOXES = 6
 BATCH_GRAPH = 1
 BATCH_REACTION_LIST = 2
 BATCH_TILE_THREADS = 3

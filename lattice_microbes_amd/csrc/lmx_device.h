@@ -32,7 +32,7 @@ struct Control {
     // Relaxed handler: entries whose own site was full at the end of a step,
     // in list order, retried after the next step before its own entries.
     uint32_t carry_count;
-    uint32_t carry_pad;
+    uint32_t box_splits;        // boxes of the boxed step that needed smaller boxes, since the host last looked
     unsigned long long ovf_keys[kMaxOverflows];
     uint32_t ovf_part[kMaxOverflows];   // the particle of list entry k
     uint32_t carry_site[kMaxOverflows];
@@ -98,6 +98,12 @@ struct Params {
     const uint8_t *RL;          // [R][nST]
     const uint8_t *sites;       // [N]
     Control *ctl;
+    // Boxed step: the zero flags of the buffer a step writes ([W][boxes], 1
+    // while that plane of that box is known all zero), and the boxes' extents;
+    // the resolver clears the flag of a box it places a particle in.  Null on
+    // the other paths.
+    uint32_t *zero_flags;
+    uint32_t box_x, box_y, box_z, box_nx, box_ny, box_n;
 };
 
 // ---------------------------------------------------------------------------
@@ -290,6 +296,16 @@ __device__ inline void clear_chunk_flag(const Params &p, uint32_t *lat, uint32_t
     uint32_t *f = chunk_flag(p, lat, k, g);
     if (__hip_atomic_load(f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u)
         __hip_atomic_store(f, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Clears the zero flag of site i's box in plane k (boxed step) after a
+// nonzero write.
+__device__ inline void clear_zero_flag(const Params &p, uint32_t k, uint32_t i)
+{
+    if (!p.zero_flags) return;
+    const uint32_t z = i / p.XY, r = i - z * p.XY, y = r / p.X, x = r - y * p.X;
+    const uint32_t box = x / p.box_x + p.box_nx * (y / p.box_y + p.box_ny * (z / p.box_z));
+    __hip_atomic_store(p.zero_flags + (size_t)k * p.box_n + box, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // One particle per 32-bit word (the uint32 lattice of IntMpdRdmeSolver):

@@ -11,6 +11,7 @@ namespace lmx {
 
 struct Params;
 struct Member;
+struct BoxGeom;
 
 hipError_t launch_sweep(const Params &p, const uint32_t *src, uint32_t *dst, int axis, hipStream_t st);
 hipError_t launch_reaction(const Params &p, uint32_t *lat, hipStream_t st);
@@ -38,6 +39,13 @@ uint32_t fused_tile_rows(uint32_t X, uint32_t W);
 hipError_t launch_fused(const Params &p, const uint32_t *src, uint32_t *dst, uint32_t zseg, hipStream_t st);
 hipError_t launch_reaction_fast(const Params &p, uint32_t *lat, hipStream_t st);
 hipError_t launch_prob_tables(const Params &p, float *prob1, float *prob0, hipStream_t st);
+// The boxed step (mpd_box.hip): one timestep from src to dst without the
+// reactions (launch_box_reactions) and the resolver.  zs and zd are the zero flags of the two buffers, rl the
+// reaction candidates (any capacity is correct).
+struct CandList;
+hipError_t launch_box_step(const Params &p, const BoxGeom &g, const uint32_t *src, uint32_t *dst, const uint32_t *zs,
+                           uint32_t *zd, const CandList &rl, hipStream_t st);
+hipError_t launch_box_reactions(const Params &p, uint32_t *lat, const CandList &rl, hipStream_t st);
 uint32_t x4_blocks(const Params &p);
 uint32_t reaction_blocks(const Params &p);
 struct TileGeom;

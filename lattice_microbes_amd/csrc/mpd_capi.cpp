@@ -18,6 +18,7 @@
 #include <vector>
 
 #include "lmx_batch.h"
+#include "lmx_box.h"
 #include "lmx_device.h"
 #include "lmx_kernels.h"
 
@@ -140,6 +141,15 @@ struct lmx_solver {
     bool fuse_reaction = true;  // the tiled z sweep lists its occupied output sites for the reaction phase
     uint4 *d_rl = nullptr;      // the reaction list: one record of list_units(W) 16-byte units per entry
     lmx::ReactionList rlist{};
+    // The boxed step (LMX_OPT_BOXES): its boxes, the level they were taken
+    // from (kBoxLevels: too crowded, the sweeps run) and the zero flags of
+    // both buffers (buf * W * nboxes), valid while zflags_fresh.
+    bool boxes = true;
+    lmx::BoxGeom box{};
+    uint32_t box_level = lmx::kBoxLevels;
+    uint32_t splits_seen = 0, splits_step = 0;  // Control::box_splits and the step when it was last looked at
+    uint32_t *d_zflags = nullptr;
+    bool zflags_fresh = false;
     uint32_t num_cu = 256;
 };
 
@@ -249,6 +259,9 @@ lmx::Params make_params(const lmx_solver *s)
     p.sto_val = s->d_sto_val;
     p.sites = s->d_sites;
     p.ctl = s->d_ctl;
+    p.zero_flags = nullptr;
+    p.box_x = lmx::kBoxX; p.box_y = s->box.TY; p.box_z = s->box.TZ;
+    p.box_nx = s->box.nbx; p.box_ny = s->box.nby; p.box_n = s->box.nboxes;
     return p;
 }
 
@@ -263,28 +276,40 @@ int require_ready(lmx_solver *s)
 // the first empty slot of its site (RDMESolver::setLatticeData + addParticle;
 // IntLattice::setFromRowMajorData for the uint32 lattice).  rm holds N*P
 // elements of bpp bytes.
-int row_major_to_native(const lmx_solver *s, const void *rm, std::vector<uint32_t> &native)
+// at, if given, receives the native site index of every particle, as long as
+// there are at most N (see plan_boxes).
+int row_major_to_native(const lmx_solver *s, const void *rm, std::vector<uint32_t> &native,
+                        std::vector<uint32_t> *at = nullptr)
 {
     const size_t N = s->N;
     const bool words = s->bpp == 4;
     const uint8_t *rb = static_cast<const uint8_t *>(rm);
     const uint32_t *rw = static_cast<const uint32_t *>(rm);
     native.assign(N * s->W, 0u);
-    std::vector<uint8_t> fill(N, 0);
     size_t idx = 0;
     for (uint32_t x = 0; x < s->X; x++)
         for (uint32_t y = 0; y < s->Y; y++)
-            for (uint32_t z = 0; z < s->Z; z++) {
+            for (uint32_t z = 0; z < s->Z; z++, idx += s->P) {
                 const size_t i = (size_t)x + (size_t)s->X * y + (size_t)s->X * s->Y * z;
-                for (uint32_t l = 0; l < s->P; l++, idx++) {
-                    const uint32_t v = words ? rw[idx] : rb[idx];
+                uint32_t j = 0;  // the site's next slot
+                for (uint32_t l = 0; l < s->P; l++) {
+                    if (!words && (l & 3u) == 0) {  // four empty slots at once: most sites are empty
+                        uint32_t q;
+                        memcpy(&q, rb + idx + l, sizeof(q));
+                        if (q == 0) {
+                            l += 3;
+                            continue;
+                        }
+                    }
+                    const uint32_t v = words ? rw[idx + l] : rb[idx + l];
                     if (v == 0) continue;
                     if (v > s->nS) return fail(LMX_ERR_ARG, "latticeData: an invalid species was found: " + std::to_string(v));
-                    const uint32_t j = fill[i]++;
+                    if (at && at->size() <= N) at->push_back((uint32_t)i);
                     if (words)
                         native[(size_t)j * N + i] = v;
                     else
                         native[(size_t)(j >> 2) * N + i] |= v << (8 * (j & 3));
+                    j++;
                 }
             }
     return LMX_OK;
@@ -323,10 +348,54 @@ int sites_row_major_to_native(const lmx_solver *s, const uint8_t *rm, std::vecto
     return LMX_OK;
 }
 
+void set_box_level(lmx_solver *s, uint32_t level)
+{
+    s->box_level = level;
+    if (level < lmx::kBoxLevels) s->box = lmx::box_geom(s->X, s->Y, s->Z, lmx::kBoxLevel[level]);
+    s->zflags_fresh = false;
+}
+
+// The boxes for a lattice with particles at the given sites: the largest whose
+// fullest region, scaled from the fullest box, takes at most 3/4 of the
+// records a block holds.  A region that holds more is halved by its block, at
+// several times the cost, so the rule leaves room for fluctuations; on the
+// 128x64x80 bimolecular lattice (P = 8) the sweeps take 26-64 us a step from
+// 0.01 to 0.4 particles a site, the boxes that fit 18-38 us.
+void plan_boxes(lmx_solver *s, const std::vector<uint32_t> &at)
+{
+    const uint32_t cap = (uint32_t)lmx::box_cap(s->P);
+    if (at.size() > s->N) return set_box_level(s, lmx::kBoxLevels);  // more than a particle a site: no box fits
+    std::vector<uint32_t> n, ybox(s->Y), zbox(s->Z);
+    for (uint32_t level = 0; level < lmx::kBoxLevels; level++) {
+        const lmx::BoxGeom g = lmx::box_geom(s->X, s->Y, s->Z, lmx::kBoxLevel[level]);
+        const double region = (double)(lmx::kBoxX + 2) * (g.TY + 2) * (g.TZ + 2) / ((double)lmx::kBoxX * g.TY * g.TZ);
+        const double most = 0.75 * cap / region;
+        if ((double)at.size() > most * g.nboxes) continue;  // the mean box is too full already
+        for (uint32_t y = 0; y < s->Y; y++) ybox[y] = g.nbx * (y / g.TY);
+        for (uint32_t z = 0; z < s->Z; z++) zbox[z] = g.nbx * g.nby * (z / g.TZ);
+        n.assign(g.nboxes, 0u);
+        uint32_t full = 0;
+        for (uint32_t i : at) {
+            const uint32_t r = i / s->X, z = r / s->Y;
+            full = std::max(full, ++n[(i - r * s->X) / lmx::kBoxX + ybox[r - z * s->Y] + zbox[z]]);
+        }
+        if (full <= most) return set_box_level(s, level);
+    }
+    set_box_level(s, lmx::kBoxLevels);
+}
+
 int check_device_error(lmx_solver *s)
 {
-    uint32_t hdr[4];
+    uint32_t hdr[offsetof(lmx::Control, box_splits) / sizeof(uint32_t) + 1];
     LMX_HIP(hipMemcpy(hdr, s->d_ctl, sizeof(hdr), hipMemcpyDeviceToHost));
+    // Many boxes had to be halved since the last look (the lattice became
+    // more crowded): smaller boxes from now on.
+    const uint32_t splits = hdr[offsetof(lmx::Control, box_splits) / sizeof(uint32_t)] - s->splits_seen;
+    if (s->diffusion_built && s->box_level < lmx::kBoxLevels && s->timestep > s->splits_step &&
+        splits > (s->timestep - s->splits_step) * (1u + s->box.nboxes / 256u))
+        set_box_level(s, s->box_level + 1);
+    s->splits_seen += splits;
+    s->splits_step = s->timestep;
     switch (hdr[2]) {
     case 0: return LMX_OK;
     case lmx::kErrOverflowCap:
@@ -356,6 +425,14 @@ uint32_t fused_zseg(lmx_solver *s)
     return (s->Z + nzs - 1) / nzs;
 }
 
+// The boxed step runs by default wherever the particles fit its boxes; the
+// launch options of the sweeps select those instead.
+bool use_boxes(const lmx_solver *s)
+{
+    return s->boxes && s->box_level < lmx::kBoxLevels && s->path == LMX_PATH_SWEEPS && s->yz_kernel == 0 && s->fuse_reaction &&
+           !s->force_generic;
+}
+
 // One timestep (runTimestep, MpdRdmeSolver.cu:996-1193).  ev, if given,
 // receives events around each launch (ev[0] before the first launch, then one
 // after every launch); kinds receives the kernel class of each launch.
@@ -381,6 +458,41 @@ int enqueue_step(lmx_solver *s, const lmx::Params &p0, hipEvent_t *ev, int *kind
         return LMX_OK;
     };
     const bool fast = !s->force_generic && lmx::fast_path_ok(p);
+    if (use_boxes(s)) {
+        const size_t nz = (size_t)s->W * s->box.nboxes;
+        if (!s->zflags_fresh) {
+            e = lmx::launch_fill(s->d_zflags, 2 * nz, 0u, s->stream);
+            if (e != hipSuccess) return hip_fail(e, "zero flag fill launch");
+            s->zflags_fresh = true;
+        }
+        s->flags_fresh = false;
+        p.plane_flags = 0u;
+        uint32_t *zs = s->d_zflags + s->cur * nz, *zd = s->d_zflags + (1 - s->cur) * nz;
+        p.zero_flags = zd;
+        if (ev) {
+            e = hipEventRecord(ev[0], s->stream);
+            if (e != hipSuccess) return hip_fail(e, "hipEventRecord");
+        }
+        // the reaction list's memory holds the candidates: four site indices a unit
+        const lmx::CandList cand{reinterpret_cast<uint32_t *>(rlist.rec), rlist.cap * 4u};
+        e = lmx::launch_box_step(p, s->box, s->d_lat[s->cur], s->d_lat[1 - s->cur], zs, zd, cand, s->stream);
+        if (e != hipSuccess) return hip_fail(e, "boxed step launch");
+        s->cur = 1 - s->cur;
+        if (int rc = mark(LMX_K_FUSED)) return rc;
+        if (s->R > 0) {
+            e = lmx::launch_box_reactions(p, s->d_lat[s->cur], cand, s->stream);
+            if (e != hipSuccess) return hip_fail(e, "reaction launch");
+            if (int rc = mark(LMX_K_REACTION)) return rc;
+        }
+        e = lmx::launch_resolve(p, s->d_lat[s->cur], s->stream);
+        if (e != hipSuccess) return hip_fail(e, "resolve launch");
+        if (int rc = mark(LMX_K_RESOLVE)) return rc;
+        if (nlaunch) *nlaunch = n;
+        s->timestep++;
+        s->packed = true;
+        return LMX_OK;
+    }
+    s->zflags_fresh = false;
     // Chunk flags: kept by the default sweeps-path kernels of the byte
     // lattice (x4, LDS tiles, the reaction phases, the resolver); any other
     // step leaves them stale, so they are zeroed before the next step that
@@ -463,6 +575,8 @@ void free_device(lmx_solver *s)
     dev_free(s->d_lat[1]);
     dev_free(s->d_sites);
     dev_free(s->d_rl);
+    dev_free(s->d_zflags);
+    s->zflags_fresh = false;
     s->rlist = lmx::ReactionList{};
     dev_free(s->d_T);
     dev_free(s->d_qp0);
@@ -691,8 +805,8 @@ int lmx_build_diffusion_model(lmx_solver *s, uint32_t nST, const double *DF, con
             if (q > 0.50f) return fail(LMX_ERR_ARG, "D: The specified diffusion coefficient is too high for the diffusion model.");
             s->T[i] = q;
         }
-        std::vector<uint32_t> native;
-        if ((rc = row_major_to_native(s, lattice, native))) return rc;
+        std::vector<uint32_t> native, at;
+        if ((rc = row_major_to_native(s, lattice, native, &at))) return rc;
         std::vector<uint8_t> nsites;
         if ((rc = sites_row_major_to_native(s, sites, nsites))) return rc;
         compute_propensities(s);
@@ -718,8 +832,11 @@ int lmx_build_diffusion_model(lmx_solver *s, uint32_t nST, const double *DF, con
         // site up to 12.5% occupancy.
         const size_t rcap = std::max<size_t>(64, (s->N / 8 + lmx::kListShards - 1) / lmx::kListShards);
         const size_t rtotal = rcap * lmx::kListShards;
-        // (the byte lattice's vector kernels only)
-        if (e == hipSuccess && s->bpp == 1) e = hipMalloc((void **)&s->d_rl, rtotal * lmx::list_units(s->W) * sizeof(uint4));
+        if (e == hipSuccess) e = hipMalloc((void **)&s->d_rl, rtotal * (s->bpp == 1 ? lmx::list_units(s->W) : 1) * sizeof(uint4));
+        // zero flags for the smallest boxes
+        if (e == hipSuccess)
+            e = hipMalloc((void **)&s->d_zflags, 2 * (size_t)s->W * sizeof(uint32_t) *
+                              lmx::box_geom(X, Y, Z, lmx::kBoxLevel[lmx::kBoxLevels - 1]).nboxes);
         if (e == hipSuccess && s->d_rl) {
             s->rlist.rec = s->d_rl;
             s->rlist.cap = (uint32_t)rcap;
@@ -769,6 +886,8 @@ int lmx_build_diffusion_model(lmx_solver *s, uint32_t nST, const double *DF, con
         if ((rc = upload_tables(s))) return rc;
         LMX_HIP(hipMemset(s->d_ctl, 0, sizeof(lmx::Control)));
         s->timestep = 0;
+        s->splits_seen = s->splits_step = 0;
+        plan_boxes(s, at);
         s->packed = true;  // row_major_to_native fills each site's first slots
         s->diffusion_built = true;
         return LMX_OK;
@@ -811,6 +930,9 @@ int lmx_set_launch_option(lmx_solver *s, int option, int value)
                         "y/z kernel must be 0 (LDS tiles), 1 (march), 2 (compacted tiles) or 3 (register columns)");
         s->yz_kernel = value;
         return LMX_OK;
+    case LMX_OPT_BOXES:
+        s->boxes = value != 0;
+        return LMX_OK;
     case LMX_OPT_FUSE_REACTION:
         s->fuse_reaction = value != 0;
         return LMX_OK;
@@ -848,8 +970,8 @@ int lmx_run_steps_static(lmx_solver *s, uint32_t nsteps)
         return fail(LMX_ERR_STATE, "lmx_run_steps_static: reaction rates changed since the tables were uploaded; "
                                    "lmx_run_steps uploads them (it allocates)");
     lmx::ReactionList rl{};
-    if (s->bpp == 1) {
-        const hipError_t e = lmx::static_reaction_list(s->device, s->W, &rl);
+    {
+        const hipError_t e = lmx::static_reaction_list(s->device, s->bpp == 1 ? s->W : 1, &rl);
         if (e != hipSuccess) return hip_fail(e, "static reaction list");
     }
     const lmx::Params p = make_params(s);
@@ -928,38 +1050,48 @@ int lmx_get_sites(lmx_solver *s, uint8_t *rm, size_t size)
 
 int lmx_set_lattice_native(lmx_solver *s, const uint32_t *native, size_t words)
 {
-    int rc = require_ready(s);
-    if (rc) return rc;
-    if (!native || words != s->N * s->W) return fail(LMX_ERR_ARG, "the buffer size was not equal to the lattice data size");
-    for (size_t i = 0; i < words; i++) {
-        if (s->bpp == 4) {
-            if (native[i] > s->nS) return fail(LMX_ERR_ARG, "latticeData: an invalid species was found");
-            continue;
+    return guarded([&]() -> int {
+        int rc = require_ready(s);
+        if (rc) return rc;
+        if (!native || words != s->N * s->W) return fail(LMX_ERR_ARG, "the buffer size was not equal to the lattice data size");
+        for (size_t i = 0; i < words; i++) {
+            if (s->bpp == 4) {
+                if (native[i] > s->nS) return fail(LMX_ERR_ARG, "latticeData: an invalid species was found");
+                continue;
+            }
+            for (int b = 0; b < 4; b++)
+                if (((native[i] >> (8 * b)) & 0xFFu) > s->nS)
+                    return fail(LMX_ERR_ARG, "latticeData: an invalid species was found");
         }
-        for (int b = 0; b < 4; b++)
-            if (((native[i] >> (8 * b)) & 0xFFu) > s->nS)
-                return fail(LMX_ERR_ARG, "latticeData: an invalid species was found");
-    }
-    // Whether every site holds its particles in its first slots.
-    bool packed = true;
-    for (size_t i = 0; i < s->N && packed; i++) {
-        bool gap = false;
-        for (uint32_t j = 0; j < s->P; j++) {
-            const uint32_t v = s->bpp == 4 ? native[(size_t)j * s->N + i]
-                                           : (native[(size_t)(j >> 2) * s->N + i] >> (8 * (j & 3))) & 0xFFu;
-            if (v == 0) {
-                gap = true;
-            } else if (gap) {
-                packed = false;
-                break;
+        // Where the particles are, and whether every site holds its particles in
+        // its first slots.
+        bool packed = true;
+        std::vector<uint32_t> at;
+        for (size_t i = 0; i < s->N; i++) {
+            bool gap = false;
+            for (uint32_t j = 0; j < s->P; j++) {
+                const uint32_t word = s->bpp == 4 ? native[(size_t)j * s->N + i] : native[(size_t)(j >> 2) * s->N + i];
+                if (word == 0 && s->bpp == 1) {  // four empty slots
+                    gap = true;
+                    j |= 3u;
+                    continue;
+                }
+                const uint32_t v = s->bpp == 4 ? word : (word >> (8 * (j & 3))) & 0xFFu;
+                if (v == 0) {
+                    gap = true;
+                } else {
+                    if (gap) packed = false;
+                    if (at.size() <= s->N) at.push_back((uint32_t)i);
+                }
             }
         }
-    }
-    LMX_HIP(hipStreamSynchronize(s->stream));
-    LMX_HIP(hipMemcpy(s->d_lat[s->cur], native, words * sizeof(uint32_t), hipMemcpyHostToDevice));
-    s->packed = packed;
-    s->flags_fresh = false;
-    return LMX_OK;
+        LMX_HIP(hipStreamSynchronize(s->stream));
+        LMX_HIP(hipMemcpy(s->d_lat[s->cur], native, words * sizeof(uint32_t), hipMemcpyHostToDevice));
+        s->packed = packed;
+        s->flags_fresh = false;
+        plan_boxes(s, at);
+        return LMX_OK;
+    });
 }
 
 int lmx_device_lattice(lmx_solver *s, void **particles, void **sites)
@@ -973,6 +1105,7 @@ int lmx_device_lattice(lmx_solver *s, void **particles, void **sites)
     *sites = s->d_sites;
     s->packed = false;  // the caller may write any slot
     s->flags_fresh = false;
+    s->zflags_fresh = false;
     return LMX_OK;
 }
 
@@ -993,12 +1126,13 @@ int lmx_set_lattice(lmx_solver *s, const uint8_t *rm, size_t size)
         int rc = require_ready(s);
         if (rc) return rc;
         if (!rm || size != s->N * s->P * s->bpp) return fail(LMX_ERR_ARG, "bufferSize: the buffer size was not equal to the lattice data size");
-        std::vector<uint32_t> native;
-        if ((rc = row_major_to_native(s, rm, native))) return rc;
+        std::vector<uint32_t> native, at;
+        if ((rc = row_major_to_native(s, rm, native, &at))) return rc;
         LMX_HIP(hipStreamSynchronize(s->stream));
         LMX_HIP(hipMemcpy(s->d_lat[s->cur], native.data(), native.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
         s->packed = true;  // each site's particles inserted at its first empty slot
         s->flags_fresh = false;
+        plan_boxes(s, at);
         return LMX_OK;
     });
 }
@@ -1096,22 +1230,25 @@ int lmx_autotune(lmx_solver *s, uint32_t nsteps, double *best_ms, int *chosen)
             s->cur = cur0;
             s->packed = packed0;
             s->flags_fresh = fresh0;
+            s->zflags_fresh = false;
             return LMX_OK;
         };
 
         struct Config {
             int path, yz;
             uint32_t seg;
-            bool fuse_reaction;
+            bool fuse_reaction, boxes;
         };
         // The y/z kernels and their window shapes; options a shape cannot use
         // fall back to the sweeps path and are timed as such.
         const Config cands[] = {
-            {LMX_PATH_SWEEPS, 0, 8, true},  {LMX_PATH_SWEEPS, 0, 8, false}, {LMX_PATH_SWEEPS, 1, 4, true},
-            {LMX_PATH_SWEEPS, 1, 8, true},  {LMX_PATH_SWEEPS, 2, 8, true},  {LMX_PATH_SWEEPS, 3, 4, true},
-            {LMX_PATH_SWEEPS, 3, 8, true},  {LMX_PATH_FUSED, 0, 8, true},
+            {LMX_PATH_SWEEPS, 0, 8, true, true},   {LMX_PATH_SWEEPS, 0, 8, true, false},
+            {LMX_PATH_SWEEPS, 0, 8, false, false}, {LMX_PATH_SWEEPS, 1, 4, true, false},
+            {LMX_PATH_SWEEPS, 1, 8, true, false},  {LMX_PATH_SWEEPS, 2, 8, true, false},
+            {LMX_PATH_SWEEPS, 3, 4, true, false},  {LMX_PATH_SWEEPS, 3, 8, true, false},
+            {LMX_PATH_FUSED, 0, 8, true, false},
         };
-        const Config before{s->path, s->yz_kernel, s->march_seg, s->fuse_reaction};
+        const Config before{s->path, s->yz_kernel, s->march_seg, s->fuse_reaction, s->boxes};
         // With LMX_OPT_FORCE_GENERIC the caller chose the one-site-per-thread
         // kernels, which have no y/z shapes to choose among: only the current
         // configuration is timed, and every option stays as it is.
@@ -1130,7 +1267,7 @@ int lmx_autotune(lmx_solver *s, uint32_t nsteps, double *best_ms, int *chosen)
         std::vector<Config> list{before};
         for (const Config &c : cands)
             if (!generic0 && (c.path != before.path || c.yz != before.yz || c.seg != before.seg ||
-                c.fuse_reaction != before.fuse_reaction))
+                c.fuse_reaction != before.fuse_reaction || c.boxes != before.boxes))
                 list.push_back(c);
         std::vector<double> times(list.size(), -1.0);
         for (int pass = 0; pass < 2 && !rc; pass++) {
@@ -1140,6 +1277,7 @@ int lmx_autotune(lmx_solver *s, uint32_t nsteps, double *best_ms, int *chosen)
                 s->yz_kernel = c.yz;
                 s->march_seg = c.seg;
                 s->fuse_reaction = c.fuse_reaction;
+                s->boxes = c.boxes;
                 if ((rc = restore())) break;
                 lmx::Params p = make_params(s);
                 if ((rc = enqueue_step(s, p, nullptr, nullptr, nullptr))) break;  // untimed first step
@@ -1166,6 +1304,7 @@ int lmx_autotune(lmx_solver *s, uint32_t nsteps, double *best_ms, int *chosen)
         s->yz_kernel = keep.yz;
         s->march_seg = keep.seg;
         s->fuse_reaction = keep.fuse_reaction;
+        s->boxes = keep.boxes;
         s->force_generic = generic0;
         const int rc2 = restore();
         LMX_HIP(hipStreamSynchronize(s->stream));
@@ -1454,6 +1593,7 @@ int batch_finish(lmx_batch *b, uint32_t nsteps)
         if (nsteps & 1u) s->cur = 1 - s->cur;
         s->timestep += nsteps;
         s->packed = true;
+        s->zflags_fresh = false;
         LMX_HIP(hipStreamWaitEvent(s->stream, b->done, 0));
     }
     return LMX_OK;

@@ -124,6 +124,7 @@ __device__ inline uint32_t site_occupancy(const Params &p, const uint32_t *lat, 
 // A particle into slot occ (the site's first empty slot) of site s.
 __device__ inline void place_particle(const Params &p, uint32_t *lat, uint32_t s, uint32_t occ, uint32_t particle)
 {
+    clear_zero_flag(p, p.word_particles ? occ : occ >> 2, s);
     if (p.word_particles) {
         store_agent(lat + (size_t)occ * p.N + s, particle);
     } else {

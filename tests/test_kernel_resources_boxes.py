@@ -1,0 +1,22 @@
+"""Register budget of the boxed step's kernels, from the compiler's report of
+the last build: 80 VGPRs are six blocks of four waves per CU, as many as its
+24 KB of LDS allow, and no spill."""
+import os
+
+import pytest
+
+from lattice_microbes_amd import build
+
+pytestmark = pytest.mark.skipif(not os.path.exists(build.RESOURCES),
+                                reason="no kernel resource report (build the library first)")
+
+
+@pytest.mark.parametrize("W", [1, 2])
+@pytest.mark.parametrize("vec", [0, 1])
+def test_box_kernels_do_not_spill(W, vec):
+    res = build.kernel_resources()
+    names = [n for n in res if f"box_step_kernelINS_9ByteSitesILi{W}EE" in n and f"ELb{vec}E" in n]
+    assert len(names) == 1, names
+    r = res[names[0]]
+    assert r["ScratchSize"] == 0 and r["Occupancy"] >= 6, r
+    assert r["LDS Size"] <= 163840 // 6, r
