@@ -23,7 +23,7 @@ LIB = os.path.join(OUT_DIR, "liblmx_mpd.so")
 RESOURCES = os.path.join(OUT_DIR, "kernel_resources.txt")
 IO_LIB = os.path.join(OUT_DIR, "liblmx_io.so")
 
-SOURCES = ["mpd_kernels.hip", "mpd_fast.hip", "mpd_box.hip", "mpd_capi.cpp"]
+SOURCES = ["mpd_kernels.hip", "mpd_fast.hip", "mpd_box.hip", "mpd_resident.hip", "mpd_capi.cpp"]
 HEADERS = ["lmx_device.h", "lmx_kernels.h", "lmx_site.h"]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")

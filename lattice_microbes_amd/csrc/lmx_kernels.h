@@ -46,6 +46,12 @@ struct CandList;
 hipError_t launch_box_step(const Params &p, const BoxGeom &g, const uint32_t *src, uint32_t *dst, const uint32_t *zs,
                            uint32_t *zd, const CandList &rl, hipStream_t st);
 hipError_t launch_box_reactions(const Params &p, uint32_t *lat, const CandList &rl, hipStream_t st);
+// Resident runs (mpd_resident.hip) of n solvers of one layout: a single job by
+// value (jobs null) or n jobs in device memory, each gathered by `per` blocks.
+struct ResidentJob;
+uint32_t resident_gather_blocks(uint32_t N);
+hipError_t launch_resident(const ResidentJob &one, const ResidentJob *jobs, uint32_t n, uint32_t per, uint32_t P,
+                           bool words, hipStream_t st);
 uint32_t x4_blocks(const Params &p);
 uint32_t reaction_blocks(const Params &p);
 struct TileGeom;

@@ -21,6 +21,7 @@
 #include "lmx_box.h"
 #include "lmx_device.h"
 #include "lmx_kernels.h"
+#include "lmx_resident.h"
 
 namespace {
 
@@ -150,6 +151,12 @@ struct lmx_solver {
     uint32_t splits_seen = 0, splits_step = 0;  // Control::box_splits and the step when it was last looked at
     uint32_t *d_zflags = nullptr;
     bool zflags_fresh = false;
+    // Resident runs (a solver of few particles in one block): the particles of
+    // the lattice as the host last set it, the run's list, and whether a run
+    // was enqueued that may have stopped short (settle).
+    size_t particles = 0;
+    uint2 *d_res = nullptr;      // kResidentCap entries, then the count
+    bool resident_ok = false, res_pending = false;
     uint32_t num_cu = 256;
 };
 
@@ -265,11 +272,19 @@ lmx::Params make_params(const lmx_solver *s)
     return p;
 }
 
-int require_ready(lmx_solver *s)
+int settle(lmx_solver *s);
+
+int require_built(lmx_solver *s)
 {
     if (!s) return fail(LMX_ERR_ARG, "null solver");
     if (!s->diffusion_built) return fail(LMX_ERR_STATE, "the diffusion model and lattice have not been set");
     return select_device(s);
+}
+
+int require_ready(lmx_solver *s)
+{
+    const int rc = require_built(s);
+    return rc ? rc : settle(s);
 }
 
 // Row-major (x,y,z,p) -> native planes, inserting each nonzero particle at
@@ -363,6 +378,8 @@ void set_box_level(lmx_solver *s, uint32_t level)
 // 0.01 to 0.4 particles a site, the boxes that fit 18-38 us.
 void plan_boxes(lmx_solver *s, const std::vector<uint32_t> &at)
 {
+    s->particles = at.size();
+    s->resident_ok = s->d_res != nullptr;
     const uint32_t cap = (uint32_t)lmx::box_cap(s->P);
     if (at.size() > s->N) return set_box_level(s, lmx::kBoxLevels);  // more than a particle a site: no box fits
     std::vector<uint32_t> n, ybox(s->Y), zbox(s->Z);
@@ -388,6 +405,14 @@ int check_device_error(lmx_solver *s)
 {
     uint32_t hdr[offsetof(lmx::Control, box_splits) / sizeof(uint32_t) + 1];
     LMX_HIP(hipMemcpy(hdr, s->d_ctl, sizeof(hdr), hipMemcpyDeviceToHost));
+    if (s->res_pending) {
+        if (hdr[0] != s->timestep) {
+            if (int rc = settle(s)) return rc;
+            LMX_HIP(hipStreamSynchronize(s->stream));
+            LMX_HIP(hipMemcpy(hdr, s->d_ctl, sizeof(hdr), hipMemcpyDeviceToHost));
+        }
+        s->res_pending = false;
+    }
     // Many boxes had to be halved since the last look (the lattice became
     // more crowded): smaller boxes from now on.
     const uint32_t splits = hdr[offsetof(lmx::Control, box_splits) / sizeof(uint32_t)] - s->splits_seen;
@@ -569,6 +594,79 @@ int enqueue_step(lmx_solver *s, const lmx::Params &p0, hipEvent_t *ev, int *kind
     return LMX_OK;
 }
 
+// Steps of one lmx_run_steps call from which a resident run pays for listing
+// the particles and writing them back.
+constexpr uint32_t kResidentMinSteps = 4;
+
+// A solver of few particles runs in one block: the default options, no
+// zero-order reactions (they would need every empty site).  The bimolecular
+// 64^3 model (2000 particles) takes 17 us a step in boxes.
+bool use_resident(const lmx_solver *s, uint32_t nsteps)
+{
+    return nsteps >= kResidentMinSteps && s->resident_ok && s->particles <= lmx::kResidentMost && !s->any_qp0 &&
+           s->boxes && s->path == LMX_PATH_SWEEPS && s->yz_kernel == 0 && s->fuse_reaction && !s->force_generic;
+}
+
+lmx::ResidentJob resident_job(const lmx_solver *s, uint32_t nsteps)
+{
+    lmx::ResidentJob j;
+    j.p = make_params(s);
+    j.lat = s->d_lat[s->cur];
+    j.list = s->d_res;
+    j.count = reinterpret_cast<uint32_t *>(s->d_res + lmx::kResidentCap);
+    j.start = s->timestep;
+    j.nsteps = nsteps;
+    return j;
+}
+
+// After a resident run of nsteps was enqueued.
+void resident_ran(lmx_solver *s, uint32_t nsteps)
+{
+    s->timestep += nsteps;
+    s->packed = true;
+    s->flags_fresh = s->zflags_fresh = false;
+    s->res_pending = true;
+}
+
+// nsteps timesteps: a resident run, or one step's launches after another.
+int enqueue_steps(lmx_solver *s, uint32_t nsteps, const lmx::ReactionList *rl = nullptr)
+{
+    if (use_resident(s, nsteps)) {
+        while (nsteps) {
+            const uint32_t m = std::min(nsteps, lmx::kResidentMaxSteps);
+            const hipError_t e = lmx::launch_resident(resident_job(s, m), nullptr, 1, lmx::resident_gather_blocks((uint32_t)s->N),
+                                                      s->P, s->bpp == 4, s->stream);
+            if (e != hipSuccess) return hip_fail(e, "resident run launch");
+            resident_ran(s, m);
+            nsteps -= m;
+        }
+        return LMX_OK;
+    }
+    if (int rc = settle(s)) return rc;
+    const lmx::Params p = make_params(s);
+    for (uint32_t i = 0; i < nsteps; i++)
+        if (int rc = enqueue_step(s, p, nullptr, nullptr, nullptr, rl)) return rc;
+    return LMX_OK;
+}
+
+// A resident run stops short when its block is full (the particles multiplied,
+// or a caller put more of them into the device's lattice); the runs enqueued
+// after it then did nothing.  The steps that are missing run here in the
+// ordinary way, before anything else looks at the state.
+int settle(lmx_solver *s)
+{
+    if (!s->res_pending) return LMX_OK;
+    LMX_HIP(hipStreamSynchronize(s->stream));
+    uint32_t t = 0;
+    LMX_HIP(hipMemcpy(&t, &s->d_ctl->timestep, sizeof(t), hipMemcpyDeviceToHost));
+    s->res_pending = false;
+    if (t == s->timestep) return LMX_OK;
+    const uint32_t missing = s->timestep - t;
+    s->timestep = t;
+    s->resident_ok = false;
+    return enqueue_steps(s, missing);
+}
+
 void free_device(lmx_solver *s)
 {
     dev_free(s->d_lat[0]);
@@ -576,6 +674,8 @@ void free_device(lmx_solver *s)
     dev_free(s->d_sites);
     dev_free(s->d_rl);
     dev_free(s->d_zflags);
+    dev_free(s->d_res);
+    s->resident_ok = s->res_pending = false;
     s->zflags_fresh = false;
     s->rlist = lmx::ReactionList{};
     dev_free(s->d_T);
@@ -665,6 +765,7 @@ int lmx_initialize(lmx_solver *s, uint32_t replicate, uint32_t seedTop, double t
         return fail(LMX_ERR_ARG, "rdme.mpd.overflowhandler: unknown handler");
     if (boundary != LMX_BOUNDARY_PERIODIC && boundary != LMX_BOUNDARY_REFLECTING)
         return fail(LMX_ERR_ARG, "unknown boundary mode");
+    if (int rc = settle(s)) return rc;  // steps already asked for keep the old parameters
     if (seedTop == 0) {
         struct timespec ts;
         clock_gettime(CLOCK_REALTIME, &ts);
@@ -837,6 +938,10 @@ int lmx_build_diffusion_model(lmx_solver *s, uint32_t nST, const double *DF, con
         if (e == hipSuccess)
             e = hipMalloc((void **)&s->d_zflags, 2 * (size_t)s->W * sizeof(uint32_t) *
                               lmx::box_geom(X, Y, Z, lmx::kBoxLevel[lmx::kBoxLevels - 1]).nboxes);
+        if (e == hipSuccess && X <= lmx::kResidentMaxEdge && Y <= lmx::kResidentMaxEdge && Z <= lmx::kResidentMaxEdge) {
+            e = hipMalloc((void **)&s->d_res, lmx::kResidentCap * sizeof(uint2) + sizeof(uint32_t));
+            if (e == hipSuccess) e = hipMemset(s->d_res + lmx::kResidentCap, 0, sizeof(uint32_t));
+        }
         if (e == hipSuccess && s->d_rl) {
             s->rlist.rec = s->d_rl;
             s->rlist.cap = (uint32_t)rcap;
@@ -899,6 +1004,7 @@ int lmx_set_reaction_rate(lmx_solver *s, uint32_t rxid, float rate)
     return guarded([&]() -> int {
         if (!s) return fail(LMX_ERR_ARG, "null solver");
         if (!s->model_built || rxid >= s->R) return fail(LMX_ERR_ARG, "reaction index is out of bounds");
+        if (int rc = settle(s)) return rc;  // steps already asked for keep the old rate
         s->k[rxid] = rate;
         if (s->diffusion_built) compute_propensities(s);
         return LMX_OK;
@@ -946,21 +1052,18 @@ int lmx_set_launch_option(lmx_solver *s, int option, int value)
 
 int lmx_run_steps(lmx_solver *s, uint32_t nsteps)
 {
-    int rc = require_ready(s);
+    int rc = require_built(s);
     if (rc) return rc;
     if (s->tables_dirty) {
         LMX_HIP(hipStreamSynchronize(s->stream));
         if ((rc = upload_tables(s))) return rc;
     }
-    const lmx::Params p = make_params(s);
-    for (uint32_t i = 0; i < nsteps; i++)
-        if ((rc = enqueue_step(s, p, nullptr, nullptr, nullptr))) return rc;
-    return LMX_OK;
+    return enqueue_steps(s, nsteps);
 }
 
 int lmx_run_steps_static(lmx_solver *s, uint32_t nsteps)
 {
-    int rc = require_ready(s);
+    int rc = require_built(s);
     if (rc) return rc;
     if (s->N > lmx::kStaticListMaxSites)
         return fail(LMX_ERR_ARG, "lmx_run_steps_static: the lattice has " + std::to_string(s->N) +
@@ -974,10 +1077,7 @@ int lmx_run_steps_static(lmx_solver *s, uint32_t nsteps)
         const hipError_t e = lmx::static_reaction_list(s->device, s->bpp == 1 ? s->W : 1, &rl);
         if (e != hipSuccess) return hip_fail(e, "static reaction list");
     }
-    const lmx::Params p = make_params(s);
-    for (uint32_t i = 0; i < nsteps; i++)
-        if ((rc = enqueue_step(s, p, nullptr, nullptr, nullptr, &rl))) return rc;
-    return LMX_OK;
+    return enqueue_steps(s, nsteps, &rl);
 }
 
 int lmx_synchronize(lmx_solver *s)
@@ -1173,6 +1273,7 @@ int lmx_get_overflow_stats(lmx_solver *s, uint64_t *entries, uint64_t *steps)
     if (!s) return fail(LMX_ERR_ARG, "null solver");
     int rc = select_device(s);
     if (rc) return rc;
+    if ((rc = settle(s))) return rc;
     LMX_HIP(hipStreamSynchronize(s->stream));
     lmx::Control c;
     LMX_HIP(hipMemcpy(&c, s->d_ctl, offsetof(lmx::Control, ovf_keys), hipMemcpyDeviceToHost));
@@ -1186,6 +1287,7 @@ int lmx_get_unresolved_overflows(lmx_solver *s, uint32_t *count)
     if (!s || !count) return fail(LMX_ERR_ARG, "null argument");
     int rc = select_device(s);
     if (rc) return rc;
+    if ((rc = settle(s))) return rc;
     LMX_HIP(hipStreamSynchronize(s->stream));
     lmx::Control c;
     LMX_HIP(hipMemcpy(&c, s->d_ctl, offsetof(lmx::Control, ovf_keys), hipMemcpyDeviceToHost));
@@ -1353,17 +1455,15 @@ int lmx_time_steps(lmx_solver *s, uint32_t nsteps, double *total_ms, double *ker
         }
         LMX_HIP(hipStreamSynchronize(s->stream));
         LMX_HIP(hipEventRecord(t0, s->stream));
-        for (uint32_t base = 0; base < nsteps; base += chunk) {
+        if (!kernel_ms && (rc = enqueue_steps(s, nsteps))) return rc;
+        for (uint32_t base = 0; kernel_ms && base < nsteps; base += chunk) {
             const uint32_t m = (nsteps - base) < chunk ? (nsteps - base) : chunk;
             std::vector<int> nl(m, 0);
             for (uint32_t i = 0; i < m; i++) {
-                if (kernel_ms)
-                    rc = enqueue_step(s, p, &ev[(size_t)i * (kMaxLaunches + 1)], &kinds[(size_t)i * kMaxLaunches], &nl[i]);
-                else
-                    rc = enqueue_step(s, p, nullptr, nullptr, nullptr);
+                rc = enqueue_step(s, p, &ev[(size_t)i * (kMaxLaunches + 1)], &kinds[(size_t)i * kMaxLaunches], &nl[i]);
                 if (rc) return rc;
             }
-            if (kernel_ms) {
+            {
                 LMX_HIP(hipEventSynchronize(ev[(size_t)(m - 1) * (kMaxLaunches + 1) + nl[m - 1]]));
                 for (uint32_t i = 0; i < m; i++) {
                     hipEvent_t *e = &ev[(size_t)i * (kMaxLaunches + 1)];
@@ -1494,6 +1594,13 @@ struct lmx_batch {
     hipStream_t stream = nullptr;
     hipEvent_t done = nullptr;
     std::vector<lmx_solver *> members;
+    // of the run being enqueued: the members the batched kernels step, and
+    // those that run in a block of their own
+    std::vector<lmx_solver *> stepped, resident;
+    hipStream_t stream2 = nullptr;   // resident runs, beside the batched steps
+    hipEvent_t fork = nullptr, join = nullptr;
+    uint32_t jobs_cap = 0;
+    lmx::ResidentJob *d_jobs = nullptr, *h_jobs = nullptr;
     uint32_t W = 0;
     bool use_graph = true;
     bool use_list = true;  // reaction phases over the members' lists (LMX_BATCH_REACTION_LIST)
@@ -1534,10 +1641,18 @@ int member_ready(lmx_solver *s, bool may_alloc)
         if (!may_alloc)
             return fail(LMX_ERR_STATE, "a member's reaction rates changed since its tables were uploaded; an allocating "
                                        "call (lmx_batch_run_steps or lmx_run_steps) uploads them");
-        int rc = upload_tables(s);
+        int rc = settle(s);
+        if (!rc) rc = upload_tables(s);
         if (rc) return rc;
     }
+    if (int rc = settle(s)) return rc;
     LMX_HIP(hipStreamSynchronize(s->stream));
+    return LMX_OK;
+}
+
+// The chunk flags of a member that the batched kernels step.
+int member_flags(lmx_solver *s)
+{
     if (s->flag_words > 0 && !s->flags_fresh) {
         for (int bb = 0; bb < 2; bb++)
             LMX_HIP(hipMemset(s->d_lat[bb] + s->N * s->W, 0, s->flag_words * sizeof(uint32_t)));
@@ -1589,25 +1704,58 @@ void fill_member(const lmx_solver *s, bool use_list, uint32_t threads, lmx::Memb
 int batch_finish(lmx_batch *b, uint32_t nsteps)
 {
     LMX_HIP(hipEventRecord(b->done, b->stream));
-    for (lmx_solver *s : b->members) {
+    for (lmx_solver *s : b->stepped) {
         if (nsteps & 1u) s->cur = 1 - s->cur;
         s->timestep += nsteps;
         s->packed = true;
         s->zflags_fresh = false;
-        LMX_HIP(hipStreamWaitEvent(s->stream, b->done, 0));
     }
+    for (lmx_solver *s : b->resident) resident_ran(s, nsteps);
+    for (lmx_solver *s : b->members) LMX_HIP(hipStreamWaitEvent(s->stream, b->done, 0));
+    return LMX_OK;
+}
+
+// The members of a run of nsteps: the ones with few particles run in a block
+// of their own each, beside the batched steps of the others (unless an option
+// of the batched kernels was set).  The 256 replicates of the ensemble
+// workload hold 2000 particles on 32^3 to 128^3 sites: the batched sweeps pay
+// 1.3 ms a step for their 1.8e8 sites.
+int batch_jobs(lmx_batch *b, uint32_t nsteps)
+{
+    b->stepped.clear();
+    b->resident.clear();
+    const bool alone = b->use_list && b->tile_threads == 0;
+    for (lmx_solver *s : b->members) (alone && use_resident(s, nsteps) ? b->resident : b->stepped).push_back(s);
+    const uint32_t n = (uint32_t)b->resident.size();
+    if (n > b->jobs_cap) {
+        uint32_t cap = b->jobs_cap ? b->jobs_cap : 16;
+        while (cap < n) cap *= 2;
+        dev_free(b->d_jobs);
+        if (b->h_jobs) hipHostFree(b->h_jobs);
+        b->h_jobs = nullptr;
+        b->jobs_cap = 0;
+        LMX_HIP(hipMalloc((void **)&b->d_jobs, sizeof(lmx::ResidentJob) * cap));
+        LMX_HIP(hipHostMalloc((void **)&b->h_jobs, sizeof(lmx::ResidentJob) * cap, hipHostMallocDefault));
+        b->jobs_cap = cap;
+    }
+    for (uint32_t r = 0; r < n; r++) b->h_jobs[r] = resident_job(b->resident[r], nsteps);
+    if (n)
+        LMX_HIP(hipMemcpyAsync(b->d_jobs, b->h_jobs, sizeof(lmx::ResidentJob) * n, hipMemcpyHostToDevice, b->stream));
     return LMX_OK;
 }
 
 // Descriptors of every member from its host-side state (buffer parity,
 // tables); the device copy is refreshed before each run.
-int batch_prepare(lmx_batch *b)
+int batch_prepare(lmx_batch *b, uint32_t nsteps)
 {
     if (b->staged_pending) {
         LMX_HIP(hipEventSynchronize(b->staged));
         b->staged_pending = false;
     }
-    const uint32_t n = (uint32_t)b->members.size();
+    for (lmx_solver *s : b->members)
+        if (int rc = member_ready(s, true)) return rc;
+    if (int rc = batch_jobs(b, nsteps)) return rc;
+    const uint32_t n = (uint32_t)b->stepped.size();
     if (n > b->cap) {
         uint32_t cap = b->cap ? b->cap : 16;
         while (cap < n) cap *= 2;
@@ -1627,9 +1775,8 @@ int batch_prepare(lmx_batch *b)
     }
     uint32_t acc[4] = {0, 0, 0, 0};
     for (uint32_t r = 0; r < n; r++) {
-        lmx_solver *s = b->members[r];
-        int rc = member_ready(s, true);
-        if (rc) return rc;
+        lmx_solver *s = b->stepped[r];
+        if (int rc = member_flags(s)) return rc;
         uint32_t blocks[4];
         fill_member(s, b->use_list, batch_tile_threads(b), b->h_members[r], blocks);
         for (int k = 0; k < 4; k++) {
@@ -1639,7 +1786,7 @@ int batch_prepare(lmx_batch *b)
     }
     size_t blocks = 0;
     for (int k = 0; k < 4; k++) {
-        b->h_start[k * (b->cap + 1) + n] = acc[k];
+        if (n) b->h_start[k * (b->cap + 1) + n] = acc[k];
         b->total[k] = acc[k];
         blocks += acc[k];
     }
@@ -1656,14 +1803,16 @@ int batch_prepare(lmx_batch *b)
         batch_drop_graph(b);
     }
     uint32_t *map = b->h_map;
-    for (int k = 0; k < 4; k++) {
+    for (int k = 0; n && k < 4; k++) {
         const uint32_t *st = b->h_start + k * (b->cap + 1);
         for (uint32_t r = 0; r < n; r++) std::fill(map + st[r], map + st[r + 1], r);
         map += acc[k];
     }
-    LMX_HIP(hipMemcpyAsync(b->d_members, b->h_members, sizeof(lmx::Member) * n, hipMemcpyHostToDevice, b->stream));
-    LMX_HIP(hipMemcpyAsync(b->d_start, b->h_start, sizeof(uint32_t) * 4 * (b->cap + 1), hipMemcpyHostToDevice,
-                           b->stream));
+    if (n) {
+        LMX_HIP(hipMemcpyAsync(b->d_members, b->h_members, sizeof(lmx::Member) * n, hipMemcpyHostToDevice, b->stream));
+        LMX_HIP(hipMemcpyAsync(b->d_start, b->h_start, sizeof(uint32_t) * 4 * (b->cap + 1), hipMemcpyHostToDevice,
+                               b->stream));
+    }
     if (blocks) LMX_HIP(hipMemcpyAsync(b->d_map, b->h_map, sizeof(uint32_t) * blocks, hipMemcpyHostToDevice, b->stream));
     LMX_HIP(hipEventRecord(b->staged, b->stream));
     b->staged_pending = true;
@@ -1672,7 +1821,7 @@ int batch_prepare(lmx_batch *b)
 
 int batch_enqueue_step(lmx_batch *b)
 {
-    const uint32_t n = (uint32_t)b->members.size();
+    const uint32_t n = (uint32_t)b->stepped.size();
     const uint32_t stride = b->cap + 1;
     const uint32_t *start[4], *map[4];
     size_t off = 0;
@@ -1691,7 +1840,7 @@ int batch_enqueue_step(lmx_batch *b)
 
 int batch_capture(lmx_batch *b)
 {
-    if (b->exec && b->graph_members == b->members && std::memcmp(b->graph_total, b->total, sizeof(b->total)) == 0)
+    if (b->exec && b->graph_members == b->stepped && std::memcmp(b->graph_total, b->total, sizeof(b->total)) == 0)
         return LMX_OK;
     batch_drop_graph(b);
     hipGraph_t g = nullptr;
@@ -1709,7 +1858,7 @@ int batch_capture(lmx_batch *b)
         b->exec = nullptr;
         return hip_fail(e, "hipGraphInstantiate");
     }
-    b->graph_members = b->members;
+    b->graph_members = b->stepped;
     std::memcpy(b->graph_total, b->total, sizeof(b->total));
     return LMX_OK;
 }
@@ -1730,6 +1879,9 @@ int lmx_batch_create(int device, lmx_batch **out)
         if (e == hipSuccess) e = hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking);
         if (e == hipSuccess) e = hipEventCreateWithFlags(&b->done, hipEventDisableTiming);
         if (e == hipSuccess) e = hipEventCreateWithFlags(&b->staged, hipEventDisableTiming);
+        if (e == hipSuccess) e = hipStreamCreateWithFlags(&b->stream2, hipStreamNonBlocking);
+        if (e == hipSuccess) e = hipEventCreateWithFlags(&b->fork, hipEventDisableTiming);
+        if (e == hipSuccess) e = hipEventCreateWithFlags(&b->join, hipEventDisableTiming);
         if (e != hipSuccess) {
             int rc = hip_fail(e, "lmx_batch_create");
             lmx_batch_destroy(b);
@@ -1755,6 +1907,11 @@ int lmx_batch_destroy(lmx_batch *b)
     if (b->h_map) hipHostFree(b->h_map);
     if (b->done) hipEventDestroy(b->done);
     if (b->staged) hipEventDestroy(b->staged);
+    dev_free(b->d_jobs);
+    if (b->h_jobs) hipHostFree(b->h_jobs);
+    if (b->fork) hipEventDestroy(b->fork);
+    if (b->join) hipEventDestroy(b->join);
+    if (b->stream2) hipStreamDestroy(b->stream2);
     if (b->stream) hipStreamDestroy(b->stream);
     delete b;
     return LMX_OK;
@@ -1832,15 +1989,31 @@ int lmx_batch_run_steps(lmx_batch *b, uint32_t nsteps)
         if (!b) return fail(LMX_ERR_ARG, "null batch");
         if (nsteps == 0 || b->members.empty()) return LMX_OK;
         LMX_HIP(hipSetDevice(b->device));
-        int rc = batch_prepare(b);
+        for (; nsteps > lmx::kResidentMaxSteps; nsteps -= lmx::kResidentMaxSteps)
+            if (int rc = lmx_batch_run_steps(b, lmx::kResidentMaxSteps)) return rc;
+        int rc = batch_prepare(b, nsteps);
         if (rc) return rc;
-        if (b->use_graph) {
+        const uint32_t nr = (uint32_t)b->resident.size();
+        if (nr) {
+            // beside the batched steps, after the uploads above
+            size_t most = 0;
+            for (lmx_solver *s : b->resident) most = std::max(most, s->N);
+            const uint32_t per = std::min(lmx::resident_gather_blocks((uint32_t)most), nr > 8 ? 128u : 512u);
+            LMX_HIP(hipEventRecord(b->fork, b->stream));
+            LMX_HIP(hipStreamWaitEvent(b->stream2, b->fork, 0));
+            const hipError_t e = lmx::launch_resident(lmx::ResidentJob{}, b->d_jobs, nr, per, b->W * 4, false, b->stream2);
+            if (e != hipSuccess) return hip_fail(e, "resident run launch");
+            LMX_HIP(hipEventRecord(b->join, b->stream2));
+        }
+        if (b->stepped.empty()) {
+        } else if (b->use_graph) {
             if ((rc = batch_capture(b))) return rc;
             for (uint32_t i = 0; i < nsteps; i++) LMX_HIP(hipGraphLaunch(b->exec, b->stream));
         } else {
             for (uint32_t i = 0; i < nsteps; i++)
                 if ((rc = batch_enqueue_step(b))) return rc;
         }
+        if (nr) LMX_HIP(hipStreamWaitEvent(b->stream, b->join, 0));
         return batch_finish(b, nsteps);
     });
 }
@@ -1865,7 +2038,7 @@ int lmx_batch_autotune(lmx_batch *b, uint32_t nsteps, double *best_ms, int *chos
         if (nsteps == 0 || nsteps > 10000) return fail(LMX_ERR_ARG, "nsteps must be in 1..10000");
         if (b->members.empty()) return fail(LMX_ERR_STATE, "the batch has no members");
         LMX_HIP(hipSetDevice(b->device));
-        int rc = batch_prepare(b);  // members' own work done, tables current
+        int rc = batch_prepare(b, 1);  // members' own work done, tables current
         if (rc) return rc;
         LMX_HIP(hipStreamSynchronize(b->stream));
 
@@ -1909,6 +2082,7 @@ int lmx_batch_autotune(lmx_batch *b, uint32_t nsteps, double *best_ms, int *chos
                     s->cur = v.cur;
                     s->packed = v.packed;
                     s->flags_fresh = v.fresh;
+                    s->zflags_fresh = s->res_pending = false;
                 }
             }
             return LMX_OK;
@@ -1983,8 +2157,8 @@ int lmx_batch_time_steps(lmx_batch *b, uint32_t nsteps, double *total_ms)
         hipEvent_t t0, t1;
         LMX_HIP(hipEventCreate(&t0));
         LMX_HIP(hipEventCreate(&t1));
-        int rc = batch_prepare(b);
-        if (!rc && b->use_graph) rc = batch_capture(b);
+        int rc = batch_prepare(b, nsteps);
+        if (!rc && b->use_graph && !b->stepped.empty()) rc = batch_capture(b);
         if (!rc) {
             LMX_HIP(hipStreamSynchronize(b->stream));
             LMX_HIP(hipEventRecord(t0, b->stream));

@@ -20,3 +20,13 @@ def test_box_kernels_do_not_spill(W, vec):
     r = res[names[0]]
     assert r["ScratchSize"] == 0 and r["Occupancy"] >= 6, r
     assert r["LDS Size"] <= 163840 // 6, r
+
+
+@pytest.mark.parametrize("W", [1, 2])
+@pytest.mark.parametrize("kernel", ["resident_run_kernel", "resident_run_jobs_kernel"])
+def test_resident_kernels_do_not_spill(W, kernel):
+    """A block of 16 waves has 128 VGPRs a lane."""
+    res = build.kernel_resources()
+    names = [n for n in res if f"{kernel}INS_9ByteSitesILi{W}EE" in n]
+    assert len(names) == 1, names
+    assert res[names[0]]["ScratchSize"] == 0 and res[names[0]]["Occupancy"] >= 4, res[names[0]]
