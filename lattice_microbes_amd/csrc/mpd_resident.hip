@@ -16,10 +16,15 @@
 // Why: a step of a small lattice is launches, not work.  The bimolecular 64^3
 // model (2000 particles) takes 17 us a step in boxes, three launches of which
 // none fills the device, and an ensemble pays every member's lattice in every
-// step although its members hold 2000 particles each.  A block of 1024 threads
-// steps 2000 particles in about 10 us (vector issue of one CU: 32 waves of 64
-// particles x ~600 instructions over 4 SIMDs, and four barriers), and an
-// ensemble runs a member per CU.
+// step although its members hold 2000 particles each.  One block steps them in
+// 11.8 us (12.4 us on 32^3, where 60 sites hold several particles), and an
+// ensemble runs a member per CU: 128 replicates on 32^3 to 128^3 sites take
+// 14.6 us a step against 970 us for the batched sweeps.
+//
+// What bounds it: a step is 28,000 cycles, 5,000 to 7,000 for each of the four
+// rounds (vector issue: two records per thread, about 200 instructions each
+// with the hash's quarter-rate multiplies, sixteen waves on four SIMDs) and
+// 5,000 for the sites to evaluate (latency of one wave's evaluation).
 #include "lmx_device.h"
 #include "lmx_kernels.h"
 #include "lmx_resident.h"
@@ -30,7 +35,7 @@ namespace lmx {
 namespace {
 
 constexpr uint32_t kNT = kResidentThreads, kCap = kResidentCap;
-constexpr uint32_t kChains = 2048u;
+constexpr uint32_t kChains = 8192u;      // two per record at least: most chains hold one particle
 constexpr uint32_t kEnd = 0xFFFFu, kDead = 0xFFFFFFFFu;
 constexpr uint32_t kIdBits = 13u;        // of a chain head: the particle; the sweep's tag above
 constexpr uint32_t kTab = 2048u;         // floats of the model's tables kept in LDS
@@ -54,7 +59,7 @@ struct ResidentLds {
     float tab[kTab];
     uint32_t occ[kBall];            // particles of the sites around an overflow entry
     unsigned long long best;
-    uint32_t n[2], ovf, spill, pick, alive;
+    uint32_t n[2], nc, ovf, spill, pick;  // records; sites to evaluate; ...
 };
 
 __device__ inline uint32_t site_of(const Params &p, uint32_t key)
@@ -107,9 +112,9 @@ __device__ inline void append(const Params &p, uint32_t *lat, ResidentLds &s, ui
 }
 
 // The reactions of a site, by one thread: its particles (the members of its
-// chain in generation 1 that fit) as words, the shared evaluation, and the
-// result back as records of generation 0 -- in the members' places, further
-// ones appended.
+// chain in generation 1 that fit) as words, the shared evaluation, and, if it
+// changed, the result back as records of generation 0 -- in the members'
+// places, further ones appended.
 template <class L>
 __device__ inline void react_chain(const Params &p, uint32_t *lat, ResidentLds &s, uint32_t key, uint32_t type,
                                    unsigned long long h3, const float2 *tab)
@@ -121,25 +126,21 @@ __device__ inline void react_chain(const Params &p, uint32_t *lat, ResidentLds &
     for (int k = 0; k < W; k++) w[k] = 0u;
     const uint32_t first = s.head[1][chain_of(key)] & ((1u << kIdBits) - 1u);
     for (uint32_t q = first; q != kEnd; q = s.next[1][q]) {
-        if (s.key[1][q] != key) continue;
-        const uint32_t o = s.ord[1][q];
-        uint32_t before, total;
-        chain_rank(s, 1, q, key, o, before, total);
-        if (before >= P) continue;
+        if (s.key[1][q] != key || s.key[0][q] == kDead) continue;
+        const uint32_t o = s.ord[0][q], j = o & 15u;  // its slot after the sweeps
 #pragma unroll
         for (int k = 0; k < W; k++) {
             if constexpr (L::kPerWord == 4) {
-                if ((before >> 2) == (uint32_t)k) w[k] |= ord_species(o) << (8u * (before & 3u));
+                if ((j >> 2) == (uint32_t)k) w[k] |= ord_species(o) << (8u * (j & 3u));
             } else {
-                if (before == (uint32_t)k) w[k] = ord_species(o);
+                if (j == (uint32_t)k) w[k] = ord_species(o);
             }
         }
     }
-    if (react_site_table_l<L>(p, site_of(p, key), type, w, h3, tab)) {
-        // products without a slot are overflow entries: only a full site has any
-        const uint32_t last = L::kPerWord == 4 ? w[W - 1] >> 24 : w[W - 1];
-        if (last) s.ovf = 1u;
-    }
+    if (!react_site_table_l<L>(p, site_of(p, key), type, w, h3, tab)) return;
+    // products without a slot are overflow entries: only a full site has any
+    const uint32_t last = L::kPerWord == 4 ? w[W - 1] >> 24 : w[W - 1];
+    if (last) s.ovf = 1u;
     uint32_t j = 0;  // the next slot to hand out
     auto slot = [&](uint32_t k) -> uint32_t {
         uint32_t v = 0;
@@ -437,7 +438,7 @@ __device__ __attribute__((always_inline)) inline void run_body(const ResidentJob
         s.n[0] = found < kCap ? found : kCap;
         s.n[1] = 0u;
         s.ovf = p.relaxed && agent_load(&ctl->carry_count) ? 1u : 0u;
-        s.spill = s.alive = 0u;
+        s.spill = s.nc = 0u;
     }
     for (uint32_t k = tid; k < found && k < kCap; k += kNT) {
         const uint2 v = job.list[k];
@@ -529,7 +530,7 @@ __device__ __attribute__((always_inline)) inline void run_body(const ResidentJob
                 if (axis == 2 && tid == 0) s.n[0] = n;
                 __syncthreads();
             }
-            // the step's lattice: generation 1 to 0, with the reactions
+            // the step's lattice: generation 1 to 0
             const unsigned long long h3 = timestep_hash(p.seed32, t, 3);
             for (uint32_t e = tid; e < n; e += kNT) {
                 const uint32_t key = s.key[1][e], ord = s.ord[1][e];
@@ -543,29 +544,36 @@ __device__ __attribute__((always_inline)) inline void run_body(const ResidentJob
                 if (before >= P) {
                     record_overflow(ctl, 2u, site_of(p, key), before - P, sp);
                     s.ovf = 1u;
-                    if (p.R == 0) s.key[0][e] = kDead;  // (else with the site's other particles)
+                    s.key[0][e] = kDead;
                     continue;
                 }
+                s.key[0][e] = key;
+                s.ord[0][e] = make_ord(before, 0u, st, sp);
                 // A particle alone takes its reaction test from the table; a
-                // site that reacts or holds several is evaluated by the
-                // thread of its first particle.
-                bool whole = false;
-                if (p.R > 0) {
-                    whole = total > 1u;
+                // site that reacts or holds several is evaluated after the
+                // barrier, one thread per site in as few waves as they need
+                // (beside this loop, every wave with such a site ran the whole
+                // evaluation: 19,000 of a step's 40,000 cycles).
+                if (p.R > 0 && before == 0u) {
+                    bool whole = total > 1u;
                     if (!whole) {
                         const float2 ap = tab[st * p.nS + (sp - 1u)];
                         whole = ap.x != 0.0f && ap.y > 0.0f && uniform01(site_of(p, key), 1, 0, h3) <= ap.y;
                     }
-                }
-                if (!whole) {
-                    s.key[0][e] = key;
-                    s.ord[0][e] = make_ord(before, 0u, st, sp);
-                } else if (before == 0u) {
-                    react_chain<L>(p, lat, s, key, st, h3, tab);
+                    if (whole) s.next[0][atomicAdd(&s.nc, 1u)] = (uint16_t)e;  // (the links of generation 0 are free)
                 }
             }
             if (tid == 0) s.n[1] = 0u;
             __syncthreads();
+            const uint32_t nc = s.nc;
+            if (nc) {
+                for (uint32_t k = tid; k < nc; k += kNT) {
+                    const uint32_t e = s.next[0][k];
+                    react_chain<L>(p, lat, s, s.key[1][e], ord_type(s.ord[1][e]), h3, tab);
+                }
+                __syncthreads();
+                if (tid == 0) s.nc = 0u;
+            }
             if (s.ovf) resolve_records<L>(p, lat, s, t);
         }
     }
