@@ -42,6 +42,7 @@ struct Control {
     // both at the end of each step.
     uint32_t list_overflow;
     uint32_t list_count[kListShards];
+    uint32_t blocks_done;       // of the launch that evaluates the candidates and resolves
 };
 
 // Sites queued for the reaction phase by a z sweep that lists its output: one
@@ -251,9 +252,10 @@ __device__ inline void record_overflow(Control *ctl, uint32_t phase, uint32_t si
                                        uint32_t particle)
 {
     const uint32_t k = atomicAdd(&ctl->ovf_count, 1u);
-    if (k < kMaxOverflows) {
-        ctl->ovf_part[k] = particle;
-        ctl->ovf_keys[k] = overflow_key(phase, site, emission, k);
+    if (k < kMaxOverflows) {  // device-scope stores: another block of the same launch may resolve them
+        __hip_atomic_store(&ctl->ovf_part[k], particle, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(&ctl->ovf_keys[k], overflow_key(phase, site, emission, k), __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
     }
 }
 

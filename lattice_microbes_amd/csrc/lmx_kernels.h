@@ -40,7 +40,8 @@ hipError_t launch_fused(const Params &p, const uint32_t *src, uint32_t *dst, uin
 hipError_t launch_reaction_fast(const Params &p, uint32_t *lat, hipStream_t st);
 hipError_t launch_prob_tables(const Params &p, float *prob1, float *prob0, hipStream_t st);
 // The boxed step (mpd_box.hip): one timestep from src to dst without the
-// reactions (launch_box_reactions) and the resolver.  zs and zd are the zero flags of the two buffers, rl the
+// reactions and the overflow resolution, which are launch_box_reactions's (a
+// model without reactions takes launch_resolve instead).  zs and zd are the zero flags of the two buffers, rl the
 // reaction candidates (any capacity is correct).
 struct CandList;
 hipError_t launch_box_step(const Params &p, const BoxGeom &g, const uint32_t *src, uint32_t *dst, const uint32_t *zs,

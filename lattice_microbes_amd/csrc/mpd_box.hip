@@ -40,6 +40,7 @@
 #include "lmx_box.h"
 #include "lmx_device.h"
 #include "lmx_kernels.h"
+#include "lmx_resolve.h"
 #include "lmx_site.h"
 
 namespace lmx {
@@ -581,31 +582,300 @@ __global__ __launch_bounds__(kBoxThreads, OCC) void box_step_kernel(Params p, Bo
     box_body<L, CAP, VEC>(p, g, src, dst, zs, zd, rl, p.ctl->timestep, logical, lds);
 }
 
+// ---------------------------------------------------------------------------
 // Reaction phase of the candidate sites that the boxes listed, one wave per
-// shard: the site's words and type are read again and evaluated in full, as in
-// the one-site-per-thread kernel.  A shard that ran out makes it the full pass.
-template <class L>
-__global__ __launch_bounds__(256, 4) void cand_react_kernel(Params p, uint32_t *__restrict__ lat, CandList rl)
+// shard, and the step's overflow resolution by the block that ends last.  A
+// shard that ran out makes it the full pass.
+//
+// The launch is latency: a candidate's chain of dependent loads.  So the table
+// entries of a site's particles are loaded together, and a reacting site
+// (checkForReaction decides it lane by lane) is taken by the whole wave: a
+// slot per lane to count and evaluate, a reaction per lane to select.  The
+// loops over slots are rolled, which keeps the kernel at 13 kB of code (71 kB
+// unrolled), and a shard's entries are dealt to four waves, so that its
+// reacting sites rarely queue behind one another.  Measured, with the
+// resolver (a launch of its own before): whole cell 256x256x512 27.0 -> 16.3
+// us, 64x64x256 uint32 lattice 21 -> 14.5, crowded P = 16 26 -> 16.7.
+// ---------------------------------------------------------------------------
+
+constexpr uint32_t kReactThreads = 1024, kShardWaves = 4, kShardThreads = 64u * kShardWaves,
+                   kReactShards = kReactThreads / kShardThreads;
+
+__device__ inline uint32_t lane_of(uint32_t v, uint32_t src)
 {
-    constexpr int W = L::W;
-    const float2 *tab = reinterpret_cast<const float2 *>(p.prob1);
-    const unsigned long long h3 = timestep_hash(p.seed32, p.ctl->timestep, 3);
-    const bool full = p.ctl->list_overflow != 0u;
-    const uint32_t wave = blockIdx.x * 4u + (threadIdx.x >> 6), lane = threadIdx.x & 63u;
-    const uint32_t n = full ? p.N : p.ctl->list_count[wave];
-    const uint32_t first = full ? wave * 64u + lane : lane, step = full ? (uint32_t)kListShards * 64u : 64u;
-    for (uint32_t k = first; k < n; k += step) {
-        const uint32_t i = full ? k : rl.site[(size_t)wave * rl.cap + k];
-        uint32_t w[W];
+    return (uint32_t)__builtin_amdgcn_readlane((int)v, (int)src);
+}
+
+// total_propensity's sum for a site of `count` particles in its first slots:
+// the same terms in the same order, a row of up to 8 pairs loaded at a time.
+// slots: the wave's copy of its sites' slots, slot-major, for this lane (a
+// slot's index is not known at compile time).
+template <uint32_t P>
+__device__ inline float packed_propensity(const Params &p, uint32_t st, const uint32_t (*slots)[64], uint32_t lane,
+                                          uint32_t count)
+{
+    constexpr uint32_t kRow = P < 8u ? P : 8u;
+    float a = p.qp0[st];
+#pragma unroll 1
+    for (uint32_t m = 0; m < count; m++) {
+        const uint32_t row = st * p.nS + slots[m][lane] - 1u;
+        const float one = p.qp1[row];
+        const float *pairs = p.qp2 + (size_t)row * p.nS;
+        uint32_t n = m + 1u;
+        float v[kRow];
+        auto load = [&] {
 #pragma unroll
-        for (int q = 0; q < W; q++) w[q] = (q == 0 || L::need_next(p, w[q > 0 ? q - 1 : 0])) ? lat[(size_t)q * p.N + i] : 0u;
-        if (!react_site_table_l<L>(p, i, p.sites[i], w, h3, tab)) continue;
+            for (uint32_t k = 0; k < kRow; k++) {
+                const uint32_t q = n + k < count ? n + k : m;
+                v[k] = pairs[slots[q][lane] - 1u];
+            }
+        };
+        load();
+        a += one;
+#pragma unroll 1
+        for (;;) {
 #pragma unroll
-        for (int q = 0; q < W; q++) {
-            lat[(size_t)q * p.N + i] = w[q];
-            if (w[q] != 0u) clear_zero_flag(p, q, i);
+            for (uint32_t k = 0; k < kRow; k++)
+                if (n + k < count) a += v[k];
+            n += kRow;
+            if (n >= count) break;
+            load();
         }
     }
+    return a;
+}
+
+// A reaction at lane src's site i (propensity a, words w): which one and the
+// site's new particles, by the whole wave.  Every lane of the wave calls it,
+// with its own site's values.
+template <class L>
+__device__ inline void wave_react(const Params &p, uint32_t *__restrict__ lat, uint32_t src, uint32_t i, uint32_t st,
+                                  const uint32_t *w, float a, unsigned long long h3)
+{
+    constexpr uint32_t P = L::P, kNone = 0xFFFFFFFFu;
+    const uint32_t lane = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+    const uint32_t si = lane_of(i, src), sst = lane_of(st, src);
+    // Lane j < P holds slot j.
+    uint32_t word = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < (uint32_t)L::W; k++) {
+        const uint32_t v = lane_of(w[k], src);
+        if (lane / L::kPerWord == k) word = v;
+    }
+    const uint32_t mine = lane >= P ? 0u : L::part(word, L::kPerWord == 1 ? 0 : (int)(lane & 3u));
+    uint32_t earlier = 0;  // of the same species
+#pragma unroll 1
+    for (uint32_t q = 0; q < P; q++) earlier += q < lane && lane_of(mine, q) == mine ? 1u : 0u;
+    // determineReactionIndex (byte_reaction_dev.cu:146-177): the reactions in
+    // ascending index, each with a positive propensity moving rp, among those
+    // listed under a species of the site (lane j: of slot j, if it is the
+    // first of its kind) and the zero-order ones (lane P).
+    uint32_t start = 0, len = 0;
+    if (lane == P || (mine != 0u && earlier == 0u)) {
+        const uint32_t bucket = lane == P ? p.nS : mine - 1u;
+        start = p.rx_off[bucket];
+        len = p.rx_off[bucket + 1] - start;
+    }
+    uint32_t total = 0;
+#pragma unroll 1
+    for (uint32_t j = 0; j <= P; j++) total += lane_of(len, j);
+    float rp = uniform01(si, 1, 1, h3) * __uint_as_float(lane_of(__float_as_uint(a), src));
+    uint32_t idx = 0, r = kNone, s0 = p.sto_off[0], s1 = p.sto_off[1], k0 = s0, k1 = s1;
+    float pr = 0.0f;
+    bool any = false;
+    while (rp > 0.0f) {
+        uint32_t br = kNone;  // this lane's lowest reaction above idx, and its propensity
+        float bp = 0.0f;
+        uint32_t bs0 = 0, bs1 = 0;
+#pragma unroll 1
+        for (uint32_t c = 0; c < total; c += 64u) {
+            if (!any || total > 64u) {  // one a lane is evaluated once and kept
+                uint32_t left = c + lane, at = kNone;
+#pragma unroll 1
+                for (uint32_t j = 0; j <= P; j++) {
+                    const uint32_t lj = lane_of(len, j), sj = lane_of(start, j);
+                    if (left < lj) at = sj + left;
+                    left = left < lj ? kNone : left - lj;
+                }
+                if (c + lane >= total) at = kNone;
+                r = kNone;
+                if (at != kNone) {
+                    r = p.rx_list[at];
+                    const bool here = p.RL[r * p.nST + sst] != 0;
+                    const uint32_t d1 = p.D1[r], d2 = p.D2[r], order = p.order[r];
+                    const float k = p.rate[r];
+                    s0 = p.sto_off[r];
+                    s1 = p.sto_off[r + 1];
+                    float n1 = 0.0f, n2 = 0.0f;
+#pragma unroll 1
+                    for (uint32_t q = 0; q < P; q++) {
+                        const uint32_t s = lane_of(mine, q);
+                        n1 += s && s == d1 ? 1.0f : 0.0f;
+                        n2 += s && s == d2 ? 1.0f : 0.0f;
+                    }
+                    // (reaction_propensity's expressions)
+                    pr = order == kZeroOrder ? k
+                         : order == kFirstOrder ? k * n1
+                         : order == kSecondOrder ? k * n1 * n2
+                         : order == kSecondOrderSelf ? k * n1 * (n1 - 1.0f) : 0.0f;
+                    if (!here || !(pr > 0.0f)) r = kNone;
+                }
+            }
+            if (r != kNone && (!any || r > idx) && r < br) {
+                br = r;
+                bp = pr;
+                bs0 = s0;
+                bs1 = s1;
+            }
+        }
+        uint32_t low = kNone;
+#pragma unroll 1
+        for (unsigned long long m = __ballot(br != kNone); m; m &= m - 1) {
+            const uint32_t v = lane_of(br, (uint32_t)__builtin_ctzll(m));
+            low = v < low ? v : low;
+        }
+        if (low == kNone) break;
+        const uint32_t who = (uint32_t)__builtin_ctzll(__ballot(br == low));
+        rp -= __uint_as_float(lane_of(__float_as_uint(bp), who));
+        k0 = lane_of(bs0, who);
+        k1 = lane_of(bs1, who);
+        idx = low;
+        any = true;
+    }
+    // evaluateReaction (:179-257): the m-th particle of species s is consumed
+    // iff fewer than -S[s] earlier ones of s were seen, the others move up,
+    // and the products follow in species order.  A reactant that was not
+    // present leaves a negative residue, which the reference turns into an
+    // unbounded loop.
+    // Lane k holds the row's k-th nonzero entry (64 of them at a time).
+    uint32_t row_s = 0;
+    int row_v = 0;
+    auto row = [&](uint32_t c) {
+        row_s = 0;
+        row_v = 0;
+        if (c + lane < k1) {
+            row_s = p.sto_sp[c + lane] + 1u;
+            row_v = p.sto_val[c + lane];
+        }
+    };
+    row(k0);
+    int change = 0;
+    bool underflow = false;
+#pragma unroll 1
+    for (uint32_t k = k0; k < k1; k++) {
+        if (k != k0 && ((k - k0) & 63u) == 0u) row(k);
+        const uint32_t s = lane_of(row_s, (k - k0) & 63u);
+        const int v = (int)lane_of((uint32_t)row_v, (k - k0) & 63u);
+        if (mine == s) change = v;
+        if (v < 0 && (int)__popcll(__ballot(mine == s)) < -v) underflow = true;
+    }
+    if (k1 - k0 > 64u) row(k0);
+    const bool stays = mine != 0u && (change >= 0 || (int)earlier >= -change);
+    const unsigned long long kept = __ballot(stays);
+    uint32_t n = (uint32_t)__popcll(kept);
+    const uint32_t to = stays ? __builtin_amdgcn_mbcnt_hi((uint32_t)(kept >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)kept, 0u))
+                              : 32u + (lane & 31u);  // (beyond the site)
+    uint32_t now = (uint32_t)__builtin_amdgcn_ds_permute((int)(to << 2), (int)mine);
+    if (lane >= n) now = 0u;
+#pragma unroll 1
+    for (uint32_t k = k0; k < k1; k++) {
+        if (k != k0 && ((k - k0) & 63u) == 0u) row(k);
+        const uint32_t s = lane_of(row_s, (k - k0) & 63u);
+#pragma unroll 1
+        for (int v = (int)lane_of((uint32_t)row_v, (k - k0) & 63u); v > 0; v--, n++) {
+            if (n < P) now = lane == n ? s : now;
+            else if (lane == 0u) record_overflow(p.ctl, 3, si, n - P, s);
+        }
+    }
+    if (underflow && lane == 0u && atomicCAS(&p.ctl->error, 0u, kErrReactionUnderflow) == 0u)
+        p.ctl->error_step = p.ctl->timestep;
+    // Device-scope stores: the last block may resolve overflow entries beside them.
+    if (lane < P && now != mine) {
+        if constexpr (L::kPerWord == 1)
+            __hip_atomic_store(lat + (size_t)lane * p.N + si, now, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        else
+            __hip_atomic_store(reinterpret_cast<uint8_t *>(lat + (size_t)(lane >> 2) * p.N + si) + (lane & 3u), (uint8_t)now,
+                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (now != 0u) clear_zero_flag(p, lane / L::kPerWord, si);
+    }
+}
+
+template <class L>
+__global__ __launch_bounds__(kReactThreads) void cand_react_kernel(Params p, uint32_t *__restrict__ lat, CandList rl)
+{
+    constexpr int W = L::W;
+    constexpr uint32_t P = L::P;
+    __shared__ uint32_t slots[kReactThreads / 64][P][64];
+    Control *ctl = p.ctl;
+    const unsigned long long h3 = timestep_hash(p.seed32, ctl->timestep, 3);
+    const bool full = ctl->list_overflow != 0u;
+    const uint32_t shard = blockIdx.x * kReactShards + threadIdx.x / kShardThreads, rank = threadIdx.x % kShardThreads;
+    const uint32_t n = full ? p.N : ctl->list_count[shard];
+    const uint32_t first = full ? shard * kShardThreads : 0u, step = full ? (uint32_t)kListShards * kShardThreads : kShardThreads;
+#pragma unroll 1
+    for (uint32_t k0 = first; k0 < n; k0 += step) {
+        // (a wave of the shard takes every kShardWaves-th entry, so that the
+        // sites that react are spread over them)
+        const uint32_t k = k0 + (rank & 63u) * kShardWaves + (rank >> 6);
+        uint32_t i = 0, st = 0, w[W];
+        float a = 0.0f;
+        bool hit = false;
+#pragma unroll
+        for (int q = 0; q < W; q++) w[q] = 0u;
+        if (k < n) {
+            i = full ? k : rl.site[(size_t)shard * rl.cap + k];
+            st = p.sites[i];
+#pragma unroll
+            for (int q = 0; q < W; q++)
+                if (q == 0 || L::need_next(p, w[q > 0 ? q - 1 : 0])) w[q] = lat[(size_t)q * p.N + i];
+            uint32_t count = 0;
+#pragma unroll
+            for (int j = 0; j < (int)P; j++) count += L::slot(w, j) != 0u ? 1u : 0u;
+            float prob = 0.0f;
+            const float u = uniform01(i, 1, 0, h3);
+            if (count == 0u) {
+                a = p.qp0[st];
+                prob = p.prob0[st];
+            } else if (count == 1u) {
+                const float2 ap = reinterpret_cast<const float2 *>(p.prob1)[st * p.nS + (L::slot(w, 0) - 1u)];
+                a = ap.x;
+                prob = ap.y;
+            } else {
+                if (count == 2u) {
+                    const uint32_t r1 = st * p.nS + (L::slot(w, 0) - 1u), s2 = L::slot(w, 1) - 1u;
+                    const float q0 = p.qp0[st], q1 = p.qp1[r1], q12 = p.qp2[r1 * p.nS + s2], q2 = p.qp1[st * p.nS + s2];
+                    a = q0;
+                    a += q1;
+                    a += q12;
+                    a += q2;
+                } else {
+#pragma unroll
+                    for (int j = 0; j < (int)P; j++) slots[threadIdx.x >> 6][j][rank & 63u] = L::slot(w, j);
+                    a = packed_propensity<P>(p, st, slots[threadIdx.x >> 6], rank & 63u, count);
+                }
+                // 1 - exp(-a) <= a, with room for the rounding of both (u is
+                // 0 or at least 2^-32): most sites need no exponential
+                if (a != 0.0f && u <= a * 1.0001f) prob = reaction_probability(a);
+            }
+            hit = a != 0.0f && prob > 0.0f && u <= prob;
+        }
+#pragma unroll 1
+        for (unsigned long long m = __ballot(hit); m; m &= m - 1)
+            wave_react<L>(p, lat, (uint32_t)__builtin_ctzll(m), i, st, w, a, h3);
+    }
+    // The block that ends last resolves the step's overflow entries.
+    __shared__ uint32_t last;
+    __builtin_amdgcn_s_waitcnt(0);  // every wave's stores have arrived
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+        last = atomicAdd(&ctl->blocks_done, 1u) == gridDim.x - 1u ? 1u : 0u;
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    }
+    __syncthreads();
+    if (!last) return;
+    if (threadIdx.x == 0) ctl->blocks_done = 0u;
+    resolve_body<kReactThreads>(p, lat);
 }
 
 template <class L, int CAP, int OCC>
@@ -624,7 +894,7 @@ hipError_t launch_box_reactions(const Params &p, uint32_t *lat, const CandList &
 {
     Params q = p;
     q.packed = 1u;  // the step has packed every site
-    const dim3 grid(kListShards / 4), block(256);
+    const dim3 grid(kListShards / kReactShards), block(kReactThreads);
     switch (p.word_particles ? 100 + (int)p.P : (int)p.W) {
     case 1: hipLaunchKernelGGL((cand_react_kernel<ByteSites<1>>), grid, block, 0, st, q, lat, rl); break;
     case 2: hipLaunchKernelGGL((cand_react_kernel<ByteSites<2>>), grid, block, 0, st, q, lat, rl); break;

@@ -507,11 +507,12 @@ int enqueue_step(lmx_solver *s, const lmx::Params &p0, hipEvent_t *ev, int *kind
         if (s->R > 0) {
             e = lmx::launch_box_reactions(p, s->d_lat[s->cur], cand, s->stream);
             if (e != hipSuccess) return hip_fail(e, "reaction launch");
-            if (int rc = mark(LMX_K_REACTION)) return rc;
+            if (int rc = mark(LMX_K_REACTION)) return rc;  // and the resolver
+        } else {
+            e = lmx::launch_resolve(p, s->d_lat[s->cur], s->stream);
+            if (e != hipSuccess) return hip_fail(e, "resolve launch");
+            if (int rc = mark(LMX_K_RESOLVE)) return rc;
         }
-        e = lmx::launch_resolve(p, s->d_lat[s->cur], s->stream);
-        if (e != hipSuccess) return hip_fail(e, "resolve launch");
-        if (int rc = mark(LMX_K_RESOLVE)) return rc;
         if (nlaunch) *nlaunch = n;
         s->timestep++;
         s->packed = true;

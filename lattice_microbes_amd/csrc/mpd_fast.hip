@@ -1543,9 +1543,11 @@ __device__ inline void reaction_list_body(const Params &p, uint32_t *__restrict_
 }
 
 // At most 128 VGPRs: four waves per SIMD to hide the table and lattice
-// latencies (measured 33 against 36 us with the compiler's 135).
+// latencies (measured 33 against 36 us with the compiler's 135).  P = 16 needs
+// 206 and takes two waves: held to 128 it spilled 121 VGPRs next to 387 SGPRs
+// and gave wrong sites.
 template <int W>
-__global__ __launch_bounds__(256, 4) void reaction_list_kernel(Params p, uint32_t *__restrict__ lat, ReactionList rl,
+__global__ __launch_bounds__(256, W == 4 ? 2 : 4) void reaction_list_kernel(Params p, uint32_t *__restrict__ lat, ReactionList rl,
                                                             uint32_t nshards)
 {
     if (p.ctl->list_overflow) {
@@ -2203,7 +2205,7 @@ __global__ __launch_bounds__(T, 8) void batch_tile_kernel(const Member *__restri
 // Reaction phase: the full pass, or the member's list (its share of blocks
 // walks the shards its z sweep filled).
 template <int W>
-__global__ __launch_bounds__(256, 4) void batch_reaction_kernel(const Member *__restrict__ m,
+__global__ __launch_bounds__(256, W == 4 ? 2 : 4) void batch_reaction_kernel(const Member *__restrict__ m,
                                                              const uint32_t *__restrict__ start,
                                                              const uint32_t *__restrict__ map, uint32_t n)
 {

@@ -18,6 +18,7 @@
 #include "lmx_batch.h"
 #include "lmx_device.h"
 #include "lmx_kernels.h"
+#include "lmx_resolve.h"
 #include "lmx_site.h"
 
 namespace lmx {
@@ -84,226 +85,9 @@ __global__ __launch_bounds__(256) void reaction_kernel(Params p, uint32_t *__res
     }
 }
 
-// ---------------------------------------------------------------------------
-// Overflow resolution: one workgroup.  Entries are sorted into canonical
-// order (phase, site, emission) and placed one after another; for each, the
-// workgroup scans the reference's candidate list (Lattice::getNearbySites,
-// Lattice.cpp:106-128: radius 0..4, shell max(R-1,0)^2 < d^2 <= R^2, x outer,
-// z inner) 256 candidates at a time and takes the first site with room and
-// the origin's site type.  The step counter advances at the end.
-// ---------------------------------------------------------------------------
-__device__ inline uint32_t load_agent(const uint32_t *ptr)
-{
-    return __hip_atomic_load(ptr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-__device__ inline void store_agent(uint32_t *ptr, uint32_t v)
-{
-    __hip_atomic_store(ptr, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// Particles up to the first empty slot (Lattice::getOccupancy).
-__device__ inline uint32_t site_occupancy(const Params &p, const uint32_t *lat, uint32_t s)
-{
-    uint32_t occ = 0;
-    for (uint32_t k = 0; k < p.W; k++) {
-        const uint32_t word = load_agent(lat + (size_t)k * p.N + s);
-        if (p.word_particles) {
-            if (word == 0) return occ;
-            occ++;
-            continue;
-        }
-        for (uint32_t b = 0; b < 4; b++) {
-            if (((word >> (8 * b)) & 0xFFu) == 0) return occ;
-            occ++;
-        }
-    }
-    return occ;
-}
-
-// A particle into slot occ (the site's first empty slot) of site s.
-__device__ inline void place_particle(const Params &p, uint32_t *lat, uint32_t s, uint32_t occ, uint32_t particle)
-{
-    clear_zero_flag(p, p.word_particles ? occ : occ >> 2, s);
-    if (p.word_particles) {
-        store_agent(lat + (size_t)occ * p.N + s, particle);
-    } else {
-        uint32_t *wp = lat + (size_t)(occ >> 2) * p.N + s;
-        const uint32_t old = load_agent(wp);
-        store_agent(wp, old | (particle << (8 * (occ & 3))));
-        if ((occ >> 2) > 0) clear_chunk_flag(p, lat, occ >> 2, s >> 2);
-    }
-}
-
-__device__ inline void set_error(Control *ctl, uint32_t code, uint32_t step)
-{
-    if (atomicCAS(&ctl->error, 0u, code) == 0u) ctl->error_step = step;
-}
-
-constexpr int kResolveThreads = 256;
-
-__device__ void resolve_body(const Params &p, uint32_t *lat)
-{
-    __shared__ unsigned long long keys[kMaxOverflows];
-    __shared__ int best;
-    __shared__ uint32_t s_t;
-    Control *ctl = p.ctl;
-    const int tid = threadIdx.x;
-    if (tid == 0) s_t = ctl->timestep;
-    const uint32_t n = ctl->ovf_count;
-    __syncthreads();
-    // The step's reaction phase has consumed the reaction list.
-    for (int k = tid; k < kListShards; k += (int)blockDim.x) ctl->list_count[k] = 0u;
-    if (tid == 0) ctl->list_overflow = 0u;
-    const uint32_t t = s_t;
-    const uint32_t carried = p.relaxed ? ctl->carry_count : 0u;
-    if (n == 0 && carried == 0) {
-        if (tid == 0) ctl->timestep = t + 1;
-        return;
-    }
-    if (n > kMaxOverflows || carried + n > kMaxOverflows) {
-        if (tid == 0) {
-            set_error(ctl, kErrOverflowCap, t);
-            ctl->ovf_count = 0;
-            ctl->timestep = t + 1;
-        }
-        return;
-    }
-    uint32_t M = 2;
-    while (M < n) M <<= 1;
-    for (uint32_t k = tid; k < M; k += kResolveThreads) keys[k] = (k < n) ? ctl->ovf_keys[k] : ~0ull;
-    __syncthreads();
-    for (uint32_t k = 2; k <= M; k <<= 1) {
-        for (uint32_t j = k >> 1; j > 0; j >>= 1) {
-            for (uint32_t a = tid; a < M; a += kResolveThreads) {
-                const uint32_t b = a ^ j;
-                if (b > a) {
-                    const unsigned long long ka = keys[a], kb = keys[b];
-                    const bool up = (a & k) == 0;
-                    if ((ka > kb) == up) {
-                        keys[a] = kb;
-                        keys[b] = ka;
-                    }
-                }
-            }
-            __syncthreads();
-        }
-    }
-
-    if (p.relaxed) {
-        // Relaxed handler (correct_overflows, MpdRdmeSolver.cu:1677-1761): the
-        // carried entries, then this step's in canonical order, each into its
-        // own site's first empty slot; entries of one site go in that order
-        // (the kernel's rounds) and different sites do not interact, so one
-        // thread walks the list.  A full site keeps the entry for the next step.
-        if (tid == 0) {
-            uint32_t kept = 0;
-            for (uint32_t e = 0; e < carried + n; e++) {
-                uint32_t site, particle;
-                if (e < carried) {
-                    site = ctl->carry_site[e];
-                    particle = ctl->carry_part[e];
-                } else {
-                    const unsigned long long key = keys[e - carried];
-                    site = (uint32_t)((key >> 24) & 0xFFFFFFFFull);
-                    particle = ctl->ovf_part[key & 0x7FFull];
-                }
-                const uint32_t occ = site_occupancy(p, lat, site);
-                if (occ < p.P) {
-                    place_particle(p, lat, site, occ, particle);
-                } else {
-                    ctl->carry_site[kept] = site;  // kept <= e: entry e has been read
-                    ctl->carry_part[kept] = particle;
-                    kept++;
-                }
-            }
-            ctl->carry_count = kept;
-            ctl->ovf_total += n;
-            if (n > 0) ctl->ovf_steps += 1;
-            ctl->ovf_count = 0;
-            ctl->timestep = t + 1;
-        }
-        return;
-    }
-
-    const uint32_t X = p.X, Y = p.Y, Z = p.Z;
-    bool failed = false;
-    for (uint32_t e = 0; e < n && !failed; e++) {
-        const unsigned long long key = keys[e];
-        const uint32_t site = (uint32_t)((key >> 24) & 0xFFFFFFFFull);
-        const uint32_t particle = ctl->ovf_part[key & 0x7FFull];
-        const uint32_t xc = site % X, yc = (site / X) % Y, zc = site / p.XY;
-        const uint32_t st0 = p.sites[site];
-        int found = 0x7fffffff;
-        for (uint32_t R = 0; R <= kMaxReplacementDist && found == 0x7fffffff; R++) {
-            const uint32_t minD = R > 0 ? R - 1 : 0;
-            const uint32_t x0 = xc >= R ? xc - R : 0, x1 = (xc <= X - 1 - R) ? xc + R : X - 1;
-            const uint32_t y0 = yc >= R ? yc - R : 0, y1 = (yc <= Y - 1 - R) ? yc + R : Y - 1;
-            const uint32_t z0 = zc >= R ? zc - R : 0, z1 = (zc <= Z - 1 - R) ? zc + R : Z - 1;
-            const uint32_t ny = y1 - y0 + 1, nz = z1 - z0 + 1;
-            const uint32_t total = (x1 - x0 + 1) * ny * nz;
-            for (uint32_t base = 0; base < total; base += kResolveThreads) {
-                if (tid == 0) best = 0x7fffffff;
-                __syncthreads();
-                const uint32_t c = base + tid;
-                if (c < total) {
-                    const uint32_t x = x0 + c / (ny * nz);
-                    const uint32_t rem = c % (ny * nz);
-                    const uint32_t y = y0 + rem / nz;
-                    const uint32_t z = z0 + rem % nz;
-                    const long long dx = (long long)x - xc, dy = (long long)y - yc, dz = (long long)z - zc;
-                    const long long r2 = dx * dx + dy * dy + dz * dz;
-                    const bool shell = r2 <= (long long)(R * R) && (r2 > (long long)(minD * minD) || R == 0);
-                    if (shell) {
-                        if (x >= X || y >= Y || z >= Z) {
-                            atomicMin(&best, (int)(2 * c + 1));
-                        } else {
-                            const uint32_t s2 = x + X * y + p.XY * z;
-                            if (p.sites[s2] == st0 && site_occupancy(p, lat, s2) < p.P)
-                                atomicMin(&best, (int)(2 * c));
-                        }
-                    }
-                }
-                __syncthreads();
-                const int b = best;
-                __syncthreads();
-                if (b != 0x7fffffff) {
-                    found = b;
-                    break;
-                }
-            }
-            if (found != 0x7fffffff) {
-                if (found & 1) {
-                    if (tid == 0) set_error(ctl, kErrOutOfRange, t);
-                    failed = true;
-                } else if (tid == 0) {
-                    const uint32_t c = (uint32_t)found >> 1;
-                    const uint32_t x = x0 + c / (ny * nz);
-                    const uint32_t rem = c % (ny * nz);
-                    const uint32_t y = y0 + rem / nz;
-                    const uint32_t z = z0 + rem % nz;
-                    const uint32_t s2 = x + X * y + p.XY * z;
-                    place_particle(p, lat, s2, site_occupancy(p, lat, s2), particle);
-                }
-            }
-        }
-        if (found == 0x7fffffff) {
-            if (tid == 0) set_error(ctl, kErrUnplaceable, t);
-            failed = true;
-        }
-        __syncthreads();
-    }
-    if (tid == 0) {
-        ctl->ovf_total += n;
-        ctl->ovf_steps += 1;
-        ctl->ovf_count = 0;
-        ctl->timestep = t + 1;
-    }
-}
-
 __global__ __launch_bounds__(kResolveThreads) void resolve_kernel(Params p, uint32_t *lat)
 {
-    resolve_body(p, lat);
+    resolve_body<kResolveThreads>(p, lat);
 }
 
 // Batched resolver: block r resolves member r's step on its post-step buffer
@@ -312,7 +96,7 @@ __global__ __launch_bounds__(kResolveThreads) void batch_resolve_kernel(Member *
 {
     Member &M = m[blockIdx.x];
     uint32_t *const before = M.lat[0], *const after = M.lat[1];
-    resolve_body(M.p, after);
+    resolve_body<kResolveThreads>(M.p, after);
     __syncthreads();  // every wave has read both pointers (resolve_body returns block-uniformly)
     if (threadIdx.x == 0) {
         M.lat[0] = after;

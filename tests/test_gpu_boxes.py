@@ -71,14 +71,14 @@ def test_boxes_are_the_default_where_they_fit(gpu):
     spec = models.bimolecular(shape=(32, 32, 32), nA=300, nB=300, seed=3)
     s = lmx.MpdRdmeSolver(0)
     spec.load_into(s, seed=2)
-    assert _kernels(s, 1) == {"fused", "reaction", "resolve"}
+    assert _kernels(s, 1) == {"fused", "reaction"}
     rng = np.random.default_rng(1)
     full = rng.integers(1, 4, (32, 32, 32, 8)).astype(np.uint8)
     full[..., 4:] = 0  # four particles a site
     s.setLattice(full)
     assert "sweep_z" in _kernels(s, 1)
     s.setLattice(spec.lattice)
-    assert _kernels(s, 1) == {"fused", "reaction", "resolve"}
+    assert _kernels(s, 1) == {"fused", "reaction"}
     s.setLaunchOption(lmx._lib.OPT_BOXES, 0)
     assert "sweep_z" in _kernels(s, 1)
     s.close()
