@@ -56,6 +56,32 @@ inline BoxGeom box_geom(uint32_t X, uint32_t Y, uint32_t Z, uint32_t most)
     return g;
 }
 
+// Blocks of the boxed step's two launches.
+constexpr uint32_t kReactThreads = 1024u, kShardWaves = 4u, kShardThreads = 64u * kShardWaves,
+                   kReactShards = kReactThreads / kShardThreads;
+inline uint32_t box_blocks(const BoxGeom &g)
+{
+    return (g.nboxes + 8u * g.chunk - 1u) / (8u * g.chunk) * 8u * g.chunk;
+}
+inline uint32_t box_react_blocks(const BoxGeom &g)
+{
+    return (std::min(g.nboxes, (uint32_t)kListShards) + kReactShards - 1u) / kReactShards;
+}
+
+// A step of a batch's member in boxes.  A run has three sets of jobs: its first
+// step (which may read an unpacked lattice), the odd ones and the later even
+// ones.
+constexpr uint32_t kBoxJobSets = 3u;
+__host__ __device__ inline uint32_t box_job_set(uint32_t step) { return step == 0u ? 0u : 2u - (step & 1u); }
+struct BoxJob {
+    Params p;
+    BoxGeom g;
+    const uint32_t *src, *zs;
+    uint32_t *dst, *zd;
+    CandList cand;
+    uint32_t first_box, first_react, react_blocks;  // its blocks of the two launches
+};
+
 // Particles a box's region may hold (its records are kept in LDS).
 constexpr int box_cap(uint32_t P) { return P == 16 ? 1024 : 768; }
 

@@ -41,12 +41,19 @@ hipError_t launch_reaction_fast(const Params &p, uint32_t *lat, hipStream_t st);
 hipError_t launch_prob_tables(const Params &p, float *prob1, float *prob0, hipStream_t st);
 // The boxed step (mpd_box.hip): one timestep from src to dst without the
 // reactions and the overflow resolution, which are launch_box_reactions's (a
-// model without reactions takes launch_resolve instead).  zs and zd are the zero flags of the two buffers, rl the
-// reaction candidates (any capacity is correct).
+// model without reactions takes launch_resolve instead).  zs and zd are the
+// zero flags of the two buffers, rl the reaction candidates (any capacity is
+// correct).
 struct CandList;
 hipError_t launch_box_step(const Params &p, const BoxGeom &g, const uint32_t *src, uint32_t *dst, const uint32_t *zs,
                            uint32_t *zd, const CandList &rl, hipStream_t st);
-hipError_t launch_box_reactions(const Params &p, uint32_t *lat, const CandList &rl, hipStream_t st);
+hipError_t launch_box_reactions(const Params &p, const BoxGeom &g, uint32_t *lat, const CandList &rl, hipStream_t st);
+// A step of a batch's boxed members (byte lattice of W words, X % 4 == 0): all
+// their boxes in one launch, then all their reactions and overflow entries.
+// jobs: the step's set; map: the member of each of the boxes, then of each of
+// the reacts blocks.
+struct BoxJob;
+hipError_t launch_box_jobs(const BoxJob *jobs, const uint32_t *map, uint32_t boxes, uint32_t reacts, uint32_t W, hipStream_t st);
 // Resident runs (mpd_resident.hip) of n solvers of one layout: a single job by
 // value (jobs null) or n jobs in device memory, each gathered by `per` blocks.
 struct ResidentJob;

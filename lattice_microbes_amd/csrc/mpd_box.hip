@@ -593,6 +593,22 @@ __global__ __launch_bounds__(kBoxThreads, OCC) void box_step_kernel(Params p, Bo
     box_body<L, CAP, VEC>(p, g, src, dst, zs, zd, rl, p.ctl->timestep, logical, lds);
 }
 
+// The boxes of a batch's members in one launch: map gives a block's member.
+template <class L, int CAP, int OCC>
+__global__ __launch_bounds__(kBoxThreads, OCC) void box_jobs_kernel(const BoxJob *__restrict__ jobs,
+                                                                    const uint32_t *__restrict__ map)
+{
+    __shared__ BoxLds<L, CAP> lds;
+    const BoxJob &job = jobs[map[blockIdx.x]];
+    const Params &p = job.p;
+    const BoxGeom &g = job.g;
+    const uint32_t b = blockIdx.x - job.first_box;  // (a multiple of 8 before it: the XCD order holds)
+    const uint32_t q = b >> 3, ch = fast_div(q, g.div_chunk);
+    const uint32_t logical = (ch * 8u + (b & 7u)) * g.chunk + (q - ch * g.chunk);
+    if (logical >= g.nboxes) return;
+    box_body<L, CAP, true>(p, g, job.src, job.dst, job.zs, job.zd, job.cand, p.ctl->timestep, logical, lds);
+}
+
 // ---------------------------------------------------------------------------
 // Reaction phase of the candidate sites that the boxes listed, one wave per
 // shard, and the step's overflow resolution by the block that ends last.  A
@@ -608,9 +624,6 @@ __global__ __launch_bounds__(kBoxThreads, OCC) void box_step_kernel(Params p, Bo
 // resolver (a launch of its own before): whole cell 256x256x512 27.0 -> 16.3
 // us, 64x64x256 uint32 lattice 21 -> 14.5, crowded P = 16 26 -> 16.7.
 // ---------------------------------------------------------------------------
-
-constexpr uint32_t kReactThreads = 1024, kShardWaves = 4, kShardThreads = 64u * kShardWaves,
-                   kReactShards = kReactThreads / kShardThreads;
 
 __device__ inline uint32_t lane_of(uint32_t v, uint32_t src)
 {
@@ -811,8 +824,10 @@ __device__ inline void wave_react(const Params &p, uint32_t *__restrict__ lat, u
     }
 }
 
+// Block `block` of a solver's nblocks.
 template <class L>
-__global__ __launch_bounds__(kReactThreads) void cand_react_kernel(Params p, uint32_t *__restrict__ lat, CandList rl)
+__device__ __attribute__((always_inline)) inline void cand_react_body(const Params &p, uint32_t *__restrict__ lat,
+                                                                      const CandList &rl, uint32_t block, uint32_t nblocks)
 {
     constexpr int W = L::W;
     constexpr uint32_t P = L::P;
@@ -820,9 +835,9 @@ __global__ __launch_bounds__(kReactThreads) void cand_react_kernel(Params p, uin
     Control *ctl = p.ctl;
     const unsigned long long h3 = timestep_hash(p.seed32, ctl->timestep, 3);
     const bool full = ctl->list_overflow != 0u;
-    const uint32_t shard = blockIdx.x * kReactShards + threadIdx.x / kShardThreads, rank = threadIdx.x % kShardThreads;
+    const uint32_t shard = block * kReactShards + threadIdx.x / kShardThreads, rank = threadIdx.x % kShardThreads;
     const uint32_t n = full ? p.N : ctl->list_count[shard];
-    const uint32_t first = full ? shard * kShardThreads : 0u, step = full ? (uint32_t)kListShards * kShardThreads : kShardThreads;
+    const uint32_t first = full ? shard * kShardThreads : 0u, step = full ? nblocks * kReactThreads : kShardThreads;
 #pragma unroll 1
     for (uint32_t k0 = first; k0 < n; k0 += step) {
         // (a wave of the shard takes every kShardWaves-th entry, so that the
@@ -880,7 +895,7 @@ __global__ __launch_bounds__(kReactThreads) void cand_react_kernel(Params p, uin
     __syncthreads();
     if (threadIdx.x == 0) {
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-        last = atomicAdd(&ctl->blocks_done, 1u) == gridDim.x - 1u ? 1u : 0u;
+        last = atomicAdd(&ctl->blocks_done, 1u) == nblocks - 1u ? 1u : 0u;
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
     }
     __syncthreads();
@@ -889,11 +904,26 @@ __global__ __launch_bounds__(kReactThreads) void cand_react_kernel(Params p, uin
     resolve_body<kReactThreads>(p, lat);
 }
 
+template <class L>
+__global__ __launch_bounds__(kReactThreads) void cand_react_kernel(Params p, uint32_t *__restrict__ lat, CandList rl)
+{
+    cand_react_body<L>(p, lat, rl, blockIdx.x, gridDim.x);
+}
+
+// A batch's members after box_jobs_kernel's same step.
+template <class L>
+__global__ __launch_bounds__(kReactThreads) void cand_react_jobs_kernel(const BoxJob *__restrict__ jobs,
+                                                                        const uint32_t *__restrict__ map)
+{
+    const BoxJob &job = jobs[map[blockIdx.x]];
+    cand_react_body<L>(job.p, job.dst, job.cand, blockIdx.x - job.first_react, job.react_blocks);
+}
+
 template <class L, int CAP, int OCC>
 static hipError_t launch_box(const Params &p, const BoxGeom &g, const uint32_t *src, uint32_t *dst, const uint32_t *zs,
                              uint32_t *zd, const CandList &rl, hipStream_t st)
 {
-    const dim3 grid((g.nboxes + 8u * g.chunk - 1u) / (8u * g.chunk) * 8u * g.chunk), block(kBoxThreads);
+    const dim3 grid(box_blocks(g)), block(kBoxThreads);
     if ((p.X & 3u) == 0)
         hipLaunchKernelGGL((box_step_kernel<L, CAP, true, OCC>), grid, block, 0, st, p, g, src, dst, zs, zd, rl);
     else
@@ -901,11 +931,11 @@ static hipError_t launch_box(const Params &p, const BoxGeom &g, const uint32_t *
     return hipGetLastError();
 }
 
-hipError_t launch_box_reactions(const Params &p, uint32_t *lat, const CandList &rl, hipStream_t st)
+hipError_t launch_box_reactions(const Params &p, const BoxGeom &g, uint32_t *lat, const CandList &rl, hipStream_t st)
 {
     Params q = p;
     q.packed = 1u;  // the step has packed every site
-    const dim3 grid(kListShards / kReactShards), block(kReactThreads);
+    const dim3 grid(box_react_blocks(g)), block(kReactThreads);
     switch (p.word_particles ? 100 + (int)p.P : (int)p.W) {
     case 1: hipLaunchKernelGGL((cand_react_kernel<ByteSites<1>>), grid, block, 0, st, q, lat, rl); break;
     case 2: hipLaunchKernelGGL((cand_react_kernel<ByteSites<2>>), grid, block, 0, st, q, lat, rl); break;
@@ -931,6 +961,24 @@ hipError_t launch_box_step(const Params &p, const BoxGeom &g, const uint32_t *sr
     case 116: return launch_box<WordSites<16>, box_cap(16), 4>(p, g, src, dst, zs, zd, rl, st);
     }
     return hipErrorInvalidValue;
+}
+
+template <int W, int OCC>
+static void launch_jobs(const BoxJob *jobs, const uint32_t *map, uint32_t boxes, uint32_t reacts, hipStream_t st)
+{
+    hipLaunchKernelGGL((box_jobs_kernel<ByteSites<W>, box_cap(4 * W), OCC>), dim3(boxes), dim3(kBoxThreads), 0, st, jobs, map);
+    hipLaunchKernelGGL((cand_react_jobs_kernel<ByteSites<W>>), dim3(reacts), dim3(kReactThreads), 0, st, jobs, map + boxes);
+}
+
+hipError_t launch_box_jobs(const BoxJob *jobs, const uint32_t *map, uint32_t boxes, uint32_t reacts, uint32_t W, hipStream_t st)
+{
+    switch (W) {
+    case 1: launch_jobs<1, 6>(jobs, map, boxes, reacts, st); break;
+    case 2: launch_jobs<2, 6>(jobs, map, boxes, reacts, st); break;
+    case 4: launch_jobs<4, 6>(jobs, map, boxes, reacts, st); break;
+    default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
 }
 
 }  // namespace lmx

@@ -458,6 +458,22 @@ bool use_boxes(const lmx_solver *s)
            !s->force_generic;
 }
 
+// The reaction list's memory holds the candidates: four site indices a unit.
+lmx::CandList cand_list(const lmx::ReactionList &rl)
+{
+    return lmx::CandList{reinterpret_cast<uint32_t *>(rl.rec), rl.cap * 4u};
+}
+
+// The boxed step's zero flags, cleared if they do not describe the lattice.
+int fresh_zero_flags(lmx_solver *s, hipStream_t st)
+{
+    if (s->zflags_fresh) return LMX_OK;
+    const hipError_t e = lmx::launch_fill(s->d_zflags, 2 * (size_t)s->W * s->box.nboxes, 0u, st);
+    if (e != hipSuccess) return hip_fail(e, "zero flag fill launch");
+    s->zflags_fresh = true;
+    return LMX_OK;
+}
+
 // One timestep (runTimestep, MpdRdmeSolver.cu:996-1193).  ev, if given,
 // receives events around each launch (ev[0] before the first launch, then one
 // after every launch); kinds receives the kernel class of each launch.
@@ -485,11 +501,7 @@ int enqueue_step(lmx_solver *s, const lmx::Params &p0, hipEvent_t *ev, int *kind
     const bool fast = !s->force_generic && lmx::fast_path_ok(p);
     if (use_boxes(s)) {
         const size_t nz = (size_t)s->W * s->box.nboxes;
-        if (!s->zflags_fresh) {
-            e = lmx::launch_fill(s->d_zflags, 2 * nz, 0u, s->stream);
-            if (e != hipSuccess) return hip_fail(e, "zero flag fill launch");
-            s->zflags_fresh = true;
-        }
+        if (int rc = fresh_zero_flags(s, s->stream)) return rc;
         s->flags_fresh = false;
         p.plane_flags = 0u;
         uint32_t *zs = s->d_zflags + s->cur * nz, *zd = s->d_zflags + (1 - s->cur) * nz;
@@ -498,14 +510,13 @@ int enqueue_step(lmx_solver *s, const lmx::Params &p0, hipEvent_t *ev, int *kind
             e = hipEventRecord(ev[0], s->stream);
             if (e != hipSuccess) return hip_fail(e, "hipEventRecord");
         }
-        // the reaction list's memory holds the candidates: four site indices a unit
-        const lmx::CandList cand{reinterpret_cast<uint32_t *>(rlist.rec), rlist.cap * 4u};
+        const lmx::CandList cand = cand_list(rlist);
         e = lmx::launch_box_step(p, s->box, s->d_lat[s->cur], s->d_lat[1 - s->cur], zs, zd, cand, s->stream);
         if (e != hipSuccess) return hip_fail(e, "boxed step launch");
         s->cur = 1 - s->cur;
         if (int rc = mark(LMX_K_FUSED)) return rc;
         if (s->R > 0) {
-            e = lmx::launch_box_reactions(p, s->d_lat[s->cur], cand, s->stream);
+            e = lmx::launch_box_reactions(p, s->box, s->d_lat[s->cur], cand, s->stream);
             if (e != hipSuccess) return hip_fail(e, "reaction launch");
             if (int rc = mark(LMX_K_REACTION)) return rc;  // and the resolver
         } else {
@@ -1595,9 +1606,13 @@ struct lmx_batch {
     hipStream_t stream = nullptr;
     hipEvent_t done = nullptr;
     std::vector<lmx_solver *> members;
-    // of the run being enqueued: the members the batched kernels step, and
-    // those that run in a block of their own
-    std::vector<lmx_solver *> stepped, resident;
+    // of the run being enqueued: the members the batched sweeps step, those
+    // that step in boxes and those that run in a block of their own
+    std::vector<lmx_solver *> stepped, boxed, resident;
+    uint32_t box_cap = 0, box_total = 0, react_total = 0;
+    size_t box_map_cap = 0;
+    lmx::BoxJob *d_boxes = nullptr, *h_boxes = nullptr;
+    uint32_t *d_box_map = nullptr, *h_box_map = nullptr;  // member of each block of the two launches
     hipStream_t stream2 = nullptr;   // resident runs, beside the batched steps
     hipEvent_t fork = nullptr, join = nullptr;
     uint32_t jobs_cap = 0;
@@ -1711,34 +1726,97 @@ int batch_finish(lmx_batch *b, uint32_t nsteps)
         s->packed = true;
         s->zflags_fresh = false;
     }
+    for (lmx_solver *s : b->boxed) {
+        if (nsteps & 1u) s->cur = 1 - s->cur;
+        s->timestep += nsteps;
+        s->packed = true;
+        s->flags_fresh = false;
+    }
     for (lmx_solver *s : b->resident) resident_ran(s, nsteps);
     for (lmx_solver *s : b->members) LMX_HIP(hipStreamWaitEvent(s->stream, b->done, 0));
     return LMX_OK;
 }
 
-// The members of a run of nsteps: the ones with few particles run in a block
-// of their own each, beside the batched steps of the others (unless an option
-// of the batched kernels was set).  The 256 replicates of the ensemble
-// workload hold 2000 particles on 32^3 to 128^3 sites: the batched sweeps pay
-// 1.3 ms a step for their 1.8e8 sites.
+// Room for n entries of a batch's array on the device and in pinned memory.
+template <class T, class N>
+int batch_room(T *&dev, T *&host, N &cap, size_t n, size_t least)
+{
+    if (n <= cap) return LMX_OK;
+    size_t want = cap ? cap : least;
+    while (want < n) want *= 2;
+    dev_free(dev);
+    if (host) hipHostFree(host);
+    host = nullptr;
+    cap = 0;
+    LMX_HIP(hipMalloc((void **)&dev, sizeof(T) * want));
+    LMX_HIP(hipHostMalloc((void **)&host, sizeof(T) * want, hipHostMallocDefault));
+    cap = (N)want;
+    return LMX_OK;
+}
+
+// Descriptors of the members that step in boxes and the members of the two
+// launches' blocks.
+int batch_boxes(lmx_batch *b)
+{
+    const uint32_t n = (uint32_t)b->boxed.size();
+    if (int rc = batch_room(b->d_boxes, b->h_boxes, b->box_cap, (size_t)lmx::kBoxJobSets * n, 48)) return rc;
+    b->box_total = b->react_total = 0;
+    for (uint32_t r = 0; r < n; r++) {
+        lmx_solver *s = b->boxed[r];
+        if (int rc = fresh_zero_flags(s, b->stream)) return rc;
+        const size_t nz = (size_t)s->W * s->box.nboxes;
+        for (uint32_t set = 0; set < lmx::kBoxJobSets; set++) {
+            lmx::BoxJob &job = b->h_boxes[(size_t)set * n + r];
+            const int from = set == 1u ? 1 - s->cur : s->cur, to = 1 - from;
+            job.p = make_params(s);
+            if (set > 0) job.p.packed = 1u;
+            job.p.zero_flags = s->d_zflags + to * nz;
+            job.g = s->box;
+            job.src = s->d_lat[from];
+            job.dst = s->d_lat[to];
+            job.zs = s->d_zflags + from * nz;
+            job.zd = s->d_zflags + to * nz;
+            job.cand = cand_list(s->rlist);
+            job.first_box = b->box_total;
+            job.first_react = b->react_total;
+            job.react_blocks = lmx::box_react_blocks(s->box);
+        }
+        b->box_total += lmx::box_blocks(s->box);
+        b->react_total += lmx::box_react_blocks(s->box);
+    }
+    const size_t blocks = (size_t)b->box_total + b->react_total;
+    if (int rc = batch_room(b->d_box_map, b->h_box_map, b->box_map_cap, blocks, 4096)) return rc;
+    for (uint32_t r = 0; r < n; r++) {
+        const lmx::BoxJob &job = b->h_boxes[r];
+        uint32_t *map = b->h_box_map + job.first_box, *react = b->h_box_map + b->box_total + job.first_react;
+        std::fill(map, map + lmx::box_blocks(job.g), r);
+        std::fill(react, react + job.react_blocks, r);
+    }
+    if (n == 0) return LMX_OK;
+    LMX_HIP(hipMemcpyAsync(b->d_boxes, b->h_boxes, sizeof(lmx::BoxJob) * lmx::kBoxJobSets * n, hipMemcpyHostToDevice,
+                           b->stream));
+    LMX_HIP(hipMemcpyAsync(b->d_box_map, b->h_box_map, sizeof(uint32_t) * blocks, hipMemcpyHostToDevice, b->stream));
+    return LMX_OK;
+}
+
+// The members of a run of nsteps: unless an option of the batched kernels was
+// set, the ones with few particles run in a block of their own each, beside
+// the steps of the others, and those whose particles fit boxes step in them,
+// as they would alone; the batched sweeps step the rest.  (The 256 replicates
+// of the ensemble workload hold 2000 particles on 32^3 to 128^3 sites: the
+// batched sweeps pay 1.3 ms a step for their 1.8e8 sites.  12 members of 64^3,
+// 64x64x256 and capsule lattices: 480 us a step in sweeps, 142 in boxes.)
 int batch_jobs(lmx_batch *b, uint32_t nsteps)
 {
     b->stepped.clear();
+    b->boxed.clear();
     b->resident.clear();
     const bool alone = b->use_list && b->tile_threads == 0;
-    for (lmx_solver *s : b->members) (alone && use_resident(s, nsteps) ? b->resident : b->stepped).push_back(s);
+    for (lmx_solver *s : b->members)
+        (!alone ? b->stepped : (use_resident(s, nsteps) ? b->resident : (use_boxes(s) ? b->boxed : b->stepped))).push_back(s);
+    if (int rc = batch_boxes(b)) return rc;
     const uint32_t n = (uint32_t)b->resident.size();
-    if (n > b->jobs_cap) {
-        uint32_t cap = b->jobs_cap ? b->jobs_cap : 16;
-        while (cap < n) cap *= 2;
-        dev_free(b->d_jobs);
-        if (b->h_jobs) hipHostFree(b->h_jobs);
-        b->h_jobs = nullptr;
-        b->jobs_cap = 0;
-        LMX_HIP(hipMalloc((void **)&b->d_jobs, sizeof(lmx::ResidentJob) * cap));
-        LMX_HIP(hipHostMalloc((void **)&b->h_jobs, sizeof(lmx::ResidentJob) * cap, hipHostMallocDefault));
-        b->jobs_cap = cap;
-    }
+    if (int rc = batch_room(b->d_jobs, b->h_jobs, b->jobs_cap, n, 16)) return rc;
     for (uint32_t r = 0; r < n; r++) b->h_jobs[r] = resident_job(b->resident[r], nsteps);
     if (n)
         LMX_HIP(hipMemcpyAsync(b->d_jobs, b->h_jobs, sizeof(lmx::ResidentJob) * n, hipMemcpyHostToDevice, b->stream));
@@ -1910,6 +1988,10 @@ int lmx_batch_destroy(lmx_batch *b)
     if (b->staged) hipEventDestroy(b->staged);
     dev_free(b->d_jobs);
     if (b->h_jobs) hipHostFree(b->h_jobs);
+    dev_free(b->d_boxes);
+    if (b->h_boxes) hipHostFree(b->h_boxes);
+    dev_free(b->d_box_map);
+    if (b->h_box_map) hipHostFree(b->h_box_map);
     if (b->fork) hipEventDestroy(b->fork);
     if (b->join) hipEventDestroy(b->join);
     if (b->stream2) hipStreamDestroy(b->stream2);
@@ -2005,6 +2087,11 @@ int lmx_batch_run_steps(lmx_batch *b, uint32_t nsteps)
             const hipError_t e = lmx::launch_resident(lmx::ResidentJob{}, b->d_jobs, nr, per, b->W * 4, false, b->stream2);
             if (e != hipSuccess) return hip_fail(e, "resident run launch");
             LMX_HIP(hipEventRecord(b->join, b->stream2));
+        }
+        for (uint32_t i = 0; i < nsteps && !b->boxed.empty(); i++) {
+            const hipError_t e = lmx::launch_box_jobs(b->d_boxes + b->boxed.size() * lmx::box_job_set(i), b->d_box_map,
+                                                      b->box_total, b->react_total, b->W, b->stream);
+            if (e != hipSuccess) return hip_fail(e, "batched boxed step launch");
         }
         if (b->stepped.empty()) {
         } else if (b->use_graph) {

@@ -118,3 +118,32 @@ def test_crowded_boxes_are_cut(gpu, per_site, P, words):
         assert np.array_equal(got, orc.native()), f"{(got != orc.native()).sum()} words differ"
     assert s.getOverflowStats()[0] == orc.stats.overflow_entries
     s.close()
+
+
+@pytest.mark.parametrize("P", [4, 8, 16])
+def test_batch_of_boxed_members(gpu, P):
+    """Members that step in boxes share two launches a step: lattices of one
+    and of many boxes, births, no reactions, a reflecting edge, and one that
+    an outside write left unpacked, beside one in sweeps (too crowded)."""
+    ens = lmx.Ensemble(0)
+    pairs = []
+    for k, (shape, density, R) in enumerate([((16, 14, 14), 0.02, 6), ((36, 27, 29), 0.02, 6), ((64, 48, 40), 0.02, 0),
+                                             ((20, 70, 17), 0.06, 9), ((16, 12, 12), 0.4, 6)]):
+        spec = models.random_model(shape=shape, P=P, nS=5, nST=3, R=R, density=density, seed=50 + k, rate_scale=0.05,
+                                   boundary="reflecting" if k % 2 else "periodic", include_zero_order=k in (0, 3))
+        s = lmx.MpdRdmeSolver(0)
+        spec.load_into(s, replicate=k, seed=3)
+        ens.add(s)
+        pairs.append((s, oracle.Oracle(spec, seed_top=3, replicate=k)))
+    s, orc = pairs[2]  # its slots reversed: the first step reads sites with holes
+    slots = np.ascontiguousarray(s.getLatticeNative()).reshape(P // 4, -1, 1).view(np.uint8)
+    s.setLatticeNative(np.ascontiguousarray(slots[::-1, :, ::-1]).view(np.uint32).reshape(orc.native().shape))
+    orc.lattice[:] = s.getLatticeNative().reshape(-1)
+    for chunk in (1, 2, 3):
+        ens.run(chunk)
+        for s, orc in pairs:
+            assert orc.run(chunk) == 0
+            got, ref = s.getLatticeNative(), orc.native()
+            assert np.array_equal(got, ref), f"{s.shape}: {(got != ref).sum()} words differ"
+            assert s.getOverflowStats()[0] == orc.stats.overflow_entries
+    ens.close()
