@@ -80,8 +80,19 @@ hipError_t launch_batch_resolve(Member *m, uint32_t n, hipStream_t st);
 hipError_t launch_copy(const void *src, void *dst, size_t bytes, int num_cu, hipStream_t st);
 hipError_t launch_fill(uint32_t *ptr, size_t n, uint32_t value, hipStream_t st);
 hipError_t launch_validate(const Params &p, const uint32_t *lat, hipStream_t st);
-hipError_t launch_counts(const uint32_t *lat, size_t nwords, uint32_t nS, bool words, uint32_t *counts,
+// Species counts of nwords lattice words to host memory (out, nS entries);
+// counts: nS + 1 zeroed device words, left zeroed.
+hipError_t launch_counts(const uint32_t *lat, size_t nwords, uint32_t nS, bool words, uint32_t *counts, uint32_t *out,
                          hipStream_t st);
+// The first kReportWords words of up to kReportMost control blocks to host
+// memory, kReportWords apart.
+constexpr uint32_t kReportWords = 16u, kReportMost = 256u;
+static_assert(offsetof(Control, box_splits) / sizeof(uint32_t) < kReportWords, "the report ends with box_splits");
+struct ReportList {
+    const Control *ctl[kReportMost];
+    uint32_t n;
+};
+hipError_t launch_report(const ReportList &c, uint32_t *out, hipStream_t st);
 hipError_t launch_exp(const double *x, double *y, size_t n, hipStream_t st);
 hipError_t launch_prob(const float *a, float *y, size_t n, hipStream_t st);
 

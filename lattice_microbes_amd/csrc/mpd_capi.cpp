@@ -101,7 +101,7 @@ struct lmx_solver {
     // Diffusion model and lattice.
     uint32_t nST = 0, X = 0, Y = 0, Z = 0, P = 0, W = 0;
     uint32_t bpp = 1;  // bytes per particle: 1 (byte lattice) or 4 (uint32 lattice, one particle per word)
-    uint32_t counts_cap = 256;  // entries of d_counts
+    uint32_t counts_cap = 0;  // species that d_counts and h_report hold
     // Every site of the current lattice holds its particles in its first
     // slots.  The kernels keep this; a lattice written from outside (native
     // words, device pointers) may break it until the next step.
@@ -129,7 +129,11 @@ struct lmx_solver {
     uint32_t *d_rx_off = nullptr, *d_rx_list = nullptr, *d_sto_off = nullptr, *d_sto_sp = nullptr;
     int32_t *d_sto_val = nullptr;
     lmx::Control *d_ctl = nullptr;
-    uint32_t *d_counts = nullptr;
+    uint32_t *d_counts = nullptr;  // counts_cap + 1, zero between counts
+    uint32_t *h_report = nullptr;  // pinned: kReportWords of the control block, then the counts
+    // Steps (or a validation) may have left an error that the host has not
+    // looked for yet; own_work: on the solver's own stream.
+    bool unchecked = true, own_work = true;
     bool tables_dirty = false;
     uint32_t timestep = 0;
     bool any_qp0 = false;
@@ -401,15 +405,36 @@ void plan_boxes(lmx_solver *s, const std::vector<uint32_t> &at)
     set_box_level(s, lmx::kBoxLevels);
 }
 
+// The report on the solver's stream, after whatever was enqueued there.
+int fetch_report(lmx_solver *s)
+{
+    lmx::ReportList c{};
+    c.ctl[0] = s->d_ctl;
+    c.n = 1;
+    const hipError_t e = lmx::launch_report(c, s->h_report, s->stream);
+    if (e != hipSuccess) return hip_fail(e, "report launch");
+    LMX_HIP(hipStreamSynchronize(s->stream));
+    s->own_work = false;
+    return LMX_OK;
+}
+
+int check_report(lmx_solver *s, const uint32_t *hdr);
+
+// Waits for the solver's stream and reports the steps' errors.
 int check_device_error(lmx_solver *s)
 {
-    uint32_t hdr[offsetof(lmx::Control, box_splits) / sizeof(uint32_t) + 1];
-    LMX_HIP(hipMemcpy(hdr, s->d_ctl, sizeof(hdr), hipMemcpyDeviceToHost));
+    if (int rc = fetch_report(s)) return rc;
+    return check_report(s, s->h_report);
+}
+
+// hdr: the head of the control block after the steps so far.
+int check_report(lmx_solver *s, const uint32_t *hdr)
+{
     if (s->res_pending) {
         if (hdr[0] != s->timestep) {
             if (int rc = settle(s)) return rc;
-            LMX_HIP(hipStreamSynchronize(s->stream));
-            LMX_HIP(hipMemcpy(hdr, s->d_ctl, sizeof(hdr), hipMemcpyDeviceToHost));
+            if (int rc = fetch_report(s)) return rc;
+            hdr = s->h_report;
         }
         s->res_pending = false;
     }
@@ -421,6 +446,7 @@ int check_device_error(lmx_solver *s)
         set_box_level(s, s->box_level + 1);
     s->splits_seen += splits;
     s->splits_step = s->timestep;
+    s->unchecked = hdr[2] != 0 || s->own_work;
     switch (hdr[2]) {
     case 0: return LMX_OK;
     case lmx::kErrOverflowCap:
@@ -482,6 +508,7 @@ int enqueue_step(lmx_solver *s, const lmx::Params &p0, hipEvent_t *ev, int *kind
                  const lmx::ReactionList *rl_in = nullptr)
 {
     const lmx::ReactionList &rlist = rl_in ? *rl_in : s->rlist;
+    s->unchecked = s->own_work = true;
     // The step writes packed sites whatever it reads, so only its first
     // kernel may see an unpacked lattice; every launch of this step takes the
     // current flag, and the next step may rely on packing.
@@ -637,7 +664,7 @@ void resident_ran(lmx_solver *s, uint32_t nsteps)
     s->timestep += nsteps;
     s->packed = true;
     s->flags_fresh = s->zflags_fresh = false;
-    s->res_pending = true;
+    s->res_pending = s->unchecked = true;
 }
 
 // nsteps timesteps: a resident run, or one step's launches after another.
@@ -650,6 +677,7 @@ int enqueue_steps(lmx_solver *s, uint32_t nsteps, const lmx::ReactionList *rl = 
                                                       s->P, s->bpp == 4, s->stream);
             if (e != hipSuccess) return hip_fail(e, "resident run launch");
             resident_ran(s, m);
+            s->own_work = true;
             nsteps -= m;
         }
         return LMX_OK;
@@ -677,6 +705,21 @@ int settle(lmx_solver *s)
     s->timestep = t;
     s->resident_ok = false;
     return enqueue_steps(s, missing);
+}
+
+// Buffers of the report and of the counts of up to `species` species.
+hipError_t alloc_counts(lmx_solver *s, uint32_t species)
+{
+    dev_free(s->d_counts);
+    if (s->h_report) hipHostFree(s->h_report);
+    s->h_report = nullptr;
+    s->counts_cap = 0;
+    hipError_t e = hipMalloc((void **)&s->d_counts, ((size_t)species + 1) * sizeof(uint32_t));
+    if (e == hipSuccess)
+        e = hipHostMalloc((void **)&s->h_report, (lmx::kReportWords + (size_t)species) * sizeof(uint32_t), hipHostMallocDefault);
+    if (e == hipSuccess) e = hipMemsetAsync(s->d_counts, 0, ((size_t)species + 1) * sizeof(uint32_t), s->stream);
+    if (e == hipSuccess) s->counts_cap = species;
+    return e;
 }
 
 void free_device(lmx_solver *s)
@@ -740,7 +783,7 @@ int lmx_create(int device, lmx_solver **out)
         if (e == hipSuccess) e = hipStreamCreateWithFlags(&s->stream, hipStreamNonBlocking);
         if (e == hipSuccess) e = hipMalloc((void **)&s->d_ctl, sizeof(lmx::Control));
         if (e == hipSuccess) e = hipMemset(s->d_ctl, 0, sizeof(lmx::Control));
-        if (e == hipSuccess) e = hipMalloc((void **)&s->d_counts, 256 * sizeof(uint32_t));
+        if (e == hipSuccess) e = alloc_counts(s, 256);
         int ncu = 0;
         if (e == hipSuccess) e = hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, device);
         if (ncu > 0) s->num_cu = (uint32_t)ncu;
@@ -763,6 +806,7 @@ int lmx_destroy(lmx_solver *s)
     free_device(s);
     dev_free(s->d_ctl);
     dev_free(s->d_counts);
+    if (s->h_report) hipHostFree(s->h_report);
     if (s->stream) hipStreamDestroy(s->stream);
     delete s;
     return LMX_OK;
@@ -933,12 +977,7 @@ int lmx_build_diffusion_model(lmx_solver *s, uint32_t nST, const double *DF, con
         hipError_t e = hipMalloc((void **)&s->d_lat[0], buf_bytes);
         if (e == hipSuccess) e = hipMalloc((void **)&s->d_lat[1], buf_bytes);
         if (e == hipSuccess) e = hipMalloc((void **)&s->d_sites, s->N);
-        if (e == hipSuccess && s->nS > s->counts_cap) {
-            hipFree(s->d_counts);
-            s->d_counts = nullptr;
-            e = hipMalloc((void **)&s->d_counts, (size_t)s->nS * sizeof(uint32_t));
-            s->counts_cap = e == hipSuccess ? s->nS : 0u;
-        }
+        if (e == hipSuccess && s->nS > s->counts_cap) e = alloc_counts(s, s->nS);
         // The reaction list: kListShards shards of cap records (index, W words,
         // type).  Any capacity is correct (an overflowing shard makes the
         // reaction phase a full pass); N/8 entries in total hold every occupied
@@ -1097,9 +1136,7 @@ int lmx_synchronize(lmx_solver *s)
     if (!s) return fail(LMX_ERR_ARG, "null solver");
     int rc = select_device(s);
     if (rc) return rc;
-    LMX_HIP(hipStreamSynchronize(s->stream));
-    if (s->d_ctl) return check_device_error(s);
-    return LMX_OK;
+    return check_device_error(s);
 }
 
 int lmx_get_timestep(lmx_solver *s, uint32_t *t)
@@ -1211,8 +1248,11 @@ int lmx_device_lattice(lmx_solver *s, void **particles, void **sites)
     int rc = require_ready(s);
     if (rc) return rc;
     if (!particles || !sites) return fail(LMX_ERR_ARG, "null argument");
-    LMX_HIP(hipStreamSynchronize(s->stream));
-    if ((rc = check_device_error(s))) return rc;
+    if (s->unchecked) {
+        if ((rc = check_device_error(s))) return rc;
+    } else {
+        LMX_HIP(hipStreamSynchronize(s->stream));
+    }
     *particles = s->d_lat[s->cur];
     *sites = s->d_sites;
     s->packed = false;  // the caller may write any slot
@@ -1228,7 +1268,6 @@ int lmx_validate_lattice(lmx_solver *s)
     const lmx::Params p = make_params(s);
     hipError_t e = lmx::launch_validate(p, s->d_lat[s->cur], s->stream);
     if (e != hipSuccess) return hip_fail(e, "validate launch");
-    LMX_HIP(hipStreamSynchronize(s->stream));
     return check_device_error(s);
 }
 
@@ -1269,12 +1308,10 @@ int lmx_get_species_counts(lmx_solver *s, uint32_t *counts, uint32_t n)
         int rc = require_ready(s);
         if (rc) return rc;
         if (!counts || n < s->nS) return fail(LMX_ERR_ARG, "counts buffer smaller than the number of species");
-        LMX_HIP(lmx::launch_fill(s->d_counts, s->counts_cap, 0u, s->stream));
-        hipError_t e = lmx::launch_counts(s->d_lat[s->cur], s->N * s->W, s->nS, s->bpp == 4, s->d_counts, s->stream);
+        uint32_t *const h = s->h_report + lmx::kReportWords;
+        hipError_t e = lmx::launch_counts(s->d_lat[s->cur], s->N * s->W, s->nS, s->bpp == 4, s->d_counts, h, s->stream);
         if (e != hipSuccess) return hip_fail(e, "count launch");
         LMX_HIP(hipStreamSynchronize(s->stream));
-        std::vector<uint32_t> h(s->counts_cap);
-        LMX_HIP(hipMemcpy(h.data(), s->d_counts, s->counts_cap * sizeof(uint32_t), hipMemcpyDeviceToHost));
         for (uint32_t i = 0; i < n; i++) counts[i] = i < s->nS ? h[i] : 0u;
         return LMX_OK;
     });
@@ -1612,6 +1649,8 @@ struct lmx_batch {
     uint32_t box_cap = 0, box_total = 0, react_total = 0;
     size_t box_map_cap = 0;
     lmx::BoxJob *d_boxes = nullptr, *h_boxes = nullptr;
+    size_t report_cap = 0;
+    uint32_t *h_report = nullptr;                         // the members' reports
     uint32_t *d_box_map = nullptr, *h_box_map = nullptr;  // member of each block of the two launches
     hipStream_t stream2 = nullptr;   // resident runs, beside the batched steps
     hipEvent_t fork = nullptr, join = nullptr;
@@ -1662,7 +1701,10 @@ int member_ready(lmx_solver *s, bool may_alloc)
         if (rc) return rc;
     }
     if (int rc = settle(s)) return rc;
-    LMX_HIP(hipStreamSynchronize(s->stream));
+    if (s->own_work) {
+        LMX_HIP(hipStreamSynchronize(s->stream));
+        s->own_work = false;
+    }
     return LMX_OK;
 }
 
@@ -1733,7 +1775,10 @@ int batch_finish(lmx_batch *b, uint32_t nsteps)
         s->flags_fresh = false;
     }
     for (lmx_solver *s : b->resident) resident_ran(s, nsteps);
-    for (lmx_solver *s : b->members) LMX_HIP(hipStreamWaitEvent(s->stream, b->done, 0));
+    for (lmx_solver *s : b->members) {
+        s->unchecked = true;
+        LMX_HIP(hipStreamWaitEvent(s->stream, b->done, 0));
+    }
     return LMX_OK;
 }
 
@@ -1991,6 +2036,7 @@ int lmx_batch_destroy(lmx_batch *b)
     dev_free(b->d_boxes);
     if (b->h_boxes) hipHostFree(b->h_boxes);
     dev_free(b->d_box_map);
+    if (b->h_report) hipHostFree(b->h_report);
     if (b->h_box_map) hipHostFree(b->h_box_map);
     if (b->fork) hipEventDestroy(b->fork);
     if (b->join) hipEventDestroy(b->join);
@@ -2109,14 +2155,31 @@ int lmx_batch_run_steps(lmx_batch *b, uint32_t nsteps)
 
 int lmx_batch_synchronize(lmx_batch *b)
 {
-    if (!b) return fail(LMX_ERR_ARG, "null batch");
-    LMX_HIP(hipSetDevice(b->device));
-    LMX_HIP(hipStreamSynchronize(b->stream));
-    for (lmx_solver *s : b->members) {
-        int rc = check_device_error(s);
-        if (rc) return rc;
-    }
-    return LMX_OK;
+    return guarded([&]() -> int {
+        if (!b) return fail(LMX_ERR_ARG, "null batch");
+        LMX_HIP(hipSetDevice(b->device));
+        // All members' reports in one wait (a copy and a wait for each took
+        // 15 us a member).
+        const size_t n = b->members.size();
+        if (n > b->report_cap) {
+            if (b->h_report) hipHostFree(b->h_report);
+            b->h_report = nullptr;
+            b->report_cap = 0;
+            LMX_HIP(hipHostMalloc((void **)&b->h_report, 2 * n * lmx::kReportWords * sizeof(uint32_t), hipHostMallocDefault));
+            b->report_cap = 2 * n;
+        }
+        for (size_t r0 = 0; r0 < n; r0 += lmx::kReportMost) {
+            lmx::ReportList c{};
+            c.n = (uint32_t)std::min<size_t>(n - r0, lmx::kReportMost);
+            for (uint32_t k = 0; k < c.n; k++) c.ctl[k] = b->members[r0 + k]->d_ctl;
+            const hipError_t e = lmx::launch_report(c, b->h_report + r0 * lmx::kReportWords, b->stream);
+            if (e != hipSuccess) return hip_fail(e, "report launch");
+        }
+        LMX_HIP(hipStreamSynchronize(b->stream));
+        for (size_t r = 0; r < n; r++)
+            if (int rc = check_report(b->members[r], b->h_report + r * lmx::kReportWords)) return rc;
+        return LMX_OK;
+    });
 }
 
 int lmx_batch_autotune(lmx_batch *b, uint32_t nsteps, double *best_ms, int *chosen)

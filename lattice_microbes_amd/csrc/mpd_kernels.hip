@@ -7,8 +7,8 @@
 //  resolve_kernel   canonical-order overflow placement on the device (the
 //                   classic host handler, MpdRdmeSolver.cu:1103-1189, or the
 //                   relaxed correct_overflows, :1677-1761)
-//  count_kernel     species counts (ByteLattice::getParticleCounts; the
-//                   uint32 lattice's in count_words_kernel)
+//  count_kernel     species counts (ByteLattice::getParticleCounts,
+//                   IntLattice::getParticleCounts)
 //
 // Every per-particle decision depends only on (site index, slot, timestep,
 // substep) through the counter-based hash, so the results do not depend on
@@ -106,41 +106,78 @@ __global__ __launch_bounds__(kResolveThreads) void batch_resolve_kernel(Member *
     }
 }
 
-// ---------------------------------------------------------------------------
-// Species counts (ByteLattice::getParticleCounts, ByteLattice.cpp:495-520):
-// each word counts up to its first empty byte.
-// ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void count_kernel(const uint32_t *__restrict__ lat, size_t nwords,
-                                                    uint32_t nS, uint32_t *__restrict__ counts)
+// Species counts: slot bytes up to a word's first empty one
+// (ByteLattice::getParticleCounts, ByteLattice.cpp:495-520), or the words of
+// the uint32 lattice (IntLattice::getParticleCounts, IntLattice.cpp:419-435:
+// every nonzero word is one particle).  Reading the lattice bounds it, so a
+// thread reads 16 bytes at a time and blocks count in LDS; counts has nS
+// entries and the number of finished blocks behind them, all zero, and the
+// block that ends last hands the counts to host memory and zeroes them again:
+// one launch, and no copy, for what took three calls.
+template <bool WORDS>
+__global__ __launch_bounds__(256) void count_kernel(const uint32_t *__restrict__ lat, size_t nwords, uint32_t nS,
+                                                    uint32_t *counts, uint32_t *out)
 {
-    __shared__ uint32_t hist[256];
-    for (uint32_t k = threadIdx.x; k < 256; k += blockDim.x) hist[k] = 0;
+    constexpr uint32_t kCountBins = WORDS ? 1024u : 256u;
+    __shared__ uint32_t hist[kCountBins], last;
+    for (uint32_t k = threadIdx.x; k < kCountBins; k += blockDim.x) hist[k] = 0;
     __syncthreads();
-    for (size_t wi = (size_t)blockIdx.x * blockDim.x + threadIdx.x; wi < nwords;
-         wi += (size_t)gridDim.x * blockDim.x) {
-        const uint32_t word = lat[wi];
-        if (word == 0) continue;
-        for (int b = 0; b < 4; b++) {
-            const uint32_t s = (word >> (8 * b)) & 0xFFu;
-            if (s == 0) break;
-            atomicAdd(&hist[s], 1u);
+    auto add = [&](uint32_t sp) {
+        if (sp < kCountBins) atomicAdd(&hist[sp], 1u);
+        else if (sp <= nS) atomicAdd(&counts[sp - 1], 1u);
+    };
+    auto word_of = [&](uint32_t word) {
+        if (WORDS) {
+            if (word) add(word);
+            return;
+        }
+        while (word & 0xFFu) {
+            add(word & 0xFFu);
+            word >>= 8;
+        }
+    };
+    const size_t tid = (size_t)blockIdx.x * blockDim.x + threadIdx.x, threads = (size_t)gridDim.x * blockDim.x;
+    const uint4 *lat4 = reinterpret_cast<const uint4 *>(lat);
+    const size_t n4 = nwords / 4;
+    for (size_t k = tid; k < n4; k += 2 * threads) {
+        const bool two = k + threads < n4;
+        const uint4 u = lat4[k], v = two ? lat4[k + threads] : make_uint4(0u, 0u, 0u, 0u);
+        if (u.x | u.y | u.z | u.w) {
+            word_of(u.x);
+            word_of(u.y);
+            word_of(u.z);
+            word_of(u.w);
+        }
+        if (v.x | v.y | v.z | v.w) {
+            word_of(v.x);
+            word_of(v.y);
+            word_of(v.z);
+            word_of(v.w);
         }
     }
+    for (size_t k = 4 * n4 + tid; k < nwords; k += threads) word_of(lat[k]);
     __syncthreads();
-    for (uint32_t k = threadIdx.x; k < 256; k += blockDim.x)
-        if (k >= 1 && k <= nS && hist[k]) atomicAdd(&counts[k - 1], hist[k]);
+    for (uint32_t k = threadIdx.x + 1u; k < kCountBins && k <= nS; k += blockDim.x)
+        if (hist[k]) atomicAdd(&counts[k - 1], hist[k]);
+    __threadfence();
+    __syncthreads();
+    if (threadIdx.x == 0) last = atomicAdd(&counts[nS], 1u) == gridDim.x - 1u ? 1u : 0u;
+    __syncthreads();
+    if (!last) return;
+    __threadfence();
+    for (uint32_t k = threadIdx.x; k < nS; k += blockDim.x) {
+        out[k] = load_agent(&counts[k]);
+        counts[k] = 0u;
+    }
+    if (threadIdx.x == 0) counts[nS] = 0u;
 }
 
-// Species counts of the uint32 lattice (IntLattice::getParticleCounts,
-// IntLattice.cpp:419-435): every nonzero word is one particle.
-__global__ __launch_bounds__(256) void count_words_kernel(const uint32_t *__restrict__ lat, size_t nwords,
-                                                          uint32_t nS, uint32_t *__restrict__ counts)
+// The first words of solvers' control blocks to host memory.
+__global__ void report_kernel(ReportList c, uint32_t *out)
 {
-    for (size_t wi = (size_t)blockIdx.x * blockDim.x + threadIdx.x; wi < nwords;
-         wi += (size_t)gridDim.x * blockDim.x) {
-        const uint32_t s = lat[wi];
-        if (s >= 1 && s <= nS) atomicAdd(&counts[s - 1], 1u);
-    }
+    const uint32_t k = threadIdx.x % kReportWords;
+    for (uint32_t m = threadIdx.x / kReportWords; m < c.n; m += blockDim.x / kReportWords)
+        out[m * kReportWords + k] = load_agent(reinterpret_cast<const uint32_t *>(c.ctl[m]) + k);
 }
 
 // Range check of a lattice changed on the device by a caller: particle
@@ -277,16 +314,21 @@ hipError_t launch_batch_resolve(Member *m, uint32_t n, hipStream_t st)
     return hipGetLastError();
 }
 
-hipError_t launch_counts(const uint32_t *lat, size_t nwords, uint32_t nS, bool words, uint32_t *counts,
+hipError_t launch_counts(const uint32_t *lat, size_t nwords, uint32_t nS, bool words, uint32_t *counts, uint32_t *out,
                          hipStream_t st)
 {
-    unsigned g = blocks_for(nwords, 256);
-    if (g > 4096) g = 4096;
-    if (g == 0) g = 1;
+    const unsigned g = std::min(std::max(blocks_for(nwords / 8, 256), 1u), 1024u);
     if (words)
-        hipLaunchKernelGGL(count_words_kernel, dim3(g), dim3(256), 0, st, lat, nwords, nS, counts);
+        hipLaunchKernelGGL(count_kernel<true>, dim3(g), dim3(256), 0, st, lat, nwords, nS, counts, out);
     else
-        hipLaunchKernelGGL(count_kernel, dim3(g), dim3(256), 0, st, lat, nwords, nS, counts);
+        hipLaunchKernelGGL(count_kernel<false>, dim3(g), dim3(256), 0, st, lat, nwords, nS, counts, out);
+    return hipGetLastError();
+}
+
+hipError_t launch_report(const ReportList &c, uint32_t *out, hipStream_t st)
+{
+    const uint32_t threads = std::min((c.n * kReportWords + 63u) / 64u * 64u, 1024u);
+    hipLaunchKernelGGL(report_kernel, dim3(1), dim3(threads), 0, st, c, out);
     return hipGetLastError();
 }
 

@@ -628,7 +628,7 @@ class DeviceHookLattice:
         else:
             shape, typestr = (s.particlesPerSite // 4, Z, Y, X, 4), "|u1"
         self._particles = torch.as_tensor(_DeviceArray(pp.value, shape, typestr), device=self._dev)
-        self._sites = torch.as_tensor(_DeviceArray(sp.value, (Z, Y, X), "|u1"), device=self._dev)
+        self._sites = sp.value
 
     def synchronize(self) -> None:
         self._torch.cuda.synchronize(self._dev)
@@ -638,6 +638,9 @@ class DeviceHookLattice:
         return self._particles
 
     def getSiteLatticeView(self):
+        if isinstance(self._sites, int):  # most hooks never look at it
+            X, Y, Z = self._solver.shape
+            self._sites = self._torch.as_tensor(_DeviceArray(self._sites, (Z, Y, X), "|u1"), device=self._dev)
         return self._sites
 
     def getXSize(self) -> int:
