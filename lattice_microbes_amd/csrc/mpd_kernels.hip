@@ -159,12 +159,11 @@ __global__ __launch_bounds__(256) void count_kernel(const uint32_t *__restrict__
     __syncthreads();
     for (uint32_t k = threadIdx.x + 1u; k < kCountBins && k <= nS; k += blockDim.x)
         if (hist[k]) atomicAdd(&counts[k - 1], hist[k]);
-    __threadfence();
+    __builtin_amdgcn_s_waitcnt(0);  // the additions are done
     __syncthreads();
     if (threadIdx.x == 0) last = atomicAdd(&counts[nS], 1u) == gridDim.x - 1u ? 1u : 0u;
     __syncthreads();
     if (!last) return;
-    __threadfence();
     for (uint32_t k = threadIdx.x; k < nS; k += blockDim.x) {
         out[k] = load_agent(&counts[k]);
         counts[k] = 0u;
