@@ -380,29 +380,45 @@ void set_box_level(lmx_solver *s, uint32_t level)
 // several times the cost, so the rule leaves room for fluctuations; on the
 // 128x64x80 bimolecular lattice (P = 8) the sweeps take 26-64 us a step from
 // 0.01 to 0.4 particles a site, the boxes that fit 18-38 us.
+// Smaller ones than those while their blocks still run all at once: a launch
+// then lasts as long as its fullest block, of which smaller boxes are shorter
+// (capsule 128x128x256, boxes of 14 -> 10: 25.6 -> 22.4 us a step; 63x61x151,
+// 6 -> 4: 28.6 -> 24.5; 96x96x96 with births, 14 -> 8: 27.8 -> 26.0).  Past
+// that their shells cost more: 256x256x128, 14 -> 10, 3741 boxes with
+// particles: 50.6 -> 59.7; the capsule in 4096 boxes of 8: 23.7.  Nor are
+// boxes of a wave's worth of particles any shorter when smaller (64x64x64,
+// 2000 particles, 14 -> 4: 16.4 -> 20.0).
 void plan_boxes(lmx_solver *s, const std::vector<uint32_t> &at)
 {
     s->particles = at.size();
     s->resident_ok = s->d_res != nullptr;
     const uint32_t cap = (uint32_t)lmx::box_cap(s->P);
     if (at.size() > s->N) return set_box_level(s, lmx::kBoxLevels);  // more than a particle a site: no box fits
+    constexpr uint32_t kAtOnce = 1024u, kBoxesAtOnce = 3072u;  // boxes with particles, boxes
+    constexpr uint32_t kShort = 64u;                           // particles that one wave moves at once
     std::vector<uint32_t> n, ybox(s->Y), zbox(s->Z);
+    uint32_t fits = lmx::kBoxLevels;  // the level taken so far
     for (uint32_t level = 0; level < lmx::kBoxLevels; level++) {
         const lmx::BoxGeom g = lmx::box_geom(s->X, s->Y, s->Z, lmx::kBoxLevel[level]);
         const double region = (double)(lmx::kBoxX + 2) * (g.TY + 2) * (g.TZ + 2) / ((double)lmx::kBoxX * g.TY * g.TZ);
         const double most = 0.75 * cap / region;
         if ((double)at.size() > most * g.nboxes) continue;  // the mean box is too full already
+        if (fits < lmx::kBoxLevels && g.nboxes > kBoxesAtOnce) break;
         for (uint32_t y = 0; y < s->Y; y++) ybox[y] = g.nbx * (y / g.TY);
         for (uint32_t z = 0; z < s->Z; z++) zbox[z] = g.nbx * g.nby * (z / g.TZ);
         n.assign(g.nboxes, 0u);
-        uint32_t full = 0;
+        uint32_t full = 0, active = 0;
         for (uint32_t i : at) {
             const uint32_t r = i / s->X, z = r / s->Y;
-            full = std::max(full, ++n[(i - r * s->X) / lmx::kBoxX + ybox[r - z * s->Y] + zbox[z]]);
+            uint32_t &count = n[(i - r * s->X) / lmx::kBoxX + ybox[r - z * s->Y] + zbox[z]];
+            active += count++ == 0u ? 1u : 0u;
+            full = std::max(full, count);
         }
-        if (full <= most) return set_box_level(s, level);
+        if (fits < lmx::kBoxLevels && active > kAtOnce) break;
+        if (full <= most) fits = level;
+        if (fits < lmx::kBoxLevels && (active > kAtOnce || full <= kShort)) break;
     }
-    set_box_level(s, lmx::kBoxLevels);
+    set_box_level(s, fits);
 }
 
 // The report on the solver's stream, after whatever was enqueued there.
