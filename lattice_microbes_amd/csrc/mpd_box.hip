@@ -621,8 +621,8 @@ __global__ __launch_bounds__(kBoxThreads, OCC) void box_jobs_kernel(const BoxJob
 // loops over slots are rolled, which keeps the kernel at 13 kB of code (71 kB
 // unrolled), and a shard's entries are dealt to four waves, so that its
 // reacting sites rarely queue behind one another.  Measured, with the
-// resolver (a launch of its own before): whole cell 256x256x512 27.0 -> 16.3
-// us, 64x64x256 uint32 lattice 21 -> 14.5, crowded P = 16 26 -> 16.7.
+// resolver (a launch of its own before): whole cell 256x256x512 27.0 -> 15.3
+// us, 256x256x128 uint32 lattice 21 -> 13.4, crowded P = 16 26 -> 15.4.
 // ---------------------------------------------------------------------------
 
 __device__ inline uint32_t lane_of(uint32_t v, uint32_t src)
@@ -891,13 +891,12 @@ __device__ __attribute__((always_inline)) inline void cand_react_body(const Para
     }
     // The block that ends last resolves the step's overflow entries.
     __shared__ uint32_t last;
+    // (What it reads of this launch, lattice words and entries, is stored and
+    // loaded at device scope, so waiting for the stores is enough: no fence,
+    // which would write back and invalidate the L2.)
     __builtin_amdgcn_s_waitcnt(0);  // every wave's stores have arrived
     __syncthreads();
-    if (threadIdx.x == 0) {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-        last = atomicAdd(&ctl->blocks_done, 1u) == nblocks - 1u ? 1u : 0u;
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-    }
+    if (threadIdx.x == 0) last = atomicAdd(&ctl->blocks_done, 1u) == nblocks - 1u ? 1u : 0u;
     __syncthreads();
     if (!last) return;
     if (threadIdx.x == 0) ctl->blocks_done = 0u;

@@ -1866,7 +1866,7 @@ int batch_boxes(lmx_batch *b)
 // as they would alone; the batched sweeps step the rest.  (The 256 replicates
 // of the ensemble workload hold 2000 particles on 32^3 to 128^3 sites: the
 // batched sweeps pay 1.3 ms a step for their 1.8e8 sites.  12 members of 64^3,
-// 64x64x256 and capsule lattices: 480 us a step in sweeps, 142 in boxes.)
+// 256x256x128 and capsule lattices: 480 us a step in sweeps, 142 in boxes.)
 int batch_jobs(lmx_batch *b, uint32_t nsteps)
 {
     b->stepped.clear();
