@@ -29,11 +29,14 @@
 // about 1000 instructions per 64.
 //
 // What bounds it (whole-cell 256x256x512, P = 8, 1e6 particles, rocprofv3): one
-// launch 125 us against 303 us for the sweeps (x 77, y 105, z 119), 30.4e6
-// vector instructions against 151e6, 0.35 GB of HBM traffic against 0.99 GB.  A block
-// lives about 32000 cycles, a third of them the region's load; six blocks of
-// 24 KB LDS and 80 VGPRs share a CU, and vector issue is 45% busy: latency of
-// the dependent phases, then issue.  Versions that kept a list of sites and
+// launch 113 us against 303 us for the sweeps (x 77, y 105, z 119), 30.4e6
+// vector instructions against 151e6, 0.35 GB of HBM traffic against 0.99 GB.  A
+// block lives about 32000 cycles, a third of them the region's load; seven
+// blocks of 20 KB LDS and 72 VGPRs share a CU, and vector issue is half busy:
+// latency of the dependent phases, then issue.  (Six blocks, with 1024 chains
+// and the region's load in one go at 80 VGPRs: whole cell 117 us, 256x256x128
+// uint32 lattice 52 -> 44; eight blocks: whole cell 112, but 96x96x96 with
+// births 17.9 -> 19.0.)  Versions that kept a list of sites and
 // looked each neighbour up in a site map took 244 us (a general path for
 // sites of several particles ran in one wave while the others waited).
 #include "lmx_batch.h"
@@ -49,7 +52,9 @@ namespace {
 
 constexpr uint32_t kNone = 0xFFFFFFFFu;
 constexpr uint32_t kEnd = 0xFFFFu;       // end of a chain
-constexpr uint32_t kChains = 1024u;      // hash chains of a sweep's targets
+// Hash chains of a sweep's targets (1024 of them keep P = 16's fuller boxes at
+// 30.1 us on 128x64x80, 512 at 32.4).
+constexpr uint32_t box_chains(int cap) { return cap > 768 ? 1024u : 512u; }
 
 // A particle's record: its site's key (13 bits), slot (4), class (2: stayed,
 // came from the minus neighbour, came from the plus neighbour) and, on the
@@ -62,10 +67,15 @@ constexpr uint32_t kKeyMask = 0x1FFFu, kDead = 0x1FFFu;
 __device__ inline uint32_t make_key(uint32_t lx, uint32_t ly, uint32_t lz) { return lx | (ly << 5) | (lz << 9); }
 __device__ inline uint32_t rec_order(uint32_t rec) { return (rec >> 13) & 63u; }
 __device__ inline uint32_t rec_slot(uint32_t rec) { return (rec >> 13) & 15u; }
-__device__ inline uint32_t chain_of(uint32_t key) { return (key ^ (key >> 4)) & (kChains - 1u); }
+template <uint32_t kChains>
+__device__ inline uint32_t chain_of(uint32_t key)
+{
+    return (key ^ (key >> 4)) & (kChains - 1u);
+}
 
 template <class L, int CAP>
 struct BoxLds {
+    static constexpr uint32_t kChains = box_chains(CAP);
     // Sweeps alternate between two sets of records, chain links and chain
     // heads, so that a wave may begin the next sweep while others still rank
     // the particles of this one.
@@ -117,6 +127,7 @@ __device__ inline uint32_t wave_slots(uint32_t *counter, uint32_t c)
 
 template <class L, int CAP>
 struct BoxCtx {
+    static constexpr uint32_t kChains = box_chains(CAP);
     const Params &p;
     BoxLds<L, CAP> &s;
     Box b;
@@ -138,7 +149,7 @@ struct BoxCtx {
     {
         before = 0;
         total = 1;
-        uint32_t q = s.head[par][chain_of(rec & kKeyMask)] & 0xFFFFu;
+        uint32_t q = s.head[par][chain_of<kChains>(rec & kKeyMask)] & 0xFFFFu;
         const uint32_t nx = s.next[par][e];
         if (q == e && nx == kEnd) return;
         total = 0;
@@ -174,7 +185,7 @@ __device__ __attribute__((always_inline)) inline bool box_pass(const BoxCtx<L, C
                                                                uint32_t &nz_planes)
 {
     constexpr int W = L::W;
-    constexpr uint32_t P = L::P;
+    constexpr uint32_t P = L::P, kChains = box_chains(CAP);
     const Params &p = c.p;
     auto &s = c.s;
     const uint32_t tid = threadIdx.x;
@@ -207,11 +218,11 @@ __device__ __attribute__((always_inline)) inline bool box_pass(const BoxCtx<L, C
     }
     __syncthreads();
     // Columns 4 gx + 1 .. 4 gx + 4 of a row as one 16-byte load (VEC): U
-    // groups a lane, z planes 4 apart, all in flight together with the V
+    // groups a lane and round, z planes 4 apart, in flight together with the V
     // single sites (the two shell columns; without VEC every column, 32 lanes
     // a row, eight rows at a time).  A lane without a site loads the box's
     // first one, so that no load waits for a branch.
-    constexpr uint32_t U = VEC ? 4 : 0, V = VEC ? 2 : 8, ROUNDS = VEC ? 1 : 4;
+    constexpr uint32_t U = VEC ? 2 : 0, V = VEC ? 1 : 8, ROUNDS = VEC ? 2 : 4;
     const uint32_t gx = tid & 3u, gly = (tid >> 2) & 15u, glz = tid >> 6;
     const uint32_t lx = VEC ? ((tid & 1u) ? b.nx + 1u : 0u) : (tid & 31u);
     auto site_row = [&](uint32_t v) { return VEC ? (tid >> 1) + 128u * v : (tid >> 5) + 8u * v; };
@@ -223,7 +234,7 @@ __device__ __attribute__((always_inline)) inline bool box_pass(const BoxCtx<L, C
         uint32_t ok = 0;  // bit u: group u exists; bit U + u: single site u
 #pragma unroll
         for (uint32_t u = 0; u < U; u++) {
-            const uint32_t row = s.row[gly + 16u * (glz + 4u * u)];
+            const uint32_t row = s.row[gly + 16u * (glz + 4u * (r * U + u))];
             const bool o = row != kNone && 4u * gx < b.nx;
             const uint32_t i = o ? b.x0 + 4u * gx + row : safe;
             v4[u] = *reinterpret_cast<const uint4 *>(src + i);
@@ -244,12 +255,12 @@ __device__ __attribute__((always_inline)) inline bool box_pass(const BoxCtx<L, C
 #pragma unroll
         for (uint32_t u = 0; u < U; u++) {
             if (!((ok >> u) & 1u)) continue;
-            uint16_t *tp = reinterpret_cast<uint16_t *>(s.typ + c.at(make_key(1u + 4u * gx, gly, glz + 4u * u)));
+            uint16_t *tp = reinterpret_cast<uint16_t *>(s.typ + c.at(make_key(1u + 4u * gx, gly, glz + 4u * (r * U + u))));
             tp[0] = (uint16_t)t4[u];
             tp[1] = (uint16_t)(t4[u] >> 16);
             uint4 q4 = v4[u];
             if (!p.packed) {  // a site may be occupied although its word 0 is empty
-                const uint32_t i = b.x0 + 4u * gx + s.row[gly + 16u * (glz + 4u * u)];
+                const uint32_t i = b.x0 + 4u * gx + s.row[gly + 16u * (glz + 4u * (r * U + u))];
                 for (uint32_t k = 1; k < (uint32_t)W; k++) {
                     const uint4 q = *reinterpret_cast<const uint4 *>(src + (size_t)k * p.N + i);
                     q4.x |= q.x;
@@ -274,7 +285,7 @@ __device__ __attribute__((always_inline)) inline bool box_pass(const BoxCtx<L, C
         while (nz) {
             const uint32_t q = (uint32_t)__builtin_ctz(nz);
             nz &= nz - 1;
-            const uint32_t key = q < 4u * U ? make_key(1u + 4u * gx + (q & 3u), gly, glz + (q & ~3u))
+            const uint32_t key = q < 4u * U ? make_key(1u + 4u * gx + (q & 3u), gly, glz + 4u * U * r + (q & ~3u))
                                             : lx | (site_row(r * V + q - 4u * U) << 5);
             if (slot < (uint32_t)CAP) s.next[0][slot] = (uint16_t)key;
             slot++;
@@ -346,7 +357,7 @@ __device__ __attribute__((always_inline)) inline bool box_pass(const BoxCtx<L, C
             if constexpr (VEC) {
                 if (4u * gx < b.nx && gly - 1u < b.ny) {
 #pragma unroll
-                    for (uint32_t u = 0; u < U; u++) {
+                    for (uint32_t u = 0; u < 4u; u++) {
                         if (glz + 4u * u - 1u >= b.nz) continue;
                         const uint32_t i = b.x0 + 4u * gx + s.row[gly + 16u * (glz + 4u * u)];
 #pragma unroll
@@ -401,7 +412,7 @@ __device__ __attribute__((always_inline)) inline bool box_pass(const BoxCtx<L, C
                 s.rec[to][e] = target | (j << 13) | ((plus ? 1u : (minus ? 2u : 0u)) << 17) |
                                (L::kPerWord == 4 ? part << 19 : 0u);
                 const uint32_t tag = axis + 1u;
-                const uint32_t old = atomicExch(&s.head[to][chain_of(target)], e | (tag << 16));
+                const uint32_t old = atomicExch(&s.head[to][chain_of<kChains>(target)], e | (tag << 16));
                 s.next[to][e] = (uint16_t)((old >> 16) == tag ? old & 0xFFFFu : kEnd);
             } else {
                 if constexpr (L::kPerWord == 4)
@@ -454,7 +465,7 @@ __device__ __attribute__((always_inline)) inline bool box_pass(const BoxCtx<L, C
                 if (!(prob[k] > 0.0f && q0[k] != 0.0f)) continue;
                 const uint32_t key = make_key(lx, ly, lz0 + k), i = c.site(key);
                 if (!(uniform01(i, 1, 0, h3) <= prob[k])) continue;
-                const uint32_t hd = s.head[0][chain_of(key)];
+                const uint32_t hd = s.head[0][chain_of<kChains>(key)];
                 bool empty = true;
                 for (uint32_t q = (hd >> 16) == 3u ? hd & 0xFFFFu : kEnd; q != kEnd; q = s.next[0][q])
                     if ((s.rec[0][q] & kKeyMask) == key) empty = false;
@@ -952,8 +963,8 @@ hipError_t launch_box_step(const Params &p, const BoxGeom &g, const uint32_t *sr
 {
     const int key = p.word_particles ? 100 + (int)p.P : (int)p.W;
     switch (key) {
-    case 1: return launch_box<ByteSites<1>, box_cap(4), 6>(p, g, src, dst, zs, zd, rl, st);
-    case 2: return launch_box<ByteSites<2>, box_cap(8), 6>(p, g, src, dst, zs, zd, rl, st);
+    case 1: return launch_box<ByteSites<1>, box_cap(4), 7>(p, g, src, dst, zs, zd, rl, st);
+    case 2: return launch_box<ByteSites<2>, box_cap(8), 7>(p, g, src, dst, zs, zd, rl, st);
     case 4: return launch_box<ByteSites<4>, box_cap(16), 6>(p, g, src, dst, zs, zd, rl, st);
     case 104: return launch_box<WordSites<4>, box_cap(4), 6>(p, g, src, dst, zs, zd, rl, st);
     case 108: return launch_box<WordSites<8>, box_cap(8), 6>(p, g, src, dst, zs, zd, rl, st);
@@ -972,8 +983,8 @@ static void launch_jobs(const BoxJob *jobs, const uint32_t *map, uint32_t boxes,
 hipError_t launch_box_jobs(const BoxJob *jobs, const uint32_t *map, uint32_t boxes, uint32_t reacts, uint32_t W, hipStream_t st)
 {
     switch (W) {
-    case 1: launch_jobs<1, 6>(jobs, map, boxes, reacts, st); break;
-    case 2: launch_jobs<2, 6>(jobs, map, boxes, reacts, st); break;
+    case 1: launch_jobs<1, 7>(jobs, map, boxes, reacts, st); break;
+    case 2: launch_jobs<2, 7>(jobs, map, boxes, reacts, st); break;
     case 4: launch_jobs<4, 6>(jobs, map, boxes, reacts, st); break;
     default: return hipErrorInvalidValue;
     }

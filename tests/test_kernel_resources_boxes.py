@@ -1,6 +1,6 @@
 """Register budget of the boxed step's kernels, from the compiler's report of
-the last build: 80 VGPRs are six blocks of four waves per CU, as many as its
-24 KB of LDS allow, and no spill."""
+the last build: 72 VGPRs are seven blocks of four waves per CU, and its 20 KB
+of LDS leave room for as many, without a spill."""
 import os
 
 import pytest
@@ -18,8 +18,8 @@ def test_box_kernels_do_not_spill(W, vec):
     names = [n for n in res if f"box_step_kernelINS_9ByteSitesILi{W}EE" in n and f"ELb{vec}E" in n]
     assert len(names) == 1, names
     r = res[names[0]]
-    assert r["ScratchSize"] == 0 and r["Occupancy"] >= 6, r
-    assert r["LDS Size"] <= 163840 // 6, r
+    assert r["ScratchSize"] == 0 and r["Occupancy"] >= 7, r
+    assert r["LDS Size"] <= 163840 // 7, r
 
 
 @pytest.mark.parametrize("W", [1, 2])
