@@ -148,13 +148,13 @@ struct lmx_solver {
     lmx::ReactionList rlist{};
     // The boxed step (LMX_OPT_BOXES): its boxes, the level they were taken
     // from (kBoxLevels: too crowded, the sweeps run) and the zero flags of
-    // both buffers (buf * W * nboxes), valid while zflags_fresh.
+    // both buffers (buf * W * nboxes), valid while the buffer's zflags_fresh.
     bool boxes = true;
     lmx::BoxGeom box{};
     uint32_t box_level = lmx::kBoxLevels;
     uint32_t splits_seen = 0, splits_step = 0;  // Control::box_splits and the step when it was last looked at
     uint32_t *d_zflags = nullptr;
-    bool zflags_fresh = false;
+    bool zflags_fresh[2] = {false, false};
     // Resident runs (a solver of few particles in one block): the particles of
     // the lattice as the host last set it, the run's list, and whether a run
     // was enqueued that may have stopped short (settle).
@@ -371,7 +371,7 @@ void set_box_level(lmx_solver *s, uint32_t level)
 {
     s->box_level = level;
     if (level < lmx::kBoxLevels) s->box = lmx::box_geom(s->X, s->Y, s->Z, lmx::kBoxLevel[level]);
-    s->zflags_fresh = false;
+    s->zflags_fresh[0] = s->zflags_fresh[1] = false;
 }
 
 // The boxes for a lattice with particles at the given sites: the largest whose
@@ -509,10 +509,12 @@ lmx::CandList cand_list(const lmx::ReactionList &rl)
 // The boxed step's zero flags, cleared if they do not describe the lattice.
 int fresh_zero_flags(lmx_solver *s, hipStream_t st)
 {
-    if (s->zflags_fresh) return LMX_OK;
-    const hipError_t e = lmx::launch_fill(s->d_zflags, 2 * (size_t)s->W * s->box.nboxes, 0u, st);
+    const size_t nz = (size_t)s->W * s->box.nboxes;
+    const int from = s->zflags_fresh[0] ? 1 : 0, stale = (s->zflags_fresh[0] ? 0 : 1) + (s->zflags_fresh[1] ? 0 : 1);
+    if (stale == 0) return LMX_OK;
+    const hipError_t e = lmx::launch_fill(s->d_zflags + from * nz, stale * nz, 0u, st);
     if (e != hipSuccess) return hip_fail(e, "zero flag fill launch");
-    s->zflags_fresh = true;
+    s->zflags_fresh[0] = s->zflags_fresh[1] = true;
     return LMX_OK;
 }
 
@@ -572,7 +574,7 @@ int enqueue_step(lmx_solver *s, const lmx::Params &p0, hipEvent_t *ev, int *kind
         s->packed = true;
         return LMX_OK;
     }
-    s->zflags_fresh = false;
+    s->zflags_fresh[0] = s->zflags_fresh[1] = false;
     // Chunk flags: kept by the default sweeps-path kernels of the byte
     // lattice (x4, LDS tiles, the reaction phases, the resolver); any other
     // step leaves them stale, so they are zeroed before the next step that
@@ -679,7 +681,7 @@ void resident_ran(lmx_solver *s, uint32_t nsteps)
 {
     s->timestep += nsteps;
     s->packed = true;
-    s->flags_fresh = s->zflags_fresh = false;
+    s->flags_fresh = s->zflags_fresh[0] = s->zflags_fresh[1] = false;
     s->res_pending = s->unchecked = true;
 }
 
@@ -747,7 +749,7 @@ void free_device(lmx_solver *s)
     dev_free(s->d_zflags);
     dev_free(s->d_res);
     s->resident_ok = s->res_pending = false;
-    s->zflags_fresh = false;
+    s->zflags_fresh[0] = s->zflags_fresh[1] = false;
     s->rlist = lmx::ReactionList{};
     dev_free(s->d_T);
     dev_free(s->d_qp0);
@@ -1273,7 +1275,7 @@ int lmx_device_lattice(lmx_solver *s, void **particles, void **sites)
     *sites = s->d_sites;
     s->packed = false;  // the caller may write any slot
     s->flags_fresh = false;
-    s->zflags_fresh = false;
+    s->zflags_fresh[s->cur] = false;  // (the other buffer is not handed out)
     return LMX_OK;
 }
 
@@ -1397,7 +1399,7 @@ int lmx_autotune(lmx_solver *s, uint32_t nsteps, double *best_ms, int *chosen)
             s->cur = cur0;
             s->packed = packed0;
             s->flags_fresh = fresh0;
-            s->zflags_fresh = false;
+            s->zflags_fresh[0] = s->zflags_fresh[1] = false;
             return LMX_OK;
         };
 
@@ -1782,7 +1784,7 @@ int batch_finish(lmx_batch *b, uint32_t nsteps)
         if (nsteps & 1u) s->cur = 1 - s->cur;
         s->timestep += nsteps;
         s->packed = true;
-        s->zflags_fresh = false;
+        s->zflags_fresh[0] = s->zflags_fresh[1] = false;
     }
     for (lmx_solver *s : b->boxed) {
         if (nsteps & 1u) s->cur = 1 - s->cur;
@@ -2249,7 +2251,7 @@ int lmx_batch_autotune(lmx_batch *b, uint32_t nsteps, double *best_ms, int *chos
                     s->cur = v.cur;
                     s->packed = v.packed;
                     s->flags_fresh = v.fresh;
-                    s->zflags_fresh = s->res_pending = false;
+                    s->zflags_fresh[0] = s->zflags_fresh[1] = s->res_pending = false;
                 }
             }
             return LMX_OK;
