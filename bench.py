@@ -344,9 +344,11 @@ def ensemble_bench(nrep: int, steps: int, seed: int, sync_steps: int):
     for L in models.ENSEMBLE_SIZES:
         spec = next(m[0] for m in mix if m[0].shape[0] == L)
         row = {}
-        for name, path in (("sweeps", lmx._lib.PATH_SWEEPS), ("fused", lmx._lib.PATH_FUSED)):
+        for name, path in (("default", None), ("sweeps", lmx._lib.PATH_SWEEPS), ("fused", lmx._lib.PATH_FUSED)):
             s = make(spec, 0, 7)
-            s.setPath(path)
+            if path is not None:
+                s.setLaunchOption(lmx._lib.OPT_BOXES, 0)
+                s.setPath(path)
             s.runTimesteps(2)
             t, _ = s.timeSteps(200)
             row[name + "_us_per_step"] = t / 200 * 1e3
@@ -376,9 +378,9 @@ def ensemble_bench(nrep: int, steps: int, seed: int, sync_steps: int):
 
 def uint32_bench(spec, steps: int, seed: int, copy_gbps: float):
     """The same model on the uint32 lattice (IntMpdRdmeSolver) with every
-    species id raised by 300 past a byte: per-step time and HBM rate of its
-    one-site-per-thread kernels (2*4P+1 B/site per sweep, 4P+1 B/site for the
-    reaction phase)."""
+    species id raised by 300 past a byte: per-step time and HBM rate of the
+    boxed step (8P+1 B/site), or of its one-site-per-thread sweeps (8P+1 B/site
+    each, 4P+1 B/site for the reaction phase)."""
     import lattice_microbes_amd as lmx
     from lattice_microbes_amd.models import ModelSpec
 
@@ -406,7 +408,7 @@ def uint32_bench(spec, steps: int, seed: int, copy_gbps: float):
         w.close()
     N, P = spec.N, spec.P
     sweep_b, react_b = (8 * P + 1) * N, (4 * P + 1) * N
-    step_b = 3 * sweep_b + (react_b if spec.R else 0)
+    step_b = sweep_b if "fused" in per else 3 * sweep_b + (react_b if spec.R else 0)
     ms = total_ms / steps
     gbps = step_b / (ms / 1e3) / 1e9
     return {"workload": f"{spec.name} {spec.shape[0]}x{spec.shape[1]}x{spec.shape[2]}, species ids +{off} "

@@ -29,11 +29,11 @@
 // about 1000 instructions per 64.
 //
 // What bounds it (whole-cell 256x256x512, P = 8, 1e6 particles, rocprofv3): one
-// launch 113 us against 303 us for the sweeps (x 77, y 105, z 119), 30.4e6
-// vector instructions against 151e6, 0.35 GB of HBM traffic against 0.99 GB.  A
+// launch 113 us against 303 us for the sweeps (x 77, y 105, z 119), 34.8e6
+// vector instructions against 151e6, 0.32 GB of HBM traffic against 0.99 GB.  A
 // block lives about 32000 cycles, a third of them the region's load; seven
-// blocks of 20 KB LDS and 72 VGPRs share a CU, and vector issue is half busy:
-// latency of the dependent phases, then issue.  (Six blocks, with 1024 chains
+// blocks of 20 KB LDS and 72 VGPRs share a CU, and vector issue takes 65 of the
+// 113 us: latency of the dependent phases, then issue.  (Six blocks, with 1024 chains
 // and the region's load in one go at 80 VGPRs: whole cell 117 us, 256x256x128
 // uint32 lattice 52 -> 44; eight blocks: whole cell 112, but 96x96x96 with
 // births 17.9 -> 19.0.)  Versions that kept a list of sites and

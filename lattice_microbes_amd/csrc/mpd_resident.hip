@@ -14,7 +14,7 @@
 // so there is no shell, and the lattice is read and written once per run.
 //
 // Why: a step of a small lattice is launches, not work.  The bimolecular 64^3
-// model (2000 particles) takes 17 us a step in boxes, three launches of which
+// model (2000 particles) takes 16.5 us a step in boxes, two launches of which
 // none fills the device, and an ensemble pays every member's lattice in every
 // step although its members hold 2000 particles each.  One block steps them in
 // 11.8 us (12.4 us on 32^3, where 60 sites hold several particles), and an
