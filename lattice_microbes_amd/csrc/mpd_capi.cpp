@@ -436,6 +436,13 @@ int fetch_report(lmx_solver *s)
 
 int check_report(lmx_solver *s, const uint32_t *hdr);
 
+// Every resident run enqueued so far took all its steps.
+void resident_ended(lmx_solver *s)
+{
+    s->res_pending = false;
+    s->packed = true;
+}
+
 // Waits for the solver's stream and reports the steps' errors.
 int check_device_error(lmx_solver *s)
 {
@@ -451,8 +458,9 @@ int check_report(lmx_solver *s, const uint32_t *hdr)
             if (int rc = settle(s)) return rc;
             if (int rc = fetch_report(s)) return rc;
             hdr = s->h_report;
+        } else {
+            resident_ended(s);
         }
-        s->res_pending = false;
     }
     // Many boxes had to be halved since the last look (the lattice became
     // more crowded): smaller boxes from now on.
@@ -676,11 +684,12 @@ lmx::ResidentJob resident_job(const lmx_solver *s, uint32_t nsteps)
     return j;
 }
 
-// After a resident run of nsteps was enqueued.
+// After a resident run of nsteps was enqueued.  It packs the lattice, unless it
+// found more particles than it holds and left them as they were: `packed`
+// stays until the run is known to have ended (resident_ended).
 void resident_ran(lmx_solver *s, uint32_t nsteps)
 {
     s->timestep += nsteps;
-    s->packed = true;
     s->flags_fresh = s->zflags_fresh[0] = s->zflags_fresh[1] = false;
     s->res_pending = s->unchecked = true;
 }
@@ -717,8 +726,11 @@ int settle(lmx_solver *s)
     LMX_HIP(hipStreamSynchronize(s->stream));
     uint32_t t = 0;
     LMX_HIP(hipMemcpy(&t, &s->d_ctl->timestep, sizeof(t), hipMemcpyDeviceToHost));
+    if (t == s->timestep) {
+        resident_ended(s);
+        return LMX_OK;
+    }
     s->res_pending = false;
-    if (t == s->timestep) return LMX_OK;
     const uint32_t missing = s->timestep - t;
     s->timestep = t;
     s->resident_ok = false;

@@ -1,0 +1,94 @@
+"""Host side of the stepping calls (mpd_capi.cpp), compiled for the CPU against
+a stand-in for the HIP runtime and the kernels (tests/standin): what a call
+enqueues, what it waits for, and what it leaves behind when a resident run
+stops short or an allocation fails."""
+import ctypes
+import os
+import shutil
+import subprocess
+
+import numpy as np
+import pytest
+
+import lattice_microbes_amd as lmx
+from lattice_microbes_amd import _lib, build, models
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+pytestmark = pytest.mark.skipif(not (shutil.which(build.HIPCC) or os.path.exists(build.HIPCC)), reason="no hipcc")
+
+
+@pytest.fixture(scope="module")
+def standin_library(tmp_path_factory):
+    out = tmp_path_factory.mktemp("standin")
+    objs = []
+    for src in (os.path.join(build.CSRC, "mpd_capi.cpp"), os.path.join(HERE, "standin", "hip_standin.cpp")):
+        objs.append(str(out / (os.path.basename(src) + ".o")))
+        subprocess.run([build.HIPCC, "-O1", "-std=c++17", "--offload-host-only", "-fPIC", "-ffp-contract=off", "-w",
+                        "-I" + os.path.join(build.ROOT, "include"), "-I" + build.CSRC, "-c", "-x", "hip", src,
+                        "-o", objs[-1]], check=True)
+    so = str(out / "libstandin.so")
+    subprocess.run([build.CXX, "-shared", "-Wl,-z,defs", *objs, "-o", so], check=True)
+    lib = ctypes.CDLL(so)
+    for name, (res, args) in _lib.SIGNATURES.items():
+        fn = getattr(lib, name)
+        fn.restype, fn.argtypes = res, args
+    lib.standin_log.restype = ctypes.c_char_p
+    lib.standin_cost.argtypes = [ctypes.c_char_p, ctypes.c_double]
+    return lib
+
+
+@pytest.fixture
+def lib(standin_library, monkeypatch):
+    monkeypatch.setattr(_lib, "_lib", standin_library)
+    standin_library.standin_reset()
+    yield standin_library
+    standin_library.standin_reset()
+
+
+def log(lib):
+    """The log since the last look at it."""
+    lines = lib.standin_log().decode().split("\n")[:-1]
+    lib.standin_clear_log()
+    return lines
+
+
+def small(words=False, **kw):
+    """A solver whose calls of four steps and more are resident runs."""
+    spec = models.bimolecular(shape=(16, 16, 16), nA=50, nB=50, seed=1, **kw)
+    if words:
+        spec.lattice = spec.lattice.astype(np.uint32)
+    s = (lmx.IntMpdRdmeSolver if words else lmx.MpdRdmeSolver)(0)
+    spec.load_into(s, seed=3)
+    return spec, s
+
+
+@pytest.mark.parametrize("words", [False, True], ids=["byte", "uint32"])
+def test_a_run_that_did_nothing_does_not_pack_the_lattice(lib, words):
+    """A resident run that found too many particles leaves them where they
+    were, with empty slots before occupied ones: the first step made up for it
+    reads every plane."""
+    spec, s = small(words)
+    p, q = ctypes.c_void_p(), ctypes.c_void_p()
+    _lib.check(lib.lmx_device_lattice(s._h, ctypes.byref(p), ctypes.byref(q)))
+    lib.standin_resident_limit(0)
+    log(lib)
+    s.runTimesteps(5)
+    lines = log(lib)
+    assert [l for l in lines if l.startswith("resident")] == ["resident t=0 steps=5 packed=0"]
+    boxes = [l for l in lines if l.startswith("box")]
+    assert [l.split()[:3] for l in boxes] == [["box", f"t={t}", f"packed={int(t > 0)}"] for t in range(5)]
+    s.close()
+
+
+def test_a_run_that_ended_packs_the_lattice(lib):
+    spec, s = small()
+    p, q = ctypes.c_void_p(), ctypes.c_void_p()
+    _lib.check(lib.lmx_device_lattice(s._h, ctypes.byref(p), ctypes.byref(q)))
+    log(lib)
+    s.runTimesteps(5)
+    s.runTimesteps(1)
+    lines = log(lib)
+    assert "resident t=0 steps=5 packed=0" in lines
+    assert [l.split()[:3] for l in lines if l.startswith("box")] == [["box", "t=5", "packed=1"]]
+    s.close()
