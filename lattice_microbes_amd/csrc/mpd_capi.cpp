@@ -723,6 +723,7 @@ int enqueue_steps(lmx_solver *s, uint32_t nsteps, const lmx::ReactionList *rl = 
 int settle(lmx_solver *s)
 {
     if (!s->res_pending) return LMX_OK;
+    if (int rc = select_device(s)) return rc;
     LMX_HIP(hipStreamSynchronize(s->stream));
     uint32_t t = 0;
     LMX_HIP(hipMemcpy(&t, &s->d_ctl->timestep, sizeof(t), hipMemcpyDeviceToHost));

@@ -92,3 +92,21 @@ def test_a_run_that_ended_packs_the_lattice(lib):
     assert "resident t=0 steps=5 packed=0" in lines
     assert [l.split()[:3] for l in lines if l.startswith("box")] == [["box", "t=5", "packed=1"]]
     s.close()
+
+
+def test_missing_steps_run_on_the_solvers_device(lib):
+    """New parameters first make up for the steps that an earlier run left
+    out, on the solver's device, whichever is current."""
+    spec = models.bimolecular(shape=(16, 16, 16), nA=50, nB=50, seed=1)
+    s = lmx.MpdRdmeSolver(1)
+    spec.load_into(s, seed=3)
+    lib.standin_resident_limit(2)
+    s.runTimesteps(6, synchronize=False)
+    other = lmx.MpdRdmeSolver(0)
+    log(lib)
+    _lib.check(lib.lmx_initialize(s._h, 0, 9, 1e-6, _lib.OVERFLOW_CLASSIC, _lib.BOUNDARY_PERIODIC))
+    lines = log(lib)
+    assert lines[0] == "device 1"
+    assert [l.split()[1] for l in lines if l.startswith("box")] == ["t=2", "t=3", "t=4", "t=5"]
+    other.close()
+    s.close()
