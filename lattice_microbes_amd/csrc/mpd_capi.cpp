@@ -884,6 +884,7 @@ int lmx_build_model(lmx_solver *s, uint32_t nS, uint32_t R, const uint32_t *init
         if (R > 16384) return fail(LMX_ERR_ARG, "The number of reaction table entries exceeds the maximum supported by the solver (16384).");
         if ((R > 0 || nS > 0) && (!types || !K || !S || !D) && R > 0) return fail(LMX_ERR_ARG, "null model array");
         if (s->batch) return fail(LMX_ERR_STATE, "the solver is an ensemble member; remove it before rebuilding its model");
+        if (int rc = settle(s)) return rc;  // steps already asked for run with the model they were asked for
         // The fields below are overwritten before every check has passed, so
         // until this call succeeds the solver has no model and no lattice:
         // a failed rebuild leaves nothing that a step or a readback could use
@@ -970,6 +971,7 @@ int lmx_build_diffusion_model(lmx_solver *s, uint32_t nST, const double *DF, con
         if (s->batch) return fail(LMX_ERR_STATE, "the solver is an ensemble member; remove it before rebuilding its lattice");
         int rc = select_device(s);
         if (rc) return rc;
+        if ((rc = settle(s))) return rc;  // steps already asked for run on the lattice they were asked for
         LMX_HIP(hipStreamSynchronize(s->stream));
         // Shape, tables and buffers are replaced below before every check and
         // allocation has passed; the solver has no lattice until this call

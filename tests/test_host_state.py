@@ -110,3 +110,29 @@ def test_missing_steps_run_on_the_solvers_device(lib):
     assert [l.split()[1] for l in lines if l.startswith("box")] == ["t=2", "t=3", "t=4", "t=5"]
     other.close()
     s.close()
+
+
+@pytest.mark.parametrize("rebuilt", ["model", "lattice"])
+@pytest.mark.parametrize("then", ["synchronize", "overflow_stats", "unresolved", "initialize"])
+def test_a_rebuild_launches_no_old_step_with_new_shapes(lib, rebuilt, then):
+    """A resident run stopped short, nothing has looked at it yet, and the
+    model is replaced, or a new lattice refused: the missing steps run with
+    the old model and lattice, and none after that."""
+    spec, s = small()
+    lib.standin_resident_limit(2)
+    s.runTimesteps(6, synchronize=False)
+    log(lib)
+    if rebuilt == "model":
+        big = models.random_model(shape=(8, 8, 8), P=8, nS=40, nST=2, R=30, density=0.01, seed=2)
+        s.buildModel(big.nS, big.R, big.initial_counts(), big.types, big.K, big.S, big.D, 1)
+    else:
+        big = models.bimolecular(shape=(64, 64, 64), nA=50, nB=50, seed=1)
+        with pytest.raises(lmx.InvalidArgException, match="diffusion coefficient is too high"):
+            s.buildDiffusionModel(big.nST, big.DF * 1e6, big.RL, 64, 64, 64, big.P, 1, big.spacing, big.lattice,
+                                  big.sites, True)
+    want = [f"box t={t} packed=1 N={spec.N} R={spec.R}" for t in (2, 3, 4, 5)]
+    assert [l for l in log(lib) if l.startswith(("box", "sweep", "fused", "resident"))] == want
+    {"synchronize": s.synchronize, "overflow_stats": s.getOverflowStats, "unresolved": s.getUnresolvedOverflows,
+     "initialize": lambda: s.initialize(0, spec.parameters(3))}[then]()
+    assert not [l for l in log(lib) if l.startswith(("box", "sweep", "fused", "resident"))]
+    s.close()
