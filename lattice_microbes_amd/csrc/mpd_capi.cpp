@@ -738,18 +738,26 @@ int settle(lmx_solver *s)
     return enqueue_steps(s, missing);
 }
 
-// Buffers of the report and of the counts of up to `species` species.
+// Buffers of the report and of the counts of up to `species` species.  The
+// ones there stay unless all the new ones were allocated: reports need them.
 hipError_t alloc_counts(lmx_solver *s, uint32_t species)
 {
+    const size_t n = (size_t)species + 1;
+    uint32_t *counts = nullptr, *report = nullptr;
+    hipError_t e = hipMalloc((void **)&counts, n * sizeof(uint32_t));
+    if (e == hipSuccess)
+        e = hipHostMalloc((void **)&report, (lmx::kReportWords + n) * sizeof(uint32_t), hipHostMallocDefault);
+    if (e == hipSuccess) e = hipMemsetAsync(counts, 0, n * sizeof(uint32_t), s->stream);
+    if (e != hipSuccess) {
+        dev_free(counts);
+        if (report) hipHostFree(report);
+        return e;
+    }
     dev_free(s->d_counts);
     if (s->h_report) hipHostFree(s->h_report);
-    s->h_report = nullptr;
-    s->counts_cap = 0;
-    hipError_t e = hipMalloc((void **)&s->d_counts, ((size_t)species + 1) * sizeof(uint32_t));
-    if (e == hipSuccess)
-        e = hipHostMalloc((void **)&s->h_report, (lmx::kReportWords + (size_t)species) * sizeof(uint32_t), hipHostMallocDefault);
-    if (e == hipSuccess) e = hipMemsetAsync(s->d_counts, 0, ((size_t)species + 1) * sizeof(uint32_t), s->stream);
-    if (e == hipSuccess) s->counts_cap = species;
+    s->d_counts = counts;
+    s->h_report = report;
+    s->counts_cap = species;
     return e;
 }
 

@@ -6,6 +6,7 @@
 //   box | sweep | fused t=<step> packed=<0,1> N=<sites> R=<reactions>
 //   resident t=<step> steps=<asked> packed=<0,1>
 //   sync | copy | device      waits, blocking copies, hipSetDevice
+//   report                    the control blocks' report
 //
 // A resident run stops after `limit` steps, as one whose block is full.
 #include <hip/hip_runtime.h>
@@ -206,7 +207,8 @@ hipError_t launch_counts(const uint32_t *, size_t, uint32_t nS, bool, uint32_t *
 }
 hipError_t launch_report(const ReportList &c, uint32_t *out, hipStream_t)
 {
-    for (uint32_t k = 0; k < c.n; k++) memcpy(out + k * kReportWords, c.ctl[k], kReportWords * sizeof(uint32_t));
+    note(out ? "report" : "report to null");
+    for (uint32_t k = 0; out && k < c.n; k++) memcpy(out + k * kReportWords, c.ctl[k], kReportWords * sizeof(uint32_t));
     return hipSuccess;
 }
 hipError_t launch_exp(const double *, double *, size_t, hipStream_t) { return hipSuccess; }

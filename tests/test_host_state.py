@@ -136,3 +136,24 @@ def test_a_rebuild_launches_no_old_step_with_new_shapes(lib, rebuilt, then):
      "initialize": lambda: s.initialize(0, spec.parameters(3))}[then]()
     assert not [l for l in log(lib) if l.startswith(("box", "sweep", "fused", "resident"))]
     s.close()
+
+
+def test_reports_survive_a_failed_allocation(lib):
+    """A model of more species than the counts' buffers hold, and no memory for
+    larger ones: the lattice is refused, and the calls that report through
+    those buffers still work."""
+    spec, s = small()
+    big = models.random_model(shape=(8, 8, 8), P=8, nS=300, nST=1, R=0, density=0.0, seed=2)
+    s2 = lmx.IntMpdRdmeSolver(0)
+    s2.initialize(0, big.parameters(3))
+    s2.buildModel(big.nS, big.R, big.initial_counts(), big.types, big.K, big.S, big.D, 1)
+    lib.standin_pinned_fails(1)
+    with pytest.raises(lmx.LmxError) as e:
+        s2.buildDiffusionModel(big.nST, big.DF, big.RL, 8, 8, 8, big.P, 4, big.spacing, big.lattice.astype(np.uint32),
+                               big.sites, True)
+    assert e.value.code == _lib.ERR_NOMEM
+    log(lib)
+    s2.synchronize()
+    assert [l for l in log(lib) if l.startswith("report")] == ["report"]
+    s2.close()
+    s.close()
