@@ -182,17 +182,22 @@ int lmx_autotune(lmx_solver *s, uint32_t nsteps, double *best_ms, int *chosen);
 /* runTimestep (MpdRdmeSolver.cu:996-1193) nsteps times, enqueued on the
  * solver's stream without a host synchronization per step (the reference
  * synchronizes every step, :1091).  Device-side errors are sticky and are
- * reported by the next lmx_synchronize. */
+ * reported by the next lmx_synchronize.  Four or more steps of a solver of at
+ * most 3000 particles without zero-order reactions run in one block in a
+ * single launch; if the particles outgrow the block, the steps it left out run
+ * (with a wait for the ones before them) in the next call that looks at the
+ * state, uploads new rates or rebuilds the solver; calls that only enqueue
+ * steps never wait for that. */
 int lmx_run_steps(lmx_solver *s, uint32_t nsteps);
 /* No counterpart in the reference: lmx_run_steps for callers that cannot
  * allocate device memory (code under HIP graph capture, tight serving loops).
  * The same kernels and results, with the z sweep's reaction list in a static
  * device array of the library (1024 shards x 256 entries, 8 MiB per GPU,
  * held until the process ends) instead of the solver's own list; the call
- * allocates nothing.  Lattices of at most 2,097,152 sites (128^3); larger
- * ones are rejected (LMX_ERR_ARG), as is a call after a reaction-rate change
- * whose tables lmx_run_steps has not uploaded yet (LMX_ERR_STATE).  Every
- * call on one GPU shares the array: calls that overlap on one GPU (solvers
+ * allocates nothing and waits for nothing.  Lattices of at most 2,097,152
+ * sites (128^3); larger ones are rejected (LMX_ERR_ARG), as is a call after a
+ * reaction-rate change whose tables lmx_run_steps has not uploaded yet
+ * (LMX_ERR_STATE).  Every call on one GPU shares the array: calls that overlap on one GPU (solvers
  * stepping concurrently on different streams) race. */
 int lmx_run_steps_static(lmx_solver *s, uint32_t nsteps);
 int lmx_synchronize(lmx_solver *s);

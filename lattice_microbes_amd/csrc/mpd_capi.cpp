@@ -709,7 +709,10 @@ int enqueue_steps(lmx_solver *s, uint32_t nsteps, const lmx::ReactionList *rl = 
         }
         return LMX_OK;
     }
-    if (int rc = settle(s)) return rc;
+    // (Behind a resident run that stops short these steps run earlier than
+    // their numbers say, from the lattice where it stands: the device's counter
+    // drives them, and the runs change no buffer.  settle() adds the steps
+    // that are missing at the end.)
     const lmx::Params p = make_params(s);
     for (uint32_t i = 0; i < nsteps; i++)
         if (int rc = enqueue_step(s, p, nullptr, nullptr, nullptr, rl)) return rc;
@@ -1096,7 +1099,8 @@ int lmx_set_reaction_rate(lmx_solver *s, uint32_t rxid, float rate)
     return guarded([&]() -> int {
         if (!s) return fail(LMX_ERR_ARG, "null solver");
         if (!s->model_built || rxid >= s->R) return fail(LMX_ERR_ARG, "reaction index is out of bounds");
-        if (int rc = settle(s)) return rc;  // steps already asked for keep the old rate
+        // (Steps already asked for keep the old rate: the tables on the device
+        // are replaced by the next run, after settle().)
         s->k[rxid] = rate;
         if (s->diffusion_built) compute_propensities(s);
         return LMX_OK;
@@ -1147,6 +1151,7 @@ int lmx_run_steps(lmx_solver *s, uint32_t nsteps)
     int rc = require_built(s);
     if (rc) return rc;
     if (s->tables_dirty) {
+        if ((rc = settle(s))) return rc;
         LMX_HIP(hipStreamSynchronize(s->stream));
         if ((rc = upload_tables(s))) return rc;
     }

@@ -6,7 +6,7 @@
 //   box | sweep | fused t=<step> packed=<0,1> N=<sites> R=<reactions>
 //   resident t=<step> steps=<asked> packed=<0,1>
 //   sync | copy | device      waits, blocking copies, hipSetDevice
-//   report                    the control blocks' report
+//   report | tables           the control blocks' report, new probability tables
 //
 // A resident run stops after `limit` steps, as one whose block is full.
 #include <hip/hip_runtime.h>
@@ -140,7 +140,7 @@ uint32_t batch_list_shards(const TileGeom &, uint32_t) { return 8u; }
 bool batch_list_by_block(uint32_t) { return false; }
 uint32_t batch_list_blocks(uint32_t, uint32_t) { return 8u; }
 uint32_t resident_gather_blocks(uint32_t) { return 1u; }
-hipError_t launch_prob_tables(const Params &, float *, float *, hipStream_t) { return hipSuccess; }
+hipError_t launch_prob_tables(const Params &, float *, float *, hipStream_t) { note("tables"); return hipSuccess; }
 
 static uint4 g_static[16];
 hipError_t static_reaction_list(int, uint32_t, ReactionList *out)

@@ -1,10 +1,13 @@
 """What a resident run leaves to the calls after it, when it ended and when it
 stopped short, on the device: every lattice is compared with the oracle."""
+import ctypes
+import time
+
 import numpy as np
 import pytest
 
 import lattice_microbes_amd as lmx
-from lattice_microbes_amd import models
+from lattice_microbes_amd import _lib, models
 from lattice_microbes_amd.solver import DeviceHookLattice
 import oracle
 
@@ -49,4 +52,79 @@ def test_unpacked_lattice_past_the_block(gpu, words):
         assert orc.run(chunk) == 0
         got = s.getLatticeNative()
         assert np.array_equal(got, orc.native()), f"{(got != orc.native()).sum()} words differ"
+    s.close()
+
+
+def _splitting(n, rate):
+    """A -> A + A: the particles multiply."""
+    spec = models.bimolecular(shape=(24, 20, 18), nA=n, nB=0, seed=5, boundary="periodic")
+    spec.types, spec.K = np.array([1], np.uint32), np.array([rate])
+    spec.S, spec.D = np.array([[1], [0], [0]], np.int32), np.array([[1], [0], [0]], np.uint32)
+    spec.RL = np.ones((1, 1), np.uint32)
+    return spec
+
+
+def _static(s, n):
+    _lib.check(_lib.load().lmx_run_steps_static(s._h, ctypes.c_uint32(n)))
+
+
+def test_short_calls_behind_a_run_that_stopped_short(gpu):
+    """Calls of one and two steps, of either kind, enqueued behind runs whose
+    block was full (about 14% more particles a step), and a new rate."""
+    spec = _splitting(2900, 3000.0)
+    s = lmx.MpdRdmeSolver(0)
+    spec.load_into(s, seed=3)
+    orc = oracle.Oracle(spec, seed_top=3)
+    for n in (4, 1, 4, 2):
+        s.runTimesteps(n, synchronize=False)
+        _static(s, 1)
+    assert orc.run(15) == 0
+    assert int(orc.species_counts().sum()) > 4096
+    assert np.array_equal(s.getLatticeNative(), orc.native())
+    assert s.timestep == orc.timestep == 15
+    s.close()
+
+
+def test_steps_behind_a_resident_run_are_enqueued(gpu):
+    """A run of 40000 steps takes half a second; calls behind it return before
+    it has ended."""
+    spec = models.bimolecular(shape=(64, 64, 64), seed=5)
+    s = lmx.MpdRdmeSolver(0)
+    spec.load_into(s, seed=3)
+    s.runTimesteps(4)
+    _static(s, 1)
+    s.synchronize()
+    t0 = time.perf_counter()
+    s.runTimesteps(40000, synchronize=False)
+    s.runTimesteps(2, synchronize=False)
+    _static(s, 2)
+    s.setReactionRate(0, float(spec.K[0]))
+    enqueued = time.perf_counter() - t0
+    s.synchronize()
+    assert enqueued < 0.5 * (time.perf_counter() - t0)
+    s.close()
+
+
+def test_static_steps_while_a_graph_is_captured(gpu):
+    """No wait and no blocking copy, which a capture elsewhere in the process
+    would refuse."""
+    import torch
+    spec = models.bimolecular(shape=(32, 32, 32), seed=5)
+    s = lmx.MpdRdmeSolver(0)
+    spec.load_into(s, seed=3)
+    orc = oracle.Oracle(spec, seed_top=3)
+    _static(s, 1)
+    s.synchronize()
+    s.runTimesteps(6, synchronize=False)
+    x = torch.zeros(8, device="cuda")
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        y = x + 1
+        _static(s, 2)
+        _static(s, 5)
+    g.replay()
+    torch.cuda.synchronize()
+    assert float(y.sum()) == 8.0
+    assert orc.run(14) == 0
+    assert np.array_equal(s.getLatticeNative(), orc.native())
     s.close()

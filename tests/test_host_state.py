@@ -157,3 +157,52 @@ def test_reports_survive_a_failed_allocation(lib):
     assert [l for l in log(lib) if l.startswith("report")] == ["report"]
     s2.close()
     s.close()
+
+
+def test_calls_behind_a_resident_run_do_not_wait(lib):
+    """Steps of any number, from either list, and a new rate are accepted
+    behind a resident run without a wait or a blocking copy."""
+    spec, s = small()
+    s.runTimesteps(8)
+    s.runTimesteps(8, synchronize=False)
+    log(lib)
+    s.runTimesteps(2, synchronize=False)
+    _lib.check(lib.lmx_run_steps_static(s._h, 3))
+    _lib.check(lib.lmx_run_steps_static(s._h, 8))
+    s.setReactionRate(0, 0.5)
+    lines = log(lib)
+    assert not {"sync", "copy"} & set(lines), lines
+    s.synchronize()
+    assert s.timestep == 29
+    s.close()
+
+
+def test_steps_behind_a_run_that_stopped_short(lib):
+    """They run from where the device stands, a later resident run does
+    nothing, and the missing steps follow when the state is looked at."""
+    spec, s = small()
+    lib.standin_resident_limit(2)
+    log(lib)
+    s.runTimesteps(6, synchronize=False)
+    s.runTimesteps(1, synchronize=False)
+    s.runTimesteps(5, synchronize=False)
+    _lib.check(lib.lmx_run_steps_static(s._h, 1))
+    assert [l.split()[:2] for l in log(lib) if l.startswith(("box", "resident"))] == [
+        ["resident", "t=0"], ["box", "t=2"], ["resident", "t=7"], ["box", "t=3"]]
+    s.synchronize()
+    assert [l.split()[1] for l in log(lib) if l.startswith("box")] == [f"t={t}" for t in range(4, 13)]
+    assert s.timestep == 13
+    s.close()
+
+
+def test_missing_steps_keep_the_old_rate(lib):
+    """New tables are uploaded after the steps that an earlier run left out."""
+    spec, s = small()
+    lib.standin_resident_limit(2)
+    s.runTimesteps(6, synchronize=False)
+    s.setReactionRate(0, 0.5)
+    log(lib)
+    s.runTimesteps(2)
+    lines = [l.split()[:2] for l in log(lib) if l.startswith(("box", "tables"))]
+    assert lines == [["box", f"t={t}"] for t in range(2, 6)] + [["tables"]] + [["box", "t=6"], ["box", "t=7"]]
+    s.close()
