@@ -197,8 +197,9 @@ int lmx_run_steps(lmx_solver *s, uint32_t nsteps);
  * allocates nothing and waits for nothing.  Lattices of at most 2,097,152
  * sites (128^3); larger ones are rejected (LMX_ERR_ARG), as is a call after a
  * reaction-rate change whose tables lmx_run_steps has not uploaded yet
- * (LMX_ERR_STATE).  Every call on one GPU shares the array: calls that overlap on one GPU (solvers
- * stepping concurrently on different streams) race. */
+ * (LMX_ERR_STATE).  Every call on one GPU shares the array: calls that overlap
+ * on one GPU (solvers stepping concurrently on different streams) race.  The
+ * uint32 lattice's calls do not use it. */
 int lmx_run_steps_static(lmx_solver *s, uint32_t nsteps);
 int lmx_synchronize(lmx_solver *s);
 /* Current timestep counter (number of steps taken since the lattice was set). */

@@ -1169,11 +1169,12 @@ int lmx_run_steps_static(lmx_solver *s, uint32_t nsteps)
     if (s->tables_dirty)
         return fail(LMX_ERR_STATE, "lmx_run_steps_static: reaction rates changed since the tables were uploaded; "
                                    "lmx_run_steps uploads them (it allocates)");
+    // (The uint32 lattice's steps keep their candidates in the solver's own
+    // list, so that calls of different solvers may overlap.)
+    if (s->bpp == 4) return enqueue_steps(s, nsteps);
     lmx::ReactionList rl{};
-    {
-        const hipError_t e = lmx::static_reaction_list(s->device, s->bpp == 1 ? s->W : 1, &rl);
-        if (e != hipSuccess) return hip_fail(e, "static reaction list");
-    }
+    const hipError_t e = lmx::static_reaction_list(s->device, s->W, &rl);
+    if (e != hipSuccess) return hip_fail(e, "static reaction list");
     return enqueue_steps(s, nsteps, &rl);
 }
 

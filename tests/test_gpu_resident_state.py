@@ -128,3 +128,21 @@ def test_static_steps_while_a_graph_is_captured(gpu):
     assert orc.run(14) == 0
     assert np.array_equal(s.getLatticeNative(), orc.native())
     s.close()
+
+
+def test_static_steps_of_the_uint32_lattice(gpu):
+    """Two solvers' calls in turn, without a wait between them."""
+    pairs = []
+    for k, shape in enumerate([(40, 36, 28), (33, 30, 31)]):
+        spec = models.random_model(shape=shape, P=8, nS=5, nST=2, R=6, density=0.03, seed=30 + k, include_zero_order=True)
+        spec.lattice = spec.lattice.astype(np.uint32)
+        s = lmx.IntMpdRdmeSolver(0)
+        spec.load_into(s, replicate=k, seed=3)
+        pairs.append((s, oracle.Oracle(spec, seed_top=3, replicate=k)))
+    for turn in range(6):
+        for s, _ in pairs:
+            _static(s, 2)
+    for s, orc in pairs:
+        assert orc.run(12) == 0
+        assert np.array_equal(s.getLatticeNative(), orc.native())
+        s.close()

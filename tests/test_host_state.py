@@ -206,3 +206,14 @@ def test_missing_steps_keep_the_old_rate(lib):
     lines = [l.split()[:2] for l in log(lib) if l.startswith(("box", "tables"))]
     assert lines == [["box", f"t={t}"] for t in range(2, 6)] + [["tables"]] + [["box", "t=6"], ["box", "t=7"]]
     s.close()
+
+
+@pytest.mark.parametrize("words", [False, True], ids=["byte", "uint32"])
+def test_static_list_is_the_byte_lattices(lib, words):
+    """Solvers of the uint32 lattice share no list, so their calls may overlap."""
+    spec, s = small(words)
+    log(lib)
+    _lib.check(lib.lmx_run_steps_static(s._h, 1))
+    lines = log(lib)
+    assert any(l.startswith("box") for l in lines) and ("static list" in lines) == (not words)
+    s.close()
