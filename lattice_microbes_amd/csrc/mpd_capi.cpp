@@ -291,12 +291,17 @@ int require_ready(lmx_solver *s)
     return rc ? rc : settle(s);
 }
 
+// Particles of a lattice that are listed for plan_boxes: one more than the
+// most that its rules look at (a particle a site for boxes, kResidentMost for
+// resident runs).
+size_t listed_most(const lmx_solver *s) { return std::max<size_t>(s->N, lmx::kResidentMost) + 1; }
+
 // Row-major (x,y,z,p) -> native planes, inserting each nonzero particle at
 // the first empty slot of its site (RDMESolver::setLatticeData + addParticle;
 // IntLattice::setFromRowMajorData for the uint32 lattice).  rm holds N*P
 // elements of bpp bytes.
-// at, if given, receives the native site index of every particle, as long as
-// there are at most N (see plan_boxes).
+// at, if given, receives the native site index of every particle, up to
+// listed_most of them.
 int row_major_to_native(const lmx_solver *s, const void *rm, std::vector<uint32_t> &native,
                         std::vector<uint32_t> *at = nullptr)
 {
@@ -305,6 +310,7 @@ int row_major_to_native(const lmx_solver *s, const void *rm, std::vector<uint32_
     const uint8_t *rb = static_cast<const uint8_t *>(rm);
     const uint32_t *rw = static_cast<const uint32_t *>(rm);
     native.assign(N * s->W, 0u);
+    const size_t most = listed_most(s);
     size_t idx = 0;
     for (uint32_t x = 0; x < s->X; x++)
         for (uint32_t y = 0; y < s->Y; y++)
@@ -323,7 +329,7 @@ int row_major_to_native(const lmx_solver *s, const void *rm, std::vector<uint32_
                     const uint32_t v = words ? rw[idx + l] : rb[idx + l];
                     if (v == 0) continue;
                     if (v > s->nS) return fail(LMX_ERR_ARG, "latticeData: an invalid species was found: " + std::to_string(v));
-                    if (at && at->size() <= N) at->push_back((uint32_t)i);
+                    if (at && at->size() < most) at->push_back((uint32_t)i);
                     if (words)
                         native[(size_t)j * N + i] = v;
                     else
@@ -1263,6 +1269,7 @@ int lmx_set_lattice_native(lmx_solver *s, const uint32_t *native, size_t words)
         // its first slots.
         bool packed = true;
         std::vector<uint32_t> at;
+        const size_t most = listed_most(s);
         for (size_t i = 0; i < s->N; i++) {
             bool gap = false;
             for (uint32_t j = 0; j < s->P; j++) {
@@ -1277,7 +1284,7 @@ int lmx_set_lattice_native(lmx_solver *s, const uint32_t *native, size_t words)
                     gap = true;
                 } else {
                     if (gap) packed = false;
-                    if (at.size() <= s->N) at.push_back((uint32_t)i);
+                    if (at.size() < most) at.push_back((uint32_t)i);
                 }
             }
         }

@@ -217,3 +217,31 @@ def test_static_list_is_the_byte_lattices(lib, words):
     lines = log(lib)
     assert any(l.startswith("box") for l in lines) and ("static list" in lines) == (not words)
     s.close()
+
+
+@pytest.mark.parametrize("n,resident", [(3000, True), (3001, False), (4000, False)])
+@pytest.mark.parametrize("by", ["build", "set", "set_native"])
+def test_crowded_small_lattices_are_counted(lib, n, resident, by):
+    """More particles than sites: a lattice of 500 sites is run in one block
+    only if its particles are few, however the lattice was set."""
+    rng = np.random.default_rng(1)
+    spec = models.random_model(shape=(10, 10, 5), P=16, nS=3, nST=1, R=0, density=0.0, seed=1)
+    lattice = np.zeros(500 * 16, np.uint8)
+    lattice[rng.permutation(lattice.size)[:n]] = 1
+    lattice = lattice.reshape(10, 10, 5, 16)
+    s = lmx.MpdRdmeSolver(0)
+    if by == "build":
+        spec.lattice = lattice
+    spec.load_into(s, seed=1)
+    if by == "set":
+        s.setLattice(lattice)
+    elif by == "set_native":
+        packed = np.zeros((4, 5, 10, 10), np.uint32)
+        for (x, y, z), c in np.ndenumerate((lattice != 0).sum(axis=3)):
+            for j in range(c):
+                packed[j // 4, z, y, x] |= np.uint32(1 << (8 * (j % 4)))
+        s.setLatticeNative(packed)
+    log(lib)
+    s.runTimesteps(4)
+    assert any(l.startswith("resident") for l in log(lib)) == resident
+    s.close()
