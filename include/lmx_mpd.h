@@ -163,10 +163,11 @@ int lmx_set_launch_option(lmx_solver *s, int option, int value);
 
 /* Launch-shape autotuner (no reference counterpart: the reference fixes its
  * block shapes at build time, options.cmake TUNE_MPD_*).  From the current
- * state it times nsteps steps (after one untimed step) of each y/z sweep
- * kernel and window shape: LDS row tiles with and without the reaction list,
- * register march and register columns of 4 and 8 rows, compacted tiles, and
- * the fused step.  It restores the state after each, times two interleaved
+ * state it times nsteps steps (after one untimed step) of the default step
+ * (boxes, or one block for the whole call where lmx_run_steps takes one; then
+ * at least four steps) and of each y/z sweep kernel and window shape: LDS row
+ * tiles with and without the reaction list, register march and register
+ * columns of 4 and 8 rows, compacted tiles, and the fused step.  It restores the state after each, times two interleaved
  * passes and keeps the fastest by the minimum of each, but keeps the current
  * configuration unless another is at least 2% faster.  With
  * LMX_OPT_FORCE_GENERIC set only the current configuration is timed and every

@@ -146,3 +146,20 @@ def test_static_steps_of_the_uint32_lattice(gpu):
         assert orc.run(12) == 0
         assert np.array_equal(s.getLatticeNative(), orc.native())
         s.close()
+
+
+def test_autotune_of_a_resident_solver_keeps_the_state(gpu):
+    """The tuner times the one-block run too (and one that outgrows its block);
+    afterwards the state is as before."""
+    for spec in (models.bimolecular(shape=(32, 32, 32), seed=5), _splitting(2900, 3000.0)):
+        s = lmx.MpdRdmeSolver(0)
+        spec.load_into(s, seed=3)
+        orc = oracle.Oracle(spec, seed_top=3)
+        s.runTimesteps(2)
+        assert orc.run(2) == 0
+        assert s.autotune(steps=8)["ms_per_step"] > 0
+        assert np.array_equal(s.getLatticeNative(), orc.native()) and s.timestep == 2
+        s.runTimesteps(9)
+        assert orc.run(9) == 0
+        assert np.array_equal(s.getLatticeNative(), orc.native()) and s.timestep == 11
+        s.close()

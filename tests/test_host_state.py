@@ -35,6 +35,7 @@ def standin_library(tmp_path_factory):
         fn.restype, fn.argtypes = res, args
     lib.standin_log.restype = ctypes.c_char_p
     lib.standin_cost.argtypes = [ctypes.c_char_p, ctypes.c_double]
+    lib.standin_resident_limit.argtypes = [ctypes.c_uint32]
     return lib
 
 
@@ -244,4 +245,29 @@ def test_crowded_small_lattices_are_counted(lib, n, resident, by):
     log(lib)
     s.runTimesteps(4)
     assert any(l.startswith("resident") for l in log(lib)) == resident
+    s.close()
+
+
+@pytest.mark.parametrize("cost,limit,steps,resident,best", [
+    (dict(resident=1, box=16, sweep=10, fused=5), None, 8, True, 1.0),
+    (dict(resident=1, box=16, sweep=10, fused=5), None, 2, True, 1.0),   # shorter than any resident run
+    (dict(resident=7, box=16, sweep=10, fused=5), None, 8, False, 5.0),
+    (dict(resident=1, box=16, sweep=10, fused=15), 3, 8, False, 10.0),    # a block that is full takes no time
+])
+def test_autotune_times_the_resident_run(lib, cost, limit, steps, resident, best):
+    """The run that calls of four steps and more would be is what the other
+    shapes have to beat."""
+    spec, s = small()
+    for kind, ms in cost.items():
+        lib.standin_cost(kind.encode(), float(ms))
+    if limit is not None:
+        lib.standin_resident_limit(limit)
+    assert s.autotune(steps=steps)["ms_per_step"] == pytest.approx(best)
+    lib.standin_resident_limit(0xFFFFFFFF)
+    log(lib)
+    assert s.timestep == 0
+    s.runTimesteps(5)
+    lines = log(lib)
+    assert any(l.startswith("resident") for l in lines) == resident
+    assert s.timestep == 5
     s.close()
