@@ -277,9 +277,11 @@ int lmx_device_reaction_probability(int device, const float *a, float *prob, siz
 /* ---- Ensembles -----------------------------------------------------------
  * No reference counterpart: the reference runs every replicate in its own
  * thread or process (src/core/ReplicateRunner.cpp, src/lm/main/Main.cpp).
- * A batch steps many independently configured solvers on one device with one
- * launch per kernel class per step (replayed from a captured HIP graph by
- * default); members may differ in lattice size, model, seed and step count.
+ * A batch steps many independently configured solvers on one device: the
+ * members of few particles in a block of their own each for a whole call, the
+ * others that lmx_run_steps would step in boxes in two launches a step, and
+ * the rest in the batched sweeps, one launch per kernel class per step
+ * (replayed from a captured HIP graph by default); members may differ in lattice size, model, seed and step count.
  * Every member's lattice is bit-identical to running that solver alone.
  * Members need X % 4 == 0 and the same particles per site.  A solver belongs
  * to at most one batch and leaves it when destroyed; its own calls stay
@@ -293,12 +295,13 @@ int lmx_batch_size(const lmx_batch *b, uint32_t *n);
 /* LMX_BATCH_GRAPH: 1 (default) = replay a captured graph of one step.
  * LMX_BATCH_REACTION_LIST: 1 (default) = a member without zero-order
  * reactions runs its reaction phase over the occupied sites its z sweep lists
- * (as a single solver does); 0 = the full in-place pass for every member.
+ * (as a single solver does); 0 = the full in-place pass for every member,
+ * all of which then step in the batched sweeps.
  * LMX_BATCH_TILE_THREADS: threads per block of the tiled y/z sweeps, which
  * sets every member's tile shape: 0 (default) = 256 (tiles 32 sites wide and
- * 32 rows tall), else a multiple of 64 from 256 up to 1024 (512 with 16
- * slots per site); above 256, tiles 256 sites wide.  Results are identical
- * whatever the options. */
+ * 32 rows tall), else a multiple of 64 up to 1024 (512 with 16 slots per
+ * site): tiles 256 sites wide, and every member steps in the batched sweeps.
+ * Results are identical whatever the options. */
 enum lmx_batch_option { LMX_BATCH_GRAPH = 1, LMX_BATCH_REACTION_LIST = 2, LMX_BATCH_TILE_THREADS = 3 };
 int lmx_batch_set_option(lmx_batch *b, int option, int value);
 /* No reference counterpart (the reference's launch shapes are build-time

@@ -2166,8 +2166,8 @@ int lmx_batch_set_option(lmx_batch *b, int option, int value)
         return LMX_OK;
     }
     if (option == LMX_BATCH_TILE_THREADS) {
-        const uint32_t t = (uint32_t)value;
-        if (value != 0 && (value < 0 || t % 64u || t < 256u || (b->W && t > lmx::tile_threads_for(b->W)) || t > 1024u))
+        const uint32_t t = value == (int)lmx::kNarrowTileThreads ? 0u : (uint32_t)value;  // (the default's size)
+        if (t != 0u && (value < 0 || t % 64u || t < 256u || (b->W && t > lmx::tile_threads_for(b->W)) || t > 1024u))
             return fail(LMX_ERR_ARG, "tile threads: 0 (default, 256) or a multiple of 64 from 256 up to 1024 (512 for P = 16)");
         if (b->tile_threads != t) batch_drop_graph(b);
         b->tile_threads = t;

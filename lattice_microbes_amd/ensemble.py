@@ -2,9 +2,11 @@
 
 No reference counterpart: the reference runs each replicate in its own
 thread or process (src/core/ReplicateRunner.cpp).  Here many independently
-configured solvers (any lattice size, model, seed) advance with one kernel
-launch per kernel class per step, replayed from a captured HIP graph; each
-member's lattice stays bit-identical to running that solver alone.
+configured solvers (any lattice size, model, seed) advance together: members
+of few particles in a block of their own for a whole call, the others in two
+launches a step over boxes of their lattices or, where these are too crowded,
+in one launch per kernel class per step, replayed from a captured HIP graph;
+each member's lattice stays bit-identical to running that solver alone.
 """
 from __future__ import annotations
 
@@ -42,12 +44,14 @@ class Ensemble:
 
     def set_reaction_list(self, on: bool) -> None:
         """Reaction phases over the occupied sites each member's z sweep lists
-        (default), or the full in-place pass; the results are identical."""
+        (default), or the full in-place pass (every member then steps in the
+        batched sweeps); the results are identical."""
         _lib.check(self._lib.lmx_batch_set_option(self._h, _lib.BATCH_REACTION_LIST, 1 if on else 0))
 
     def set_tile_threads(self, threads: int) -> None:
-        """Threads per block of the tiled y/z sweeps (0: the default); the
-        results are identical."""
+        """Threads per block of the tiled y/z sweeps (0 or 256: the default;
+        with others every member steps in the batched sweeps); the results
+        are identical."""
         _lib.check(self._lib.lmx_batch_set_option(self._h, _lib.BATCH_TILE_THREADS, int(threads)))
 
     def autotune(self, steps: int = 8) -> dict:

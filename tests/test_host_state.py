@@ -271,3 +271,22 @@ def test_autotune_times_the_resident_run(lib, cost, limit, steps, resident, best
     assert any(l.startswith("resident") for l in lines) == resident
     assert s.timestep == 5
     s.close()
+
+
+@pytest.mark.parametrize("threads,sweeps", [(0, False), (256, False), (512, True)])
+def test_default_tile_threads_by_their_number(lib, threads, sweeps):
+    """256 threads are the default and leave the members' routes alone, also
+    after another size was set."""
+    ens = lmx.Ensemble(0, graph=False)
+    few, many = small()[1], lmx.MpdRdmeSolver(0)
+    models.bimolecular(shape=(64, 64, 64), nA=5000, nB=50, seed=1).load_into(many, seed=2)
+    for s in (few, many):
+        ens.add(s)
+    ens.set_tile_threads(1024)
+    ens.set_tile_threads(threads)
+    log(lib)
+    ens.run(5)
+    kinds = {l.split()[0] for l in log(lib)} & {"resident", "box", "sweep"}
+    assert kinds == ({"sweep"} if sweeps else {"resident", "box"})
+    assert few.timestep == many.timestep == 5
+    ens.close()
