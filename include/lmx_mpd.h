@@ -305,14 +305,15 @@ int lmx_batch_size(const lmx_batch *b, uint32_t *n);
 enum lmx_batch_option { LMX_BATCH_GRAPH = 1, LMX_BATCH_REACTION_LIST = 2, LMX_BATCH_TILE_THREADS = 3 };
 int lmx_batch_set_option(lmx_batch *b, int option, int value);
 /* No reference counterpart (the reference's launch shapes are build-time
- * TUNE_MPD_* constants): times nsteps batched steps (after one untimed step)
- * for each launch configuration -- reaction list on and off, tile blocks of
- * 256, half the maximum and the maximum threads -- in two interleaved passes,
- * restoring every member's lattice buffers, control block and step counter
- * before each and at the end, and keeps the fastest (the current one unless
- * another is at least 2% faster).  chosen[0] = reaction list (0/1),
- * chosen[1] = tile threads.  Allocates a copy of every member's buffers for
- * the duration of the call. */
+ * TUNE_MPD_* constants): times nsteps batched steps (at least four where
+ * members run in one block, after one untimed step) for each launch
+ * configuration -- reaction list on and off, tile blocks of 256, half the
+ * maximum and the maximum threads -- in two interleaved passes, restoring
+ * every member's lattice buffers, control block and step counter before each
+ * and at the end, and keeps the fastest (the current one unless another is at
+ * least 2% faster).  chosen[0] = reaction list (0/1), chosen[1] = tile
+ * threads.  Allocates a copy of every member's buffers for the duration of
+ * the call. */
 int lmx_batch_autotune(lmx_batch *b, uint32_t nsteps, double *best_ms, int *chosen);
 /* Advances every member by nsteps (asynchronous; errors are reported by
  * lmx_batch_synchronize, or by a member's own calls). */

@@ -2263,13 +2263,13 @@ int lmx_batch_autotune(lmx_batch *b, uint32_t nsteps, double *best_ms, int *chos
             size_t off, buf_bytes;
             uint32_t timestep;
             int cur;
-            bool packed, fresh;
+            bool packed, fresh, resident;
         };
         std::vector<Saved> saved;
         size_t total = 0;
         for (lmx_solver *s : b->members) {
             const size_t bb = (s->N * s->W + s->flag_words) * sizeof(uint32_t);
-            saved.push_back({total, bb, s->timestep, s->cur, s->packed, s->flags_fresh});
+            saved.push_back({total, bb, s->timestep, s->cur, s->packed, s->flags_fresh, s->resident_ok});
             total += 2 * bb + sizeof(lmx::Control);
             total = (total + 255) & ~(size_t)255;
         }
@@ -2297,12 +2297,19 @@ int lmx_batch_autotune(lmx_batch *b, uint32_t nsteps, double *best_ms, int *chos
                     s->cur = v.cur;
                     s->packed = v.packed;
                     s->flags_fresh = v.fresh;
+                    s->resident_ok = v.resident;
                     s->zflags_fresh[0] = s->zflags_fresh[1] = s->res_pending = false;
                 }
             }
             return LMX_OK;
         };
         if ((rc = copy_state(true))) return rc;
+
+        // Members that run in one block do so in calls of at least
+        // kResidentMinSteps.
+        uint32_t timed = nsteps;
+        for (const lmx_solver *s : b->members)
+            if (use_resident(s, kResidentMinSteps)) timed = std::max(nsteps, kResidentMinSteps);
 
         struct Config {
             bool list;
@@ -2333,12 +2340,12 @@ int lmx_batch_autotune(lmx_batch *b, uint32_t nsteps, double *best_ms, int *chos
                 if ((rc = copy_state(false))) break;
                 if ((rc = lmx_batch_run_steps(b, 1))) break;  // untimed first step (captures the graph)
                 LMX_HIP(hipEventRecord(e0, b->stream));
-                if ((rc = lmx_batch_run_steps(b, nsteps))) break;
+                if ((rc = lmx_batch_run_steps(b, timed))) break;
                 LMX_HIP(hipEventRecord(e1, b->stream));
                 LMX_HIP(hipEventSynchronize(e1));
                 float ms = 0.0f;
                 LMX_HIP(hipEventElapsedTime(&ms, e0, e1));
-                const double per = (double)ms / nsteps;
+                const double per = (double)ms / timed;
                 if (times[k] < 0.0 || per < times[k]) times[k] = per;
             }
         }

@@ -290,3 +290,18 @@ def test_default_tile_threads_by_their_number(lib, threads, sweeps):
     assert kinds == ({"sweep"} if sweeps else {"resident", "box"})
     assert few.timestep == many.timestep == 5
     ens.close()
+
+
+@pytest.mark.parametrize("steps", [2, 8])
+def test_batch_autotune_times_the_resident_runs(lib, steps):
+    """Also when asked for fewer steps than a run in one block takes."""
+    ens = lmx.Ensemble(0, graph=False)
+    spec, s = small()
+    ens.add(s)
+    for kind, ms in dict(resident=1, box=16, sweep=10).items():
+        lib.standin_cost(kind.encode(), float(ms))
+    assert ens.autotune(steps=steps) == {"reaction_list": True, "tile_threads": 256, "ms_per_step": 1.0}
+    log(lib)
+    ens.run(5)
+    assert {l.split()[0] for l in log(lib)} & {"resident", "box", "sweep"} == {"resident"}
+    ens.close()
