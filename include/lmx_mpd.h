@@ -160,6 +160,9 @@ enum lmx_option {
     LMX_OPT_FUSE_REACTION = 5, LMX_OPT_BOXES = 6
 };
 int lmx_set_launch_option(lmx_solver *s, int option, int value);
+/* The option's current value, for instance whether lmx_autotune kept
+ * LMX_OPT_BOXES. */
+int lmx_get_launch_option(lmx_solver *s, int option, int *value);
 
 /* Launch-shape autotuner (no reference counterpart: the reference fixes its
  * block shapes at build time, options.cmake TUNE_MPD_*).  From the current
@@ -175,7 +178,8 @@ int lmx_set_launch_option(lmx_solver *s, int option, int value);
  * results, so afterwards the lattice, step counter, overflow statistics and
  * carried entries are as before the call.  best_ms (optional) receives the
  * best time per step; chosen (optional, 4 ints) the path, LMX_OPT_YZ_KERNEL,
- * LMX_OPT_MARCH_SEGMENT and LMX_OPT_FUSE_REACTION kept.  Allocates a copy of
+ * LMX_OPT_MARCH_SEGMENT and LMX_OPT_FUSE_REACTION kept (LMX_OPT_BOXES, which
+ * tells the boxed step from the row tiles, by lmx_get_launch_option).  Allocates a copy of
  * both lattice buffers for the duration of the call; not for ensemble
  * members (LMX_ERR_STATE). */
 int lmx_autotune(lmx_solver *s, uint32_t nsteps, double *best_ms, int *chosen);

@@ -67,6 +67,7 @@ SIGNATURES = {
     "lmx_set_reaction_rate": (c_int, [c_void_p, c_uint32, c_float]),
     "lmx_set_path": (c_int, [c_void_p, c_int]),
     "lmx_set_launch_option": (c_int, [c_void_p, c_int, c_int]),
+    "lmx_get_launch_option": (c_int, [c_void_p, c_int, POINTER(c_int)]),
     "lmx_run_steps": (c_int, [c_void_p, c_uint32]),
     "lmx_run_steps_static": (c_int, [c_void_p, c_uint32]),
     "lmx_synchronize": (c_int, [c_void_p]),

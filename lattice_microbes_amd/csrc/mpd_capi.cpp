@@ -1152,6 +1152,20 @@ int lmx_set_launch_option(lmx_solver *s, int option, int value)
     return fail(LMX_ERR_ARG, "unknown launch option");
 }
 
+int lmx_get_launch_option(lmx_solver *s, int option, int *value)
+{
+    if (!s || !value) return fail(LMX_ERR_ARG, "null argument");
+    switch (option) {
+    case LMX_OPT_MARCH_SEGMENT: *value = (int)s->march_seg; return LMX_OK;
+    case LMX_OPT_FORCE_GENERIC: *value = s->force_generic ? 1 : 0; return LMX_OK;
+    case LMX_OPT_YZ_KERNEL: *value = s->yz_kernel; return LMX_OK;
+    case LMX_OPT_BOXES: *value = s->boxes ? 1 : 0; return LMX_OK;
+    case LMX_OPT_FUSE_REACTION: *value = s->fuse_reaction ? 1 : 0; return LMX_OK;
+    case LMX_OPT_FUSED_ZSEG: *value = (int)s->fused_zseg; return LMX_OK;
+    }
+    return fail(LMX_ERR_ARG, "unknown launch option");
+}
+
 int lmx_run_steps(lmx_solver *s, uint32_t nsteps)
 {
     int rc = require_built(s);

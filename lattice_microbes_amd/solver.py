@@ -210,6 +210,11 @@ class MpdRdmeSolver:
         """Launch-shape options (lmx_option); results do not depend on them."""
         _lib.check(self._lib.lmx_set_launch_option(self._h, int(option), int(value)))
 
+    def getLaunchOption(self, option: int) -> int:
+        v = ctypes.c_int()
+        _lib.check(self._lib.lmx_get_launch_option(self._h, int(option), byref(v)))
+        return v.value
+
     def autotune(self, steps: int = 8) -> Dict[str, object]:
         """Times every y/z sweep kernel and window shape for ``steps`` steps
         from the current state and keeps the fastest (lmx_autotune); the state
@@ -218,7 +223,8 @@ class MpdRdmeSolver:
         chosen = (ctypes.c_int * 4)()
         _lib.check(self._lib.lmx_autotune(self._h, int(steps), byref(best), chosen))
         return {"path": int(chosen[0]), "yz_kernel": int(chosen[1]), "march_segment": int(chosen[2]),
-                "fuse_reaction": bool(chosen[3]), "ms_per_step": best.value}
+                "fuse_reaction": bool(chosen[3]), "boxes": bool(self.getLaunchOption(_lib.OPT_BOXES)),
+                "ms_per_step": best.value}
 
     # ------------------------------------------------------------------ stepping
     def runTimesteps(self, nsteps: int, synchronize: bool = True) -> None:

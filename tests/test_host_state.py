@@ -305,3 +305,22 @@ def test_batch_autotune_times_the_resident_runs(lib, steps):
     ens.run(5)
     assert {l.split()[0] for l in log(lib)} & {"resident", "box", "sweep"} == {"resident"}
     ens.close()
+
+
+@pytest.mark.parametrize("box,boxes", [(5, True), (20, False)])
+def test_autotune_tells_boxes_from_tiles(lib, box, boxes):
+    """The other options read the same for the boxed step and the row tiles."""
+    s = lmx.MpdRdmeSolver(0)
+    models.bimolecular(shape=(64, 64, 64), nA=5000, nB=50, seed=1).load_into(s, seed=2)
+    for kind, ms in dict(box=box, sweep=10, fused=15).items():
+        lib.standin_cost(kind.encode(), float(ms))
+    tuned = s.autotune()
+    assert (tuned["path"], tuned["yz_kernel"], tuned["fuse_reaction"]) == (_lib.PATH_SWEEPS, 0, True)
+    assert tuned["boxes"] == boxes
+    for option, value in ((_lib.OPT_MARCH_SEGMENT, 4), (_lib.OPT_FORCE_GENERIC, 1), (_lib.OPT_YZ_KERNEL, 3),
+                          (_lib.OPT_FUSED_ZSEG, 7), (_lib.OPT_FUSE_REACTION, 0), (_lib.OPT_BOXES, 1)):
+        s.setLaunchOption(option, value)
+        assert s.getLaunchOption(option) == value
+    with pytest.raises(lmx.InvalidArgException):
+        s.getLaunchOption(99)
+    s.close()
