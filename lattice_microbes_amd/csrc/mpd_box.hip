@@ -45,6 +45,7 @@
 #include "lmx_kernels.h"
 #include "lmx_resolve.h"
 #include "lmx_site.h"
+#include "lmx_wave.h"
 
 namespace lmx {
 
@@ -636,11 +637,6 @@ __global__ __launch_bounds__(kBoxThreads, OCC) void box_jobs_kernel(const BoxJob
 // us, 256x256x128 uint32 lattice 21 -> 13.4, crowded P = 16 26 -> 15.4.
 // ---------------------------------------------------------------------------
 
-__device__ inline uint32_t lane_of(uint32_t v, uint32_t src)
-{
-    return (uint32_t)__builtin_amdgcn_readlane((int)v, (int)src);
-}
-
 // total_propensity's sum for a site of `count` particles in its first slots:
 // the same terms in the same order, a row of up to 8 pairs loaded at a time.
 // slots: the wave's copy of its sites' slots, slot-major, for this lane (a
@@ -680,15 +676,14 @@ __device__ inline float packed_propensity(const Params &p, uint32_t st, const ui
     return a;
 }
 
-// A reaction at lane src's site i (propensity a, words w): which one and the
-// site's new particles, by the whole wave.  Every lane of the wave calls it,
-// with its own site's values.
+// A reaction at lane src's site i (propensity a, words w), by the whole wave.
+// Every lane of the wave calls it, with its own site's values.
 template <class L>
 __device__ inline void wave_react(const Params &p, uint32_t *__restrict__ lat, uint32_t src, uint32_t i, uint32_t st,
                                   const uint32_t *w, float a, unsigned long long h3)
 {
-    constexpr uint32_t P = L::P, kNone = 0xFFFFFFFFu;
-    const uint32_t lane = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+    constexpr uint32_t P = L::P;
+    const uint32_t lane = lane_id();
     const uint32_t si = lane_of(i, src), sst = lane_of(st, src);
     // Lane j < P holds slot j.
     uint32_t word = 0;
@@ -698,130 +693,8 @@ __device__ inline void wave_react(const Params &p, uint32_t *__restrict__ lat, u
         if (lane / L::kPerWord == k) word = v;
     }
     const uint32_t mine = lane >= P ? 0u : L::part(word, L::kPerWord == 1 ? 0 : (int)(lane & 3u));
-    uint32_t earlier = 0;  // of the same species
-#pragma unroll 1
-    for (uint32_t q = 0; q < P; q++) earlier += q < lane && lane_of(mine, q) == mine ? 1u : 0u;
-    // determineReactionIndex (byte_reaction_dev.cu:146-177): the reactions in
-    // ascending index, each with a positive propensity moving rp, among those
-    // listed under a species of the site (lane j: of slot j, if it is the
-    // first of its kind) and the zero-order ones (lane P).
-    uint32_t start = 0, len = 0;
-    if (lane == P || (mine != 0u && earlier == 0u)) {
-        const uint32_t bucket = lane == P ? p.nS : mine - 1u;
-        start = p.rx_off[bucket];
-        len = p.rx_off[bucket + 1] - start;
-    }
-    uint32_t total = 0;
-#pragma unroll 1
-    for (uint32_t j = 0; j <= P; j++) total += lane_of(len, j);
-    float rp = uniform01(si, 1, 1, h3) * __uint_as_float(lane_of(__float_as_uint(a), src));
-    uint32_t idx = 0, r = kNone, s0 = p.sto_off[0], s1 = p.sto_off[1], k0 = s0, k1 = s1;
-    float pr = 0.0f;
-    bool any = false;
-    while (rp > 0.0f) {
-        uint32_t br = kNone;  // this lane's lowest reaction above idx, and its propensity
-        float bp = 0.0f;
-        uint32_t bs0 = 0, bs1 = 0;
-#pragma unroll 1
-        for (uint32_t c = 0; c < total; c += 64u) {
-            if (!any || total > 64u) {  // one a lane is evaluated once and kept
-                uint32_t left = c + lane, at = kNone;
-#pragma unroll 1
-                for (uint32_t j = 0; j <= P; j++) {
-                    const uint32_t lj = lane_of(len, j), sj = lane_of(start, j);
-                    if (left < lj) at = sj + left;
-                    left = left < lj ? kNone : left - lj;
-                }
-                if (c + lane >= total) at = kNone;
-                r = kNone;
-                if (at != kNone) {
-                    r = p.rx_list[at];
-                    const bool here = p.RL[r * p.nST + sst] != 0;
-                    const uint32_t d1 = p.D1[r], d2 = p.D2[r], order = p.order[r];
-                    const float k = p.rate[r];
-                    s0 = p.sto_off[r];
-                    s1 = p.sto_off[r + 1];
-                    float n1 = 0.0f, n2 = 0.0f;
-#pragma unroll 1
-                    for (uint32_t q = 0; q < P; q++) {
-                        const uint32_t s = lane_of(mine, q);
-                        n1 += s && s == d1 ? 1.0f : 0.0f;
-                        n2 += s && s == d2 ? 1.0f : 0.0f;
-                    }
-                    // (reaction_propensity's expressions)
-                    pr = order == kZeroOrder ? k
-                         : order == kFirstOrder ? k * n1
-                         : order == kSecondOrder ? k * n1 * n2
-                         : order == kSecondOrderSelf ? k * n1 * (n1 - 1.0f) : 0.0f;
-                    if (!here || !(pr > 0.0f)) r = kNone;
-                }
-            }
-            if (r != kNone && (!any || r > idx) && r < br) {
-                br = r;
-                bp = pr;
-                bs0 = s0;
-                bs1 = s1;
-            }
-        }
-        uint32_t low = kNone;
-#pragma unroll 1
-        for (unsigned long long m = __ballot(br != kNone); m; m &= m - 1) {
-            const uint32_t v = lane_of(br, (uint32_t)__builtin_ctzll(m));
-            low = v < low ? v : low;
-        }
-        if (low == kNone) break;
-        const uint32_t who = (uint32_t)__builtin_ctzll(__ballot(br == low));
-        rp -= __uint_as_float(lane_of(__float_as_uint(bp), who));
-        k0 = lane_of(bs0, who);
-        k1 = lane_of(bs1, who);
-        idx = low;
-        any = true;
-    }
-    // evaluateReaction (:179-257): the m-th particle of species s is consumed
-    // iff fewer than -S[s] earlier ones of s were seen, the others move up,
-    // and the products follow in species order.  A reactant that was not
-    // present leaves a negative residue, which the reference turns into an
-    // unbounded loop.
-    // Lane k holds the row's k-th nonzero entry (64 of them at a time).
-    uint32_t row_s = 0;
-    int row_v = 0;
-    auto row = [&](uint32_t c) {
-        row_s = 0;
-        row_v = 0;
-        if (c + lane < k1) {
-            row_s = p.sto_sp[c + lane] + 1u;
-            row_v = p.sto_val[c + lane];
-        }
-    };
-    row(k0);
-    int change = 0;
     bool underflow = false;
-#pragma unroll 1
-    for (uint32_t k = k0; k < k1; k++) {
-        if (k != k0 && ((k - k0) & 63u) == 0u) row(k);
-        const uint32_t s = lane_of(row_s, (k - k0) & 63u);
-        const int v = (int)lane_of((uint32_t)row_v, (k - k0) & 63u);
-        if (mine == s) change = v;
-        if (v < 0 && (int)__popcll(__ballot(mine == s)) < -v) underflow = true;
-    }
-    if (k1 - k0 > 64u) row(k0);
-    const bool stays = mine != 0u && (change >= 0 || (int)earlier >= -change);
-    const unsigned long long kept = __ballot(stays);
-    uint32_t n = (uint32_t)__popcll(kept);
-    const uint32_t to = stays ? __builtin_amdgcn_mbcnt_hi((uint32_t)(kept >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)kept, 0u))
-                              : 32u + (lane & 31u);  // (beyond the site)
-    uint32_t now = (uint32_t)__builtin_amdgcn_ds_permute((int)(to << 2), (int)mine);
-    if (lane >= n) now = 0u;
-#pragma unroll 1
-    for (uint32_t k = k0; k < k1; k++) {
-        if (k != k0 && ((k - k0) & 63u) == 0u) row(k);
-        const uint32_t s = lane_of(row_s, (k - k0) & 63u);
-#pragma unroll 1
-        for (int v = (int)lane_of((uint32_t)row_v, (k - k0) & 63u); v > 0; v--, n++) {
-            if (n < P) now = lane == n ? s : now;
-            else if (lane == 0u) record_overflow(p.ctl, 3, si, n - P, s);
-        }
-    }
+    const uint32_t now = wave_products<P>(p, si, sst, mine, __uint_as_float(lane_of(__float_as_uint(a), src)), h3, underflow);
     if (underflow && lane == 0u && atomicCAS(&p.ctl->error, 0u, kErrReactionUnderflow) == 0u)
         p.ctl->error_step = p.ctl->timestep;
     // Device-scope stores: the last block may resolve overflow entries beside them.

@@ -17,7 +17,7 @@
 // model (2000 particles) takes 16.5 us a step in boxes, two launches of which
 // none fills the device, and an ensemble pays every member's lattice in every
 // step although its members hold 2000 particles each.  One block steps them in
-// 11.8 us (12.4 us on 32^3, where 60 sites hold several particles), and an
+// 10.9 us (10.2 to 11.8 on 32^3, where 60 sites hold several particles), and an
 // ensemble runs a member per CU: 128 replicates on 32^3 to 128^3 sites take
 // 14.6 us a step against 970 us for the batched sweeps.
 //
@@ -28,7 +28,7 @@
 #include "lmx_device.h"
 #include "lmx_kernels.h"
 #include "lmx_resident.h"
-#include "lmx_site.h"
+#include "lmx_wave.h"
 
 namespace lmx {
 
@@ -111,58 +111,150 @@ __device__ inline void append(const Params &p, uint32_t *lat, ResidentLds &s, ui
     }
 }
 
-// The reactions of a site, by one thread: its particles (the members of its
-// chain in generation 1 that fit) as words, the shared evaluation, and, if it
-// changed, the result back as records of generation 0 -- in the members'
-// places, further ones appended.
+// Whether a site of several particles with total propensity a reacts
+// (checkForReaction, byte_reaction_dev.cu:139-144).  1 - exp(-a) <= a, with room
+// for the rounding of both, and u is 0 or at least 2^-32: most sites need no
+// exponential.
+__device__ inline bool reacts(float a, float u)
+{
+    if (a == 0.0f || !(u <= a * 1.0001f)) return false;
+    const float prob = reaction_probability(a);
+    return prob > 0.0f && u <= prob;
+}
+
+// The site of record e, by a wave: its total propensity a, or, if known is
+// set, its reaction.  The site's particles (the members of its chain in
+// generation 1 that fit) lie a slot per lane; a reaction's result goes back as
+// records of generation 0 -- in the members' places, further ones appended.
 template <class L>
-__device__ inline void react_chain(const Params &p, uint32_t *lat, ResidentLds &s, uint32_t key, uint32_t type,
+__device__ inline void react_site_wave(const Params &p, uint32_t *lat, ResidentLds &s, uint32_t e, bool known, float a,
+                                       uint32_t t, unsigned long long h3)
+{
+    constexpr uint32_t P = L::P;
+    const uint32_t lane = lane_id(), key = s.key[1][e], type = ord_type(s.ord[1][e]);
+    uint32_t mine = 0, rec = kDead;  // this lane's slot: its species and its record
+    for (uint32_t q = s.head[1][chain_of(key)] & ((1u << kIdBits) - 1u); q != kEnd; q = s.next[1][q]) {
+        if (s.key[1][q] != key || s.key[0][q] == kDead) continue;
+        const uint32_t o = s.ord[0][q];  // (its slot after the sweeps)
+        if (lane == (o & 15u)) {
+            mine = ord_species(o);
+            rec = q;
+        }
+    }
+    const uint32_t i = site_of(p, key);
+    if (!known) {
+        // total_propensity's sum: the same terms in the same order, a
+        // particle's row of them a lane each.
+        const uint32_t count = (uint32_t)__popcll(__ballot(mine != 0u));
+        a = p.qp0[type];
+#pragma unroll 1
+        for (uint32_t m = 0; m < count; m++) {
+            const uint32_t row = type * p.nS + lane_of(mine, m) - 1u;
+            float v = 0.0f;
+            if (lane == m) v = p.qp1[row];
+            else if (lane > m && lane < count) v = p.qp2[(size_t)row * p.nS + (mine - 1u)];
+#pragma unroll 1
+            for (uint32_t n = m; n < count; n++) a += __uint_as_float(lane_of(__float_as_uint(v), n));
+        }
+        if (!reacts(a, uniform01(i, 1, 0, h3))) return;
+    }
+    bool underflow;
+    const uint32_t now = wave_products<P>(p, i, type, mine, a, h3, underflow);
+    if (underflow && lane == 0u && atomicCAS(&p.ctl->error, 0u, kErrReactionUnderflow) == 0u) p.ctl->error_step = t;
+    if (lane >= P) return;
+    // products without a slot are overflow entries: only a full site has any
+    if (lane == P - 1u && now) s.ovf = 1u;
+    if (rec != kDead) {
+        if (now) s.ord[0][rec] = make_ord(lane, 0u, type, now);
+        else s.key[0][rec] = kDead;
+    } else if (now) {
+        append<L>(p, lat, s, key, make_ord(lane, 0u, type, now));
+    }
+}
+
+// total_propensity's sum for a site of 2 to K particles, in slot order: the
+// terms loaded together, added in its order.
+template <uint32_t K>
+__device__ inline float few_propensity(const Params &p, uint32_t type, const uint32_t *sp, uint32_t count)
+{
+    float a = p.qp0[type], one[K], two[K][K];
+    uint32_t row[K];
+#pragma unroll
+    for (uint32_t m = 0; m < K; m++) row[m] = (m < count ? sp[m] : sp[0]) - 1u;
+#pragma unroll
+    for (uint32_t m = 0; m < K; m++) {
+        const uint32_t r = type * p.nS + row[m];
+        one[m] = p.qp1[r];
+#pragma unroll
+        for (uint32_t n = m + 1u; n < K; n++) two[m][n] = p.qp2[(size_t)r * p.nS + row[n]];
+    }
+#pragma unroll
+    for (uint32_t m = 0; m < K; m++) {
+        if (m >= count) break;
+        a += one[m];
+#pragma unroll
+        for (uint32_t n = m + 1u; n < K; n++)
+            if (n < count) a += two[m][n];
+    }
+    return a;
+}
+
+// The nc sites listed in s.next[0], whose particles are several or whose one
+// passed its test.  A lane per site sums the propensities of up to kFew
+// particles; the sites that react, and those of more particles, are taken by
+// the whole wave.  Latency bounds it where the sites are few, so that one wave
+// takes up to 32 of them (32^3, 2000 particles, 60 sites: 10.2 us a step, dealt
+// to sixteen waves 10.7), and issue where they are many (16^3, 2000 particles:
+// 12.0, in one wave 15.6).  kFew: 12^3, 2500 particles 14.7 us a step, with 4
+// of them 16.3.
+//
+// A thread per site for everything, with the site's slots in registers,
+// unrolls the evaluation over every slot: with 16 of them 40 VGPRs and 138
+// SGPRs spilled at this block's 128, and 64^3 took 14.6 us a step against
+// 10.9 (8 slots, where nothing spilled: 11.4 against 10.9).
+template <class L>
+__device__ inline void react_sites(const Params &p, uint32_t *lat, ResidentLds &s, uint32_t nc, uint32_t t,
                                    unsigned long long h3, const float2 *tab)
 {
-    constexpr int W = L::W;
-    constexpr uint32_t P = L::P;
-    uint32_t w[W];
+    constexpr uint32_t kFew = L::P < 6 ? L::P : 6;
+    const uint32_t waves = nc <= 32u ? 1u : (nc >= 512u ? 16u : (nc + 31u) / 32u);
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    if (wave >= waves) return;
+#pragma unroll 1
+    for (uint32_t k0 = 0; k0 < nc; k0 += 64u * waves) {
+        const uint32_t k = k0 + lane_id() * waves + wave;
+        uint32_t e = 0, count = 0, type = 0, sp[kFew] = {};
+        float a = 0.0f, u = 1.0f;
+        bool hit = false;
+        if (k < nc) {
+            e = s.next[0][k];
+            const uint32_t key = s.key[1][e];
+            type = ord_type(s.ord[1][e]);
+            for (uint32_t q = s.head[1][chain_of(key)] & ((1u << kIdBits) - 1u); q != kEnd; q = s.next[1][q]) {
+                if (s.key[1][q] != key || s.key[0][q] == kDead) continue;
+                const uint32_t o = s.ord[0][q], j = o & 15u;
+                count++;
 #pragma unroll
-    for (int k = 0; k < W; k++) w[k] = 0u;
-    const uint32_t first = s.head[1][chain_of(key)] & ((1u << kIdBits) - 1u);
-    for (uint32_t q = first; q != kEnd; q = s.next[1][q]) {
-        if (s.key[1][q] != key || s.key[0][q] == kDead) continue;
-        const uint32_t o = s.ord[0][q], j = o & 15u;  // its slot after the sweeps
-#pragma unroll
-        for (int k = 0; k < W; k++) {
-            if constexpr (L::kPerWord == 4) {
-                if ((j >> 2) == (uint32_t)k) w[k] |= ord_species(o) << (8u * (j & 3u));
-            } else {
-                if (j == (uint32_t)k) w[k] = ord_species(o);
+                for (uint32_t m = 0; m < kFew; m++)
+                    if (j == m) sp[m] = ord_species(o);
             }
+            u = uniform01(site_of(p, key), 1, 0, h3);
         }
-    }
-    if (!react_site_table_l<L>(p, site_of(p, key), type, w, h3, tab)) return;
-    // products without a slot are overflow entries: only a full site has any
-    const uint32_t last = L::kPerWord == 4 ? w[W - 1] >> 24 : w[W - 1];
-    if (last) s.ovf = 1u;
-    uint32_t j = 0;  // the next slot to hand out
-    auto slot = [&](uint32_t k) -> uint32_t {
-        uint32_t v = 0;
-#pragma unroll
-        for (int q = 0; q < W; q++) {
-            if constexpr (L::kPerWord == 4) v = (k >> 2) == (uint32_t)q ? (w[q] >> (8u * (k & 3u))) & 0xFFu : v;
-            else v = k == (uint32_t)q ? w[q] : v;
+        const bool pairs = __ballot(count > 2u && count <= kFew) == 0ull;  // no site of three and more
+        if (count == 1u) {
+            const float2 ap = tab[type * p.nS + sp[0] - 1u];
+            a = ap.x;
+            hit = a != 0.0f && ap.y > 0.0f && u <= ap.y;
+        } else if (count >= 2u && count <= kFew) {
+            a = pairs ? few_propensity<2>(p, type, sp, count) : few_propensity<kFew>(p, type, sp, count);
+            hit = reacts(a, u);
         }
-        return v;
-    };
-    for (uint32_t q = first; q != kEnd; q = s.next[1][q]) {
-        if (s.key[1][q] != key) continue;
-        const uint32_t sp = j < P ? slot(j) : 0u;
-        s.key[0][q] = sp ? key : kDead;
-        s.ord[0][q] = make_ord(j, 0u, type, sp);
-        if (sp) j++;
-    }
-    while (j < P) {
-        const uint32_t sp = slot(j);
-        if (!sp) break;
-        append<L>(p, lat, s, key, make_ord(j, 0u, type, sp));
-        j++;
+#pragma unroll 1
+        for (unsigned long long m = __ballot(hit || count > kFew); m; m &= m - 1) {
+            const uint32_t src = (uint32_t)__builtin_ctzll(m);
+            react_site_wave<L>(p, lat, s, lane_of(e, src), lane_of(count, src) <= kFew,
+                               __uint_as_float(lane_of(__float_as_uint(a), src)), t, h3);
+        }
     }
 }
 
@@ -551,9 +643,9 @@ __device__ __attribute__((always_inline)) inline void run_body(const ResidentJob
                 s.ord[0][e] = make_ord(before, 0u, st, sp);
                 // A particle alone takes its reaction test from the table; a
                 // site that reacts or holds several is evaluated after the
-                // barrier, one thread per site in as few waves as they need
-                // (beside this loop, every wave with such a site ran the whole
-                // evaluation: 19,000 of a step's 40,000 cycles).
+                // barrier, by a wave of its own (beside this loop, every wave
+                // with such a site ran the whole evaluation: 19,000 of a
+                // step's 40,000 cycles).
                 if (p.R > 0 && before == 0u) {
                     bool whole = total > 1u;
                     if (!whole) {
@@ -567,10 +659,7 @@ __device__ __attribute__((always_inline)) inline void run_body(const ResidentJob
             __syncthreads();
             const uint32_t nc = s.nc;
             if (nc) {
-                for (uint32_t k = tid; k < nc; k += kNT) {
-                    const uint32_t e = s.next[0][k];
-                    react_chain<L>(p, lat, s, s.key[1][e], ord_type(s.ord[1][e]), h3, tab);
-                }
+                react_sites<L>(p, lat, s, nc, t, h3, tab);
                 __syncthreads();
                 if (tid == 0) s.nc = 0u;
             }

@@ -163,3 +163,61 @@ def test_autotune_of_a_resident_solver_keeps_the_state(gpu):
         assert orc.run(9) == 0
         assert np.array_equal(s.getLatticeNative(), orc.native()) and s.timestep == 11
         s.close()
+
+
+MEMBERS = [
+    # shape, particles per slot, boundary
+    ((12, 10, 8), 0.15, "periodic"),
+    ((4, 6, 5), 0.6, "reflecting"),     # sites of many particles, overflow entries
+    ((16, 16, 24), 0.02, "periodic"),
+    ((8, 3, 40), 0.1, "reflecting"),
+]
+
+
+@pytest.mark.parametrize("P", [4, 8, 16])
+def test_ensemble_of_resident_members(gpu, P):
+    """Every slot count, in calls of four steps and more, from lattices of
+    single particles to sites of all their slots."""
+    ens = lmx.Ensemble(0)
+    pairs = []
+    for k, (shape, density, boundary) in enumerate(MEMBERS):
+        spec = models.random_model(shape=shape, P=P, nS=5, nST=3, R=9, density=density, seed=90 + k, boundary=boundary,
+                                   include_zero_order=False, rate_scale=0.1)
+        assert 0 < int(spec.initial_counts().sum()) <= 3000
+        s = lmx.MpdRdmeSolver(0)
+        spec.load_into(s, replicate=k, seed=5)
+        ens.add(s)
+        pairs.append((s, oracle.Oracle(spec, seed_top=5, replicate=k)))
+    for chunk in (4, 7, 12):
+        ens.run(chunk)
+        for s, orc in pairs:
+            assert orc.run(chunk) == 0
+            got = s.getLatticeNative()
+            assert np.array_equal(got, orc.native()), f"{s.shape}: {(got != orc.native()).sum()} words differ"
+            assert s.getOverflowStats() == (orc.stats.overflow_entries, orc.stats.overflow_steps)
+    assert pairs[1][1].stats.overflow_entries > 0
+    ens.close()
+
+
+@pytest.mark.parametrize("words", [False, True], ids=["byte", "uint32"])
+@pytest.mark.parametrize("P", [4, 8, 16])
+def test_resident_reactions_of_full_sites(gpu, P, words):
+    """Reactions of one to three products at sites of up to all their slots:
+    records that are reused, that die and that are appended."""
+    for shape, density in (((6, 5, 4), 0.5), ((20, 18, 16), 2400 / (20 * 18 * 16 * P))):
+        spec = models.random_model(shape=shape, P=P, nS=6, nST=2, R=12, density=density, seed=7, include_zero_order=False,
+                                   rate_scale=0.2)
+        assert 0 < int(spec.initial_counts().sum()) <= 3000
+        if words:
+            spec.lattice = spec.lattice.astype(np.uint32)
+        s = (lmx.IntMpdRdmeSolver if words else lmx.MpdRdmeSolver)(0)
+        spec.load_into(s, seed=8)
+        orc = oracle.Oracle(spec, seed_top=8)
+        changed = orc.species_counts()
+        for chunk in (4, 16):
+            s.runTimesteps(chunk)
+            assert orc.run(chunk) == 0
+            got = s.getLatticeNative()
+            assert np.array_equal(got, orc.native()), f"{shape}: {(got != orc.native()).sum()} words differ"
+        assert not np.array_equal(changed, orc.species_counts())
+        s.close()
