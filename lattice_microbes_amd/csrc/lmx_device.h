@@ -300,6 +300,18 @@ __device__ inline void clear_chunk_flag(const Params &p, uint32_t *lat, uint32_t
         __hip_atomic_store(f, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// Waits until every store and atomic that the wave has issued is done.  With a
+// block barrier after it, what the block wrote at device scope is visible to
+// whoever then sees the block counted as finished, without the L2 write-back
+// of a release.  The compiler may move memory accesses across the bare wait,
+// so it stands between fences that only the compiler sees.
+__device__ inline void wait_for_stores()
+{
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    __builtin_amdgcn_s_waitcnt(0);
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+}
+
 // Clears the zero flag of site i's box in plane k (boxed step) after a
 // nonzero write.
 __device__ inline void clear_zero_flag(const Params &p, uint32_t k, uint32_t i)

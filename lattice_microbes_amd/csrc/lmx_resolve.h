@@ -285,7 +285,7 @@ __device__ inline void resolve_body(const Params &p, uint32_t *lat)
                 const uint32_t r = upto < count ? f_room[upto] : 1u;
                 failure = r == 0u ? kErrUnplaceable : (r == kOut ? kErrOutOfRange : 0u);
             }
-            __builtin_amdgcn_s_waitcnt(0);  // the next round's loads see the stores
+            wait_for_stores();  // the next round's loads see the stores
         }
         __syncthreads();
         if (failure != 0u) {

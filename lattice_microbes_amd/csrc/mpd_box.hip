@@ -436,7 +436,7 @@ __device__ __attribute__((always_inline)) inline bool box_pass(const BoxCtx<L, C
             }
         }
         // The zeros are in place before any wave of the block writes over them.
-        if (axis == 2) __builtin_amdgcn_s_waitcnt(0);
+        if (axis == 2) wait_for_stores();
         __syncthreads();
     }
 
@@ -778,7 +778,7 @@ __device__ __attribute__((always_inline)) inline void cand_react_body(const Para
     // (What it reads of this launch, lattice words and entries, is stored and
     // loaded at device scope, so waiting for the stores is enough: no fence,
     // which would write back and invalidate the L2.)
-    __builtin_amdgcn_s_waitcnt(0);  // every wave's stores have arrived
+    wait_for_stores();  // every wave's have arrived
     __syncthreads();
     if (threadIdx.x == 0) last = atomicAdd(&ctl->blocks_done, 1u) == nblocks - 1u ? 1u : 0u;
     __syncthreads();

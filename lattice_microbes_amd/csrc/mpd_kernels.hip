@@ -159,7 +159,7 @@ __global__ __launch_bounds__(256) void count_kernel(const uint32_t *__restrict__
     __syncthreads();
     for (uint32_t k = threadIdx.x + 1u; k < kCountBins && k <= nS; k += blockDim.x)
         if (hist[k]) atomicAdd(&counts[k - 1], hist[k]);
-    __builtin_amdgcn_s_waitcnt(0);  // the additions are done
+    wait_for_stores();  // the additions are done
     __syncthreads();
     if (threadIdx.x == 0) last = atomicAdd(&counts[nS], 1u) == gridDim.x - 1u ? 1u : 0u;
     __syncthreads();
