@@ -834,18 +834,14 @@ hipError_t launch_box_reactions(const Params &p, const BoxGeom &g, uint32_t *lat
 hipError_t launch_box_step(const Params &p, const BoxGeom &g, const uint32_t *src, uint32_t *dst, const uint32_t *zs,
                            uint32_t *zd, const CandList &rl, hipStream_t st)
 {
-    // Waves per SIMD: the most whose registers do not spill.  (The uint32
-    // lattice's 8 slots at six waves and 16 slots at four spilled 3 and 6
-    // VGPRs: 128x64x80, 40000 particles 24.6 -> 24.3 and 27.8 -> 27.2 us a
-    // step without.)
     const int key = p.word_particles ? 100 + (int)p.P : (int)p.W;
     switch (key) {
     case 1: return launch_box<ByteSites<1>, box_cap(4), 7>(p, g, src, dst, zs, zd, rl, st);
     case 2: return launch_box<ByteSites<2>, box_cap(8), 7>(p, g, src, dst, zs, zd, rl, st);
     case 4: return launch_box<ByteSites<4>, box_cap(16), 6>(p, g, src, dst, zs, zd, rl, st);
     case 104: return launch_box<WordSites<4>, box_cap(4), 6>(p, g, src, dst, zs, zd, rl, st);
-    case 108: return launch_box<WordSites<8>, box_cap(8), 5>(p, g, src, dst, zs, zd, rl, st);
-    case 116: return launch_box<WordSites<16>, box_cap(16), 3>(p, g, src, dst, zs, zd, rl, st);
+    case 108: return launch_box<WordSites<8>, box_cap(8), 6>(p, g, src, dst, zs, zd, rl, st);
+    case 116: return launch_box<WordSites<16>, box_cap(16), 4>(p, g, src, dst, zs, zd, rl, st);
     }
     return hipErrorInvalidValue;
 }

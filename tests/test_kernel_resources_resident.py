@@ -1,6 +1,6 @@
-"""Register budget of the resident kernels and of the boxed step's in every
-slot layout, from the compiler's report of the last build: a resident block of
-16 waves has 128 VGPRs a lane, and its records fill the LDS of a CU."""
+"""Register budget of the resident kernels of every slot layout, from the
+compiler's report of the last build: a block of 16 waves has 128 VGPRs a lane,
+and its records fill the LDS of a CU."""
 import os
 
 import pytest
@@ -21,18 +21,3 @@ def test_resident_kernels_of_every_layout_do_not_spill(kernel, layout):
     r = res[names[0]]
     assert r["ScratchSize"] == 0 and r["VGPRs Spill"] == 0, r
     assert r["Occupancy"] >= 4 and r["LDS Size"] <= 163840, r
-
-
-@pytest.mark.parametrize("layout,waves", [("9ByteSitesILi1E", 7), ("9ByteSitesILi2E", 7), ("9ByteSitesILi4E", 6),
-                                          ("9WordSitesILi4E", 6), ("9WordSitesILi8E", 5), ("9WordSitesILi16E", 3)])
-def test_boxed_kernels_of_every_layout_do_not_spill(layout, waves):
-    """Single solvers' kernels; a batch's (byte lattice) keep as many waves and
-    may spill a register or two."""
-    res = build.kernel_resources()
-    for kernel in ("box_step_kernel", "cand_react_kernel", "cand_react_jobs_kernel"):
-        for n in [n for n in res if f"{kernel}INS_{layout}E" in n]:
-            assert res[n]["ScratchSize"] == 0, (n, res[n])
-    step = [n for n in res if f"box_step_kernelINS_{layout}E" in n]
-    assert len(step) == 2 and all(res[n]["Occupancy"] >= waves for n in step), step
-    for n in [n for n in res if f"box_jobs_kernelINS_{layout}E" in n]:
-        assert res[n]["ScratchSize"] <= 16 and res[n]["Occupancy"] >= waves, (n, res[n])
