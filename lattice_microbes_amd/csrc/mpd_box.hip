@@ -834,6 +834,10 @@ hipError_t launch_box_reactions(const Params &p, const BoxGeom &g, uint32_t *lat
 hipError_t launch_box_step(const Params &p, const BoxGeom &g, const uint32_t *src, uint32_t *dst, const uint32_t *zs,
                            uint32_t *zd, const CandList &rl, hipStream_t st)
 {
+    // Waves per SIMD: the most without a spill, but for the uint32 lattice's 8
+    // and 16 slots, which spill 3 and 6 VGPRs.  (With one wave fewer each they
+    // spill none and take 128x128x256 with a crowded spot from 125 to 139 and
+    // from 189 to 232 us a step.)
     const int key = p.word_particles ? 100 + (int)p.P : (int)p.W;
     switch (key) {
     case 1: return launch_box<ByteSites<1>, box_cap(4), 7>(p, g, src, dst, zs, zd, rl, st);

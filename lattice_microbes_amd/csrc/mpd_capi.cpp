@@ -380,12 +380,58 @@ void set_box_level(lmx_solver *s, uint32_t level)
     s->zflags_fresh[0] = s->zflags_fresh[1] = false;
 }
 
+// Whether a lattice that only boxes of at most `level` fit is stepped in them,
+// by the sites up to which they are the faster.  Boxes of 4 cost 6 ns each
+// (23 ps a site) and 20 to 50 ps a record of their regions, which hold 2.5
+// times their particles; the sweeps 8 to 40 ps a site and 50 ps a particle, but
+// more launches.  So small boxes pay on small lattices, and where the sweeps are
+// slow.  us a step, boxes against sweeps, bimolecular model, particles a site
+// (spot: 32^3 crowded sites in a sparse lattice):
+//   8 slots             96^3 0.5 60/78, 160x160x100 0.5 129/124, 256^3 0.5
+//                       733/486, spot 128x128x256 101/55
+//   8 slots, X % 4 != 0 63x61x151 0.5 54/44, spot 95x93x91 42/31
+//   16 slots            256x256x64 0.85 282/357, spot 128x128x256 in 0.01 116/104,
+//                       in 0.04 124/127
+//   16 slots, X % 4     63x61x151 0.7 64/61 (with 40 reactions 69/80),
+//                       255x255x65 0.6 278/244, spot 255x253x129 285/215
+//   4 slots             256x256x64 0.5 465/631, spot 128x128x256 105/58, 96^3 41/49,
+//                       95x93x91 47/38
+//   4 slots, no reactions  96^3 0.4 169/145; in boxes of 6 96^3 0.3 63/66,
+//                       256x256x64 0.3 247/217
+//   uint32, 8 slots     32^3 0.5 31/31, 96^3 0.5 76/72, spot 255x253x129 297/334
+//   uint32, 16 slots    32^3 0.6 36/40, 96^3 0.6 117/105, spot 255x253x129 388/715
+// Boxes of 6 lose only to a spot in a large sparse lattice (8 slots 128x128x256
+// 59/54, 256^3 177/134).
+bool box_level_pays(const lmx_solver *s, uint32_t level)
+{
+    const bool bytes = s->bpp == 1, rows4 = (s->X & 3u) == 0, spot = s->particles < s->N / 4;
+    const bool idle4 = bytes && s->P == 4 && s->R == 0;
+    const size_t any = ~(size_t)0;
+    size_t most = any;
+    if (level + 1u < lmx::kBoxLevels) {
+        if (lmx::kBoxLevel[level] <= 6u && idle4) most = 1u << 20;
+        else if (lmx::kBoxLevel[level] <= 6u && bytes && rows4 && s->P <= 8 && spot) most = 1u << 21;
+    } else if (!bytes) {
+        most = spot ? any : 1u << 16;
+    } else if (idle4) {
+        most = 1u << 15;
+    } else if (s->P == 4) {
+        most = !spot ? any : (rows4 ? 3u << 19 : 0u);
+    } else if (s->P == 8) {
+        most = rows4 ? 3u << 19 : 0u;
+    } else {
+        most = rows4 ? (s->particles < s->N / 32 ? 3u << 19 : any) : (spot ? 0u : 1u << 20);
+    }
+    return s->N <= most;
+}
+
 // The boxes for a lattice with particles at the given sites: the largest whose
 // fullest region, scaled from the fullest box, takes at most 3/4 of the
 // records a block holds.  A region that holds more is halved by its block, at
 // several times the cost, so the rule leaves room for fluctuations; on the
 // 128x64x80 bimolecular lattice (P = 8) the sweeps take 26-64 us a step from
-// 0.01 to 0.4 particles a site, the boxes that fit 18-38 us.
+// 0.01 to 0.4 particles a site, the boxes that fit 18-38 us.  Where only the
+// smallest boxes fit, the sweeps may be the faster (box_level_pays).
 // Smaller ones than those while their blocks still run all at once: a launch
 // then lasts as long as its fullest block, of which smaller boxes are shorter
 // (capsule 128x128x256, boxes of 14 -> 10: 25.6 -> 22.4 us a step; 63x61x151,
@@ -421,7 +467,7 @@ void plan_boxes(lmx_solver *s, const std::vector<uint32_t> &at)
             full = std::max(full, count);
         }
         if (fits < lmx::kBoxLevels && active > kAtOnce) break;
-        if (full <= most) fits = level;
+        if (full <= most && (fits < lmx::kBoxLevels || box_level_pays(s, level))) fits = level;
         if (fits < lmx::kBoxLevels && (active > kAtOnce || full <= kShort)) break;
     }
     set_box_level(s, fits);
@@ -472,8 +518,10 @@ int check_report(lmx_solver *s, const uint32_t *hdr)
     // more crowded): smaller boxes from now on.
     const uint32_t splits = hdr[offsetof(lmx::Control, box_splits) / sizeof(uint32_t)] - s->splits_seen;
     if (s->diffusion_built && s->box_level < lmx::kBoxLevels && s->timestep > s->splits_step &&
-        splits > (s->timestep - s->splits_step) * (1u + s->box.nboxes / 256u))
-        set_box_level(s, s->box_level + 1);
+        splits > (s->timestep - s->splits_step) * (1u + s->box.nboxes / 256u)) {
+        const uint32_t next = s->box_level + 1;
+        set_box_level(s, next < lmx::kBoxLevels && box_level_pays(s, next) ? next : lmx::kBoxLevels);
+    }
     s->splits_seen += splits;
     s->splits_step = s->timestep;
     s->unchecked = hdr[2] != 0 || s->own_work;

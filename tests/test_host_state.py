@@ -324,3 +324,48 @@ def test_autotune_tells_boxes_from_tiles(lib, box, boxes):
     with pytest.raises(lmx.InvalidArgException):
         s.getLaunchOption(99)
     s.close()
+
+
+def _crowded(shape, P, density, spot, words, R):
+    """Uniform particles, one a site, and a cube of 32^3 sites (at most) with
+    `spot` a site."""
+    spec = models.bimolecular(shape=shape, nA=1, nB=1, P=P, seed=1)
+    if not R:
+        spec = models.random_model(shape=shape, P=P, nS=3, nST=1, R=0, density=0.0, seed=1)
+    rng = np.random.default_rng(3)
+    first = rng.random(shape) < density
+    if spot:
+        first[:32, :32, :32] = rng.random(first[:32, :32, :32].shape) < spot
+    spec.lattice = np.zeros(shape + (P,), np.uint32 if words else np.uint8)
+    spec.lattice[..., 0] = first
+    return spec
+
+
+@pytest.mark.parametrize("shape,P,density,spot,words,R,boxes", [
+    ((96, 96, 96), 8, 0.5, 0, False, 2, True),
+    ((160, 160, 100), 8, 0.5, 0, False, 2, False),
+    ((160, 160, 100), 8, 0.2, 0, False, 2, True),
+    ((160, 160, 100), 8, 0.01, 0.6, False, 2, False),
+    ((96, 96, 96), 8, 0.01, 0.6, False, 2, True),
+    ((63, 61, 151), 8, 0.5, 0, False, 2, False),
+    ((63, 61, 151), 8, 0.3, 0, False, 2, True),
+    ((160, 160, 100), 16, 0.8, 0, False, 2, True),
+    ((63, 61, 151), 16, 0.5, 0, False, 2, True),
+    ((95, 93, 91), 16, 0.01, 0.9, False, 2, False),
+    ((96, 96, 96), 4, 0.5, 0, False, 2, True),
+    ((96, 96, 96), 4, 0.45, 0, False, 0, False),
+    ((96, 96, 96), 4, 0.3, 0, False, 0, True),
+    ((96, 96, 96), 8, 0.5, 0, True, 2, False),
+    ((96, 96, 96), 8, 0.2, 0, True, 2, True),
+    ((95, 93, 91), 8, 0.01, 0.6, True, 2, True),
+    ((32, 32, 32), 8, 0.5, 0, True, 2, True),
+])
+def test_crowded_lattices_step_in_what_is_faster(lib, shape, P, density, spot, words, R, boxes):
+    """Both sides of each line of the rule for the smallest boxes that fit."""
+    spec = _crowded(shape, P, density, spot, words, R)
+    s = (lmx.IntMpdRdmeSolver if words else lmx.MpdRdmeSolver)(0)
+    spec.load_into(s, seed=2)
+    log(lib)
+    s.runTimesteps(1)
+    assert [l.split()[0] for l in log(lib) if l.startswith(("box", "sweep"))] == ["box" if boxes else "sweep"]
+    s.close()
