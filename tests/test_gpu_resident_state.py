@@ -221,3 +221,41 @@ def test_resident_reactions_of_full_sites(gpu, P, words):
             assert np.array_equal(got, orc.native()), f"{shape}: {(got != orc.native()).sum()} words differ"
         assert not np.array_equal(changed, orc.species_counts())
         s.close()
+
+
+class RelaxedInt(lmx.IntMpdRdmeSolver):
+    _parses_overflow_handler = True
+
+
+def _spot(shape, P, spot, density, seed, boundary):
+    """A sparse lattice with a crowded corner, so that a run in one block has
+    overflow entries in every step."""
+    spec = models.random_model(shape=shape, P=P, nS=6, nST=2, R=9, density=0.002, seed=seed, boundary=boundary,
+                               include_zero_order=False)
+    corner = spec.lattice[tuple(slice(0, k) for k in spot)]
+    rng = np.random.default_rng(seed)
+    corner[...] = np.where(rng.random(corner.shape) < density, rng.integers(1, 7, corner.shape), 0)
+    return spec
+
+
+@pytest.mark.parametrize("words", [False, True], ids=["byte", "uint32"])
+@pytest.mark.parametrize("handler", ["classic", "relaxed"])
+@pytest.mark.parametrize("P,spot,density", [(4, (10, 9, 8), 0.6), (8, (8, 7, 6), 0.75), (16, (5, 5, 6), 0.85)])
+def test_overflow_entries_of_resident_runs(gpu, P, spot, density, handler, words):
+    spec = _spot((30, 28, 24), P, spot, density, 12, "periodic" if P == 8 else "reflecting")
+    n = int((spec.lattice != 0).sum())
+    assert 0 < n <= 3000
+    if words:
+        spec.lattice = spec.lattice.astype(np.uint32)
+    orc = oracle.Oracle(spec, seed_top=7, replicate=2, overflow=handler)
+    s = (RelaxedInt if words else lmx.MpdRdmeSolver)(0)
+    spec.load_into(s, replicate=2, seed=7, extra={"rdme.mpd.overflowhandler": handler})
+    for chunk in (10, 4, 11):
+        s.runTimesteps(chunk)
+        assert orc.run(chunk) == 0
+        got = s.getLatticeNative()
+        assert np.array_equal(got, orc.native()), f"{(got != orc.native()).sum()} words differ"
+        assert s.getOverflowStats() == (orc.stats.overflow_entries, orc.stats.overflow_steps)
+        assert s.getUnresolvedOverflows() == orc.unresolved
+    assert orc.stats.overflow_entries > 20
+    s.close()

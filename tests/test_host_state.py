@@ -369,3 +369,18 @@ def test_crowded_lattices_step_in_what_is_faster(lib, shape, P, density, spot, w
     s.runTimesteps(1)
     assert [l.split()[0] for l in log(lib) if l.startswith(("box", "sweep"))] == ["box" if boxes else "sweep"]
     s.close()
+
+
+@pytest.mark.parametrize("P,n,resident", [(4, 1000, True), (4, 1001, False), (8, 2000, True), (8, 2001, False),
+                                          (16, 3000, True)])
+def test_crowded_lattices_are_not_run_in_one_block(lib, P, n, resident):
+    spec = models.random_model(shape=(10, 10, 10), P=P, nS=3, nST=1, R=0, density=0.0, seed=1)
+    spec.lattice = np.zeros(1000 * P, np.uint8)
+    spec.lattice[np.random.default_rng(1).permutation(1000 * P)[:n]] = 1
+    spec.lattice = spec.lattice.reshape(10, 10, 10, P)
+    s = lmx.MpdRdmeSolver(0)
+    spec.load_into(s, seed=1)
+    log(lib)
+    s.runTimesteps(8)
+    assert any(l.startswith("resident") for l in log(lib)) == resident
+    s.close()
