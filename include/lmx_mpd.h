@@ -168,7 +168,7 @@ int lmx_get_launch_option(lmx_solver *s, int option, int *value);
  * block shapes at build time, options.cmake TUNE_MPD_*).  From the current
  * state it times nsteps steps (after one untimed step) of the default step
  * (boxes, or one block for the whole call where lmx_run_steps takes one; then
- * at least four steps) and of each y/z sweep kernel and window shape: LDS row
+ * at least as many steps as such a call has) and of each y/z sweep kernel and window shape: LDS row
  * tiles with and without the reaction list, register march and register
  * columns of 4 and 8 rows, compacted tiles, and the fused step.  It restores the state after each, times two interleaved
  * passes and keeps the fastest by the minimum of each, but keeps the current
@@ -188,8 +188,9 @@ int lmx_autotune(lmx_solver *s, uint32_t nsteps, double *best_ms, int *chosen);
  * solver's stream without a host synchronization per step (the reference
  * synchronizes every step, :1091).  Device-side errors are sticky and are
  * reported by the next lmx_synchronize.  Four or more steps of a solver of at
- * most 3000 particles without zero-order reactions run in one block in a
- * single launch; if the particles outgrow the block, the steps it left out run
+ * most 2048 particles without zero-order reactions run in one block in a
+ * single launch, as do eight or more of at most 3000 (four on lattices of more
+ * than 128^3 sites), unless the lattice is crowded; if the particles outgrow the block, the steps it left out run
  * (with a wait for the ones before them) in the next call that looks at the
  * state, uploads new rates or rebuilds the solver; calls that only enqueue
  * steps never wait for that. */

@@ -713,9 +713,15 @@ int enqueue_step(lmx_solver *s, const lmx::Params &p0, hipEvent_t *ev, int *kind
     return LMX_OK;
 }
 
-// Steps of one lmx_run_steps call from which a resident run pays for listing
-// the particles and writing them back.
-constexpr uint32_t kResidentMinSteps = 4;
+// Steps of one call from which a resident run pays for listing the particles
+// and writing them back.  More than two records a thread take half as long
+// again, so that alone on a small lattice it takes more of them (64^3, 3000
+// particles, us a call of 4 steps: one block 109, boxes 80, sweeps 96; of 10
+// steps 203, 177, 221; 256^3, 4 steps 121, 221, 374).
+uint32_t resident_min_steps(const lmx_solver *s, bool alone)
+{
+    return alone && s->particles > 2u * lmx::kResidentThreads && s->N <= 1u << 21 ? 8u : 4u;
+}
 
 // Whether the sites of a lattice hold so many particles that its overflow
 // entries and sites of many particles, which a resident run takes one after
@@ -731,9 +737,9 @@ bool crowded(const lmx_solver *s)
 // A solver of few particles runs in one block: the default options, no
 // zero-order reactions (they would need every empty site).  The bimolecular
 // 64^3 model (2000 particles) takes 16.5 us a step in boxes, 10.9 in one block.
-bool use_resident(const lmx_solver *s, uint32_t nsteps)
+bool use_resident(const lmx_solver *s, uint32_t nsteps, bool alone)
 {
-    return nsteps >= kResidentMinSteps && s->resident_ok && s->particles <= lmx::kResidentMost && !crowded(s) && !s->any_qp0 &&
+    return nsteps >= resident_min_steps(s, alone) && s->resident_ok && s->particles <= lmx::kResidentMost && !crowded(s) && !s->any_qp0 &&
            s->boxes && s->path == LMX_PATH_SWEEPS && s->yz_kernel == 0 && s->fuse_reaction && !s->force_generic;
 }
 
@@ -762,7 +768,7 @@ void resident_ran(lmx_solver *s, uint32_t nsteps)
 // nsteps timesteps: a resident run, or one step's launches after another.
 int enqueue_steps(lmx_solver *s, uint32_t nsteps, const lmx::ReactionList *rl = nullptr)
 {
-    if (use_resident(s, nsteps)) {
+    if (use_resident(s, nsteps, true)) {
         while (nsteps) {
             const uint32_t m = std::min(nsteps, lmx::kResidentMaxSteps);
             const hipError_t e = lmx::launch_resident(resident_job(s, m), nullptr, 1, lmx::resident_gather_blocks((uint32_t)s->N),
@@ -1557,15 +1563,15 @@ int lmx_autotune(lmx_solver *s, uint32_t nsteps, double *best_ms, int *chosen)
                 s->fuse_reaction = c.fuse_reaction;
                 s->boxes = c.boxes;
                 // As lmx_run_steps would step: in one block where it does (in
-                // calls of kResidentMinSteps and more, so at least that many),
+                // calls of some steps and more, so at least that many),
                 // unless that stops short, which is timed once more without.
                 float ms = 0.0f;
                 uint32_t timed = 0;
                 for (bool again = true; again && !rc;) {
                     if ((rc = restore())) break;
                     if ((rc = enqueue_step(s, make_params(s), nullptr, nullptr, nullptr))) break;  // untimed first step
-                    const uint32_t longer = std::max(nsteps, kResidentMinSteps);
-                    timed = use_resident(s, longer) ? longer : nsteps;
+                    const uint32_t longer = std::max(nsteps, resident_min_steps(s, true));
+                    timed = use_resident(s, longer, true) ? longer : nsteps;
                     LMX_HIP(hipEventRecord(e0, s->stream));
                     if ((rc = enqueue_steps(s, timed))) break;
                     LMX_HIP(hipEventRecord(e1, s->stream));
@@ -1995,7 +2001,7 @@ int batch_jobs(lmx_batch *b, uint32_t nsteps)
     b->resident.clear();
     const bool alone = b->use_list && b->tile_threads == 0;
     for (lmx_solver *s : b->members)
-        (!alone ? b->stepped : (use_resident(s, nsteps) ? b->resident : (use_boxes(s) ? b->boxed : b->stepped))).push_back(s);
+        (!alone ? b->stepped : (use_resident(s, nsteps, false) ? b->resident : (use_boxes(s) ? b->boxed : b->stepped))).push_back(s);
     if (int rc = batch_boxes(b)) return rc;
     const uint32_t n = (uint32_t)b->resident.size();
     if (int rc = batch_room(b->d_jobs, b->h_jobs, b->jobs_cap, n, 16)) return rc;
@@ -2378,11 +2384,12 @@ int lmx_batch_autotune(lmx_batch *b, uint32_t nsteps, double *best_ms, int *chos
         };
         if ((rc = copy_state(true))) return rc;
 
-        // Members that run in one block do so in calls of at least
-        // kResidentMinSteps.
+        // Members that run in one block do so in calls of some steps and more.
         uint32_t timed = nsteps;
-        for (const lmx_solver *s : b->members)
-            if (use_resident(s, kResidentMinSteps)) timed = std::max(nsteps, kResidentMinSteps);
+        for (const lmx_solver *s : b->members) {
+            const uint32_t longer = std::max(nsteps, resident_min_steps(s, false));
+            if (use_resident(s, longer, false)) timed = std::max(timed, longer);
+        }
 
         struct Config {
             bool list;

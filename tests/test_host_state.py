@@ -243,7 +243,7 @@ def test_crowded_small_lattices_are_counted(lib, n, resident, by):
                 packed[j // 4, z, y, x] |= np.uint32(1 << (8 * (j % 4)))
         s.setLatticeNative(packed)
     log(lib)
-    s.runTimesteps(4)
+    s.runTimesteps(8)
     assert any(l.startswith("resident") for l in log(lib)) == resident
     s.close()
 
@@ -384,3 +384,21 @@ def test_crowded_lattices_are_not_run_in_one_block(lib, P, n, resident):
     s.runTimesteps(8)
     assert any(l.startswith("resident") for l in log(lib)) == resident
     s.close()
+
+
+@pytest.mark.parametrize("edge,n,steps,resident", [(64, 2048, 3, False), (64, 2048, 4, True), (64, 2049, 7, False),
+                                                   (64, 2049, 8, True), (160, 2049, 4, True)])
+def test_short_calls_of_more_particles_than_two_a_thread(lib, edge, n, steps, resident):
+    """Alone on a small lattice; beside others in an ensemble they run in one
+    block from four steps on."""
+    s = lmx.MpdRdmeSolver(0)
+    models.bimolecular(shape=(edge,) * 3, nA=n // 2, nB=n - n // 2, seed=1).load_into(s, seed=2)
+    log(lib)
+    s.runTimesteps(steps)
+    assert any(l.startswith("resident") for l in log(lib)) == resident
+    ens = lmx.Ensemble(0, graph=False)
+    ens.add(s)
+    log(lib)
+    ens.run(steps)
+    assert any(l.startswith("resident") for l in log(lib)) == (steps >= 4)
+    ens.close()
