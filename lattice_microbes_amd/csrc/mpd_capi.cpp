@@ -14,6 +14,7 @@
 #include <cmath>
 #include <cstddef>
 #include <cstring>
+#include <memory>
 #include <string>
 #include <vector>
 
@@ -291,50 +292,67 @@ int require_ready(lmx_solver *s)
     return rc ? rc : settle(s);
 }
 
-// Particles of a lattice that are listed for plan_boxes: one more than the
-// most that its rules look at (a particle a site for boxes, kResidentMost for
-// resident runs).
-size_t listed_most(const lmx_solver *s) { return std::max<size_t>(s->N, lmx::kResidentMost) + 1; }
+// The native site index of every particle of a lattice, for plan_boxes: one
+// more at most than its rules look at (a particle a site for boxes,
+// kResidentMost for resident runs).
+struct SiteList {
+    size_t most, n = 0;
+    std::unique_ptr<uint32_t[]> at;
+    explicit SiteList(const lmx_solver *s)
+        : most(std::max<size_t>(s->N, lmx::kResidentMost) + 1), at(new uint32_t[most + 1]) {}
+    void add(size_t i, bool there)  // without a branch on `there`
+    {
+        at[n] = (uint32_t)i;
+        n += there && n < most ? 1u : 0u;
+    }
+};
+
+// Whether four slots in a row, at any alignment, are empty.
+bool four_empty(const uint8_t *v)
+{
+    uint32_t q;
+    memcpy(&q, v, sizeof(q));
+    return q == 0;
+}
+
+bool four_empty(const uint32_t *v)
+{
+    uint64_t q[2];
+    memcpy(q, v, sizeof(q));
+    return (q[0] | q[1]) == 0;
+}
 
 // Row-major (x,y,z,p) -> native planes, inserting each nonzero particle at
 // the first empty slot of its site (RDMESolver::setLatticeData + addParticle;
 // IntLattice::setFromRowMajorData for the uint32 lattice).  rm holds N*P
 // elements of bpp bytes.
-// at, if given, receives the native site index of every particle, up to
-// listed_most of them.
-int row_major_to_native(const lmx_solver *s, const void *rm, std::vector<uint32_t> &native,
-                        std::vector<uint32_t> *at = nullptr)
+// at receives the particles' sites.
+int row_major_to_native(const lmx_solver *s, const void *rm, std::vector<uint32_t> &native, SiteList &at)
 {
     const size_t N = s->N;
     const bool words = s->bpp == 4;
     const uint8_t *rb = static_cast<const uint8_t *>(rm);
     const uint32_t *rw = static_cast<const uint32_t *>(rm);
     native.assign(N * s->W, 0u);
-    const size_t most = listed_most(s);
     size_t idx = 0;
     for (uint32_t x = 0; x < s->X; x++)
         for (uint32_t y = 0; y < s->Y; y++)
             for (uint32_t z = 0; z < s->Z; z++, idx += s->P) {
                 const size_t i = (size_t)x + (size_t)s->X * y + (size_t)s->X * s->Y * z;
                 uint32_t j = 0;  // the site's next slot
-                for (uint32_t l = 0; l < s->P; l++) {
-                    if (!words && (l & 3u) == 0) {  // four empty slots at once: most sites are empty
-                        uint32_t q;
-                        memcpy(&q, rb + idx + l, sizeof(q));
-                        if (q == 0) {
-                            l += 3;
-                            continue;
-                        }
+                for (uint32_t l = 0; l < s->P; l += 4) {  // most sites are empty
+                    if (words ? four_empty(rw + idx + l) : four_empty(rb + idx + l)) continue;
+                    for (uint32_t c = l; c < l + 4; c++) {
+                        const uint32_t v = words ? rw[idx + c] : rb[idx + c];
+                        if (v == 0) continue;
+                        if (v > s->nS) return fail(LMX_ERR_ARG, "latticeData: an invalid species was found: " + std::to_string(v));
+                        at.add(i, true);
+                        if (words)
+                            native[(size_t)j * N + i] = v;
+                        else
+                            native[(size_t)(j >> 2) * N + i] |= v << (8 * (j & 3));
+                        j++;
                     }
-                    const uint32_t v = words ? rw[idx + l] : rb[idx + l];
-                    if (v == 0) continue;
-                    if (v > s->nS) return fail(LMX_ERR_ARG, "latticeData: an invalid species was found: " + std::to_string(v));
-                    if (at && at->size() < most) at->push_back((uint32_t)i);
-                    if (words)
-                        native[(size_t)j * N + i] = v;
-                    else
-                        native[(size_t)(j >> 2) * N + i] |= v << (8 * (j & 3));
-                    j++;
                 }
             }
     return LMX_OK;
@@ -440,12 +458,12 @@ bool box_level_pays(const lmx_solver *s, uint32_t level)
 // particles: 50.6 -> 59.7; the capsule in 4096 boxes of 8: 23.7.  Nor are
 // boxes of a wave's worth of particles any shorter when smaller (64x64x64,
 // 2000 particles, 14 -> 4: 16.4 -> 20.0).
-void plan_boxes(lmx_solver *s, const std::vector<uint32_t> &at)
+void plan_boxes(lmx_solver *s, const SiteList &at)
 {
-    s->particles = at.size();
+    s->particles = at.n;
     s->resident_ok = s->d_res != nullptr;
     const uint32_t cap = (uint32_t)lmx::box_cap(s->P);
-    if (at.size() > s->N) return set_box_level(s, lmx::kBoxLevels);  // more than a particle a site: no box fits
+    if (at.n > s->N) return set_box_level(s, lmx::kBoxLevels);  // more than a particle a site: no box fits
     constexpr uint32_t kAtOnce = 1024u, kBoxesAtOnce = 3072u;  // boxes with particles, boxes
     constexpr uint32_t kShort = 64u;                           // particles that one wave moves at once
     std::vector<uint32_t> n, ybox(s->Y), zbox(s->Z);
@@ -454,20 +472,22 @@ void plan_boxes(lmx_solver *s, const std::vector<uint32_t> &at)
         const lmx::BoxGeom g = lmx::box_geom(s->X, s->Y, s->Z, lmx::kBoxLevel[level]);
         const double region = (double)(lmx::kBoxX + 2) * (g.TY + 2) * (g.TZ + 2) / ((double)lmx::kBoxX * g.TY * g.TZ);
         const double most = 0.75 * cap / region;
-        if ((double)at.size() > most * g.nboxes) continue;  // the mean box is too full already
+        if ((double)at.n > most * g.nboxes) continue;  // the mean box is too full already
+        if (fits == lmx::kBoxLevels && !box_level_pays(s, level)) continue;
         if (fits < lmx::kBoxLevels && g.nboxes > kBoxesAtOnce) break;
         for (uint32_t y = 0; y < s->Y; y++) ybox[y] = g.nbx * (y / g.TY);
         for (uint32_t z = 0; z < s->Z; z++) zbox[z] = g.nbx * g.nby * (z / g.TZ);
         n.assign(g.nboxes, 0u);
         uint32_t full = 0, active = 0;
-        for (uint32_t i : at) {
-            const uint32_t r = i / s->X, z = r / s->Y;
+        for (size_t q = 0; q < at.n; q++) {
+            const uint32_t i = at.at[q], r = i / s->X, z = r / s->Y;
             uint32_t &count = n[(i - r * s->X) / lmx::kBoxX + ybox[r - z * s->Y] + zbox[z]];
             active += count++ == 0u ? 1u : 0u;
             full = std::max(full, count);
+            if (full > most && fits == lmx::kBoxLevels) break;  // too full a box: the next level
         }
         if (fits < lmx::kBoxLevels && active > kAtOnce) break;
-        if (full <= most && (fits < lmx::kBoxLevels || box_level_pays(s, level))) fits = level;
+        if (full <= most) fits = level;
         if (fits < lmx::kBoxLevels && (active > kAtOnce || full <= kShort)) break;
     }
     set_box_level(s, fits);
@@ -1077,8 +1097,9 @@ int lmx_build_diffusion_model(lmx_solver *s, uint32_t nST, const double *DF, con
             if (q > 0.50f) return fail(LMX_ERR_ARG, "D: The specified diffusion coefficient is too high for the diffusion model.");
             s->T[i] = q;
         }
-        std::vector<uint32_t> native, at;
-        if ((rc = row_major_to_native(s, lattice, native, &at))) return rc;
+        std::vector<uint32_t> native;
+        SiteList at(s);
+        if ((rc = row_major_to_native(s, lattice, native, at))) return rc;
         std::vector<uint8_t> nsites;
         if ((rc = sites_row_major_to_native(s, sites, nsites))) return rc;
         compute_propensities(s);
@@ -1335,37 +1356,31 @@ int lmx_set_lattice_native(lmx_solver *s, const uint32_t *native, size_t words)
         int rc = require_ready(s);
         if (rc) return rc;
         if (!native || words != s->N * s->W) return fail(LMX_ERR_ARG, "the buffer size was not equal to the lattice data size");
-        for (size_t i = 0; i < words; i++) {
-            if (s->bpp == 4) {
-                if (native[i] > s->nS) return fail(LMX_ERR_ARG, "latticeData: an invalid species was found");
-                continue;
-            }
-            for (int b = 0; b < 4; b++)
-                if (((native[i] >> (8 * b)) & 0xFFu) > s->nS)
-                    return fail(LMX_ERR_ARG, "latticeData: an invalid species was found");
-        }
-        // Where the particles are, and whether every site holds its particles in
-        // its first slots.
+        // The species, where the particles are, and whether every site holds its
+        // particles in its first slots: a plane after the other, four words at a
+        // time where these are empty.
         bool packed = true;
-        std::vector<uint32_t> at;
-        const size_t most = listed_most(s);
-        for (size_t i = 0; i < s->N; i++) {
-            bool gap = false;
-            for (uint32_t j = 0; j < s->P; j++) {
-                const uint32_t word = s->bpp == 4 ? native[(size_t)j * s->N + i] : native[(size_t)(j >> 2) * s->N + i];
-                if (word == 0 && s->bpp == 1) {  // four empty slots
-                    gap = true;
-                    j |= 3u;
-                    continue;
-                }
-                const uint32_t v = s->bpp == 4 ? word : (word >> (8 * (j & 3))) & 0xFFu;
-                if (v == 0) {
-                    gap = true;
-                } else {
-                    if (gap) packed = false;
-                    if (at.size() < most) at.push_back((uint32_t)i);
+        SiteList at(s);
+        const size_t N = s->N;
+        const uint32_t per = s->bpp == 4 ? 1u : 4u;  // slots of a word
+        for (uint32_t k = 0; k < s->W; k++) {
+            const uint32_t *plane = native + k * N, *below = k ? plane - N : nullptr;
+            bool gaps = false, species = true;
+            for (size_t i0 = 0; i0 < N; i0 += 4) {
+                if (i0 + 4 <= N && four_empty(plane + i0)) continue;
+                for (size_t i = i0; i < std::min(i0 + 4, N); i++) {
+                    uint32_t before = !below ? 1u : (per == 1 ? below[i] : below[i] >> 24);  // the slot before
+                    for (uint32_t b = 0; b < per; b++) {
+                        const uint32_t v = per == 1 ? plane[i] : (plane[i] >> (8 * b)) & 0xFFu;
+                        species = species && v <= s->nS;
+                        gaps = gaps || (v != 0 && before == 0);
+                        at.add(i, v != 0);
+                        before = v;
+                    }
                 }
             }
+            if (!species) return fail(LMX_ERR_ARG, "latticeData: an invalid species was found");
+            packed = packed && !gaps;
         }
         LMX_HIP(hipStreamSynchronize(s->stream));
         LMX_HIP(hipMemcpy(s->d_lat[s->cur], native, words * sizeof(uint32_t), hipMemcpyHostToDevice));
@@ -1410,8 +1425,9 @@ int lmx_set_lattice(lmx_solver *s, const uint8_t *rm, size_t size)
         int rc = require_ready(s);
         if (rc) return rc;
         if (!rm || size != s->N * s->P * s->bpp) return fail(LMX_ERR_ARG, "bufferSize: the buffer size was not equal to the lattice data size");
-        std::vector<uint32_t> native, at;
-        if ((rc = row_major_to_native(s, rm, native, &at))) return rc;
+        std::vector<uint32_t> native;
+        SiteList at(s);
+        if ((rc = row_major_to_native(s, rm, native, at))) return rc;
         LMX_HIP(hipStreamSynchronize(s->stream));
         LMX_HIP(hipMemcpy(s->d_lat[s->cur], native.data(), native.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
         s->packed = true;  // each site's particles inserted at its first empty slot

@@ -402,3 +402,56 @@ def test_short_calls_of_more_particles_than_two_a_thread(lib, edge, n, steps, re
     ens.run(steps)
     assert any(l.startswith("resident") for l in log(lib)) == (steps >= 4)
     ens.close()
+
+
+@pytest.mark.parametrize("words", [False, True], ids=["byte", "uint32"])
+@pytest.mark.parametrize("shape", [(1, 1, 1), (3, 1, 1), (5, 3, 7), (8, 4, 6)])
+@pytest.mark.parametrize("P", [4, 8, 16])
+def test_host_lattice_writes(lib, shape, P, words):
+    """Row-major writes pack every site's particles in their order; native
+    writes stay as they are, and whether a site has an empty slot before an
+    occupied one, in one word or across words, is seen at every site; a
+    species that the model does not have is refused wherever it stands."""
+    rng = np.random.default_rng(P + len(shape))
+    spec = models.random_model(shape=shape, P=P, nS=5, nST=1, R=0, density=0.0, seed=1)
+    s = (lmx.IntMpdRdmeSolver if words else lmx.MpdRdmeSolver)(0)
+    if words:
+        spec.lattice = spec.lattice.astype(np.uint32)
+    spec.load_into(s, seed=1)
+    rm = np.where(rng.random(shape + (P,)) < 0.4, rng.integers(1, 6, shape + (P,)), 0).astype(spec.lattice.dtype)
+    packed = np.zeros_like(rm)
+    for at in np.ndindex(*shape):
+        v = rm[at][rm[at] != 0]
+        packed[at][:v.size] = v
+    s.setLattice(rm)
+    np.testing.assert_array_equal(s.getLattice(), packed)
+
+    def native(lattice):
+        z = lattice.transpose(2, 1, 0, 3)
+        w = z if words else np.ascontiguousarray(z).view(np.uint32)
+        return np.ascontiguousarray(np.moveaxis(w, 3, 0)).astype(np.uint32)
+
+    def first_step_reads_as_packed():
+        log(lib)
+        s.runTimesteps(1)
+        return "packed=1" in [l for l in log(lib) if l.startswith(("box", "sweep"))][0]
+
+    s.setLatticeNative(native(packed))
+    np.testing.assert_array_equal(s.getLatticeNative(), native(packed))
+    assert first_step_reads_as_packed()
+    for trial in range(8):
+        one = np.zeros_like(rm)
+        at = tuple(int(rng.integers(0, k)) for k in shape)
+        slot = int(rng.integers(1, P))
+        one[at][slot] = 3
+        one[at][:slot] = 1
+        s.setLatticeNative(native(one))
+        assert first_step_reads_as_packed()
+        one[at][int(rng.integers(0, slot))] = 0
+        s.setLatticeNative(native(one))
+        assert not first_step_reads_as_packed()
+        one[at][slot] = 6
+        for write, lattice in ((s.setLatticeNative, native(one)), (s.setLattice, one)):
+            with pytest.raises(lmx.InvalidArgException, match="invalid species"):
+                write(lattice)
+    s.close()
