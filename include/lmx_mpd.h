@@ -190,9 +190,9 @@ int lmx_autotune(lmx_solver *s, uint32_t nsteps, double *best_ms, int *chosen);
  * reported by the next lmx_synchronize.  Four or more steps of a solver of at
  * most 2048 particles without zero-order reactions run in one block in a
  * single launch, as do eight or more of at most 3000 (four on lattices of more
- * than 128^3 sites), unless the lattice is crowded; if the particles outgrow the block, the steps it left out run
- * (with a wait for the ones before them) in the next call that looks at the
- * state, uploads new rates or rebuilds the solver; calls that only enqueue
+ * than 128^3 sites); if the particles outgrow the block, the steps it left out
+ * run (with a wait for the ones before them) in the next call that looks at
+ * the state, uploads new rates or rebuilds the solver; calls that only enqueue
  * steps never wait for that. */
 int lmx_run_steps(lmx_solver *s, uint32_t nsteps);
 /* No counterpart in the reference: lmx_run_steps for callers that cannot

@@ -50,20 +50,6 @@ __device__ inline uint32_t site_occupancy(const Params &p, const uint32_t *lat, 
     return occ;
 }
 
-// A particle into slot occ (the site's first empty slot) of site s.
-__device__ inline void place_particle(const Params &p, uint32_t *lat, uint32_t s, uint32_t occ, uint32_t particle)
-{
-    clear_zero_flag(p, p.word_particles ? occ : occ >> 2, s);
-    if (p.word_particles) {
-        store_agent(lat + (size_t)occ * p.N + s, particle);
-    } else {
-        uint32_t *wp = lat + (size_t)(occ >> 2) * p.N + s;
-        const uint32_t old = load_agent(wp);
-        store_agent(wp, old | (particle << (8 * (occ & 3))));
-        if ((occ >> 2) > 0) clear_chunk_flag(p, lat, occ >> 2, s >> 2);
-    }
-}
-
 __device__ inline void set_error(Control *ctl, uint32_t code, uint32_t step)
 {
     if (atomicCAS(&ctl->error, 0u, code) == 0u) ctl->error_step = step;
@@ -92,38 +78,67 @@ constexpr Ball make_ball()
 }
 static __constant__ const Ball kBall = make_ball();
 
+// LDS of the resolver's block beside the sorted keys.
 template <int kThreads>
-__device__ inline void resolve_body(const Params &p, uint32_t *lat)
+struct ResolveLds {
+    static constexpr int kRound = kThreads / 64;  // entries searched at once
+    uint32_t parts[64], f_site[kRound], f_slot[kRound], f_room[kRound], placed, failure;
+};
+
+// What the resolver looks up and changes: the sites of a lattice in device
+// memory.
+struct LatticeSites {
+    const Params &p;
+    uint32_t *lat;
+
+    // The first empty slot of site s | the empty slots in a row from there << 8.
+    __device__ inline uint32_t look(bool in, uint32_t s) const
+    {
+        const uint32_t slots = p.word_particles ? 1u : 4u;
+        uint32_t slot = 0, room = 0;
+#pragma unroll 1
+        for (uint32_t k0 = 0; k0 < p.W; k0 += 2u) {
+            uint32_t word[2];
+#pragma unroll
+            for (int k = 0; k < 2; k++)
+                word[k] = in && k0 + k < p.W ? load_agent(lat + (size_t)(k0 + k) * p.N + s) : ~0u;
+#pragma unroll
+            for (int k = 0; k < 2; k++)
+                for (uint32_t b = 0; b < slots; b++) {
+                    const bool empty = slots == 1u ? word[k] == 0u : (word[k] >> (8u * b) & 0xFFu) == 0u;
+                    // (a taken slot after the first empty one ends the row)
+                    if (empty && slot + room == (k0 + k) * slots + b) room++;
+                    else if (!empty && room == 0u) slot++;
+                }
+        }
+        return slot | room << 8;
+    }
+    // A particle into an empty slot; several lanes may fill one word.
+    __device__ inline void place(uint32_t s, uint32_t slot, uint32_t particle) const
+    {
+        clear_zero_flag(p, p.word_particles ? slot : slot >> 2, s);
+        if (p.word_particles) {
+            store_agent(lat + (size_t)slot * p.N + s, particle);
+        } else {
+            __hip_atomic_store(reinterpret_cast<uint8_t *>(lat + (size_t)(slot >> 2) * p.N + s) + (slot & 3u),
+                               (uint8_t)particle, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if ((slot >> 2) > 0) clear_chunk_flag(p, lat, slot >> 2, s >> 2);
+        }
+    }
+    __device__ inline uint32_t occupancy(uint32_t s) const { return site_occupancy(p, lat, s); }
+};
+
+// Places a step's n entries (at most kMaxOverflows, with the carried ones);
+// key0 and part0: entry threadIdx.x & 63.  All threads of the block call it.
+// On thread 0 it returns how many entries stay listed.
+template <int kThreads, class Sites>
+__device__ inline uint32_t resolve_entries(const Params &p, const Sites &sites, unsigned long long *keys,
+                                           ResolveLds<kThreads> &sh, uint32_t n, uint32_t carried, uint32_t t,
+                                           unsigned long long key0, uint32_t part0)
 {
-    constexpr int kRound = kThreads / 64;  // entries searched at once
-    __shared__ unsigned long long keys[kMaxOverflows];
-    __shared__ uint32_t parts[64], s_t, f_site[kRound], f_slot[kRound], f_room[kRound], placed, failure;
+    constexpr int kRound = ResolveLds<kThreads>::kRound;
     Control *ctl = p.ctl;
     const int tid = threadIdx.x;
-    if (tid == 0) s_t = ctl->timestep;
-    // A few entries are read along with their number.
-    const uint32_t n = load_agent(&ctl->ovf_count);
-    const unsigned long long key0 =
-        __hip_atomic_load(&ctl->ovf_keys[tid & 63], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const uint32_t part0 = load_agent(&ctl->ovf_part[tid & 63]);
-    __syncthreads();
-    // The step's reaction phase has consumed the reaction list.
-    for (int k = tid; k < kListShards; k += kThreads) ctl->list_count[k] = 0u;
-    if (tid == 0) ctl->list_overflow = 0u;
-    const uint32_t t = s_t;
-    const uint32_t carried = p.relaxed ? ctl->carry_count : 0u;
-    if (n == 0 && carried == 0) {
-        if (tid == 0) ctl->timestep = t + 1;
-        return;
-    }
-    if (n > kMaxOverflows || carried + n > kMaxOverflows) {
-        if (tid == 0) {
-            set_error(ctl, kErrOverflowCap, t);
-            ctl->ovf_count = 0;
-            ctl->timestep = t + 1;
-        }
-        return;
-    }
     if (n <= 64u) {
         // Entry k's rank is the number of smaller keys (no two are equal).
         uint32_t rank = 0;
@@ -134,7 +149,7 @@ __device__ inline void resolve_body(const Params &p, uint32_t *lat)
         }
         if (tid < (int)n) {
             keys[rank] = key0;
-            parts[rank] = part0;
+            sh.parts[rank] = part0;
         }
         __syncthreads();
     } else {
@@ -160,49 +175,59 @@ __device__ inline void resolve_body(const Params &p, uint32_t *lat)
         }
     }
 
+    const uint32_t X = p.X, Y = p.Y, Z = p.Z, lane = tid & 63, wave = tid >> 6;
     if (p.relaxed) {
         // Relaxed handler (correct_overflows, MpdRdmeSolver.cu:1677-1761): the
         // carried entries, then this step's in canonical order, each into its
         // own site's first empty slot; entries of one site go in that order
-        // (the kernel's rounds) and different sites do not interact, so one
-        // thread walks the list.  A full site keeps the entry for the next step.
-        if (tid == 0) {
-            uint32_t kept = 0;
-            for (uint32_t e = 0; e < carried + n; e++) {
-                uint32_t site, particle;
-                if (e < carried) {
-                    site = ctl->carry_site[e];
-                    particle = ctl->carry_part[e];
-                } else {
-                    const unsigned long long key = keys[e - carried];
-                    site = (uint32_t)((key >> 24) & 0xFFFFFFFFull);
-                    particle = load_agent(&ctl->ovf_part[key & 0x7FFull]);
-                }
-                const uint32_t occ = site_occupancy(p, lat, site);
-                if (occ < p.P) {
-                    place_particle(p, lat, site, occ, particle);
-                } else {
-                    ctl->carry_site[kept] = site;  // kept <= e: entry e has been read
-                    ctl->carry_part[kept] = particle;
-                    kept++;
-                }
+        // (the kernel's rounds) and different sites do not interact.  So a wave
+        // takes 64 of them at a time: an entry's slot is its site's occupancy
+        // and the chunk's earlier entries of that site, which all fit if it
+        // does.  A full site keeps the entry for the next step.
+        uint32_t kept = 0;
+        if (wave != 0) return 0;
+        for (uint32_t e0 = 0; e0 < carried + n; e0 += 64u) {
+            const uint32_t e = e0 + lane;
+            const bool have = e < carried + n;
+            uint32_t site = ~0u, particle = 0;
+            if (e < carried) {
+                site = load_agent(&ctl->carry_site[e]);
+                particle = load_agent(&ctl->carry_part[e]);
+            } else if (have) {
+                const unsigned long long key = keys[e - carried];
+                site = (uint32_t)((key >> 24) & 0xFFFFFFFFull);
+                particle = load_agent(&ctl->ovf_part[key & 0x7FFull]);
             }
+            uint32_t slot = have ? sites.occupancy(site) : p.P;
+#pragma unroll 1
+            for (uint32_t q = 0; q < 63u; q++)
+                slot += q < lane && (uint32_t)__builtin_amdgcn_readlane((int)site, (int)q) == site ? 1u : 0u;
+            const bool fits = slot < p.P;
+            if (fits) sites.place(site, slot, particle);
+            const unsigned long long stay = __ballot(have && !fits);
+            if (have && !fits) {  // (at its own place or before: those have been read)
+                const uint32_t k = kept + __builtin_amdgcn_mbcnt_hi((uint32_t)(stay >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)stay, 0u));
+                store_agent(&ctl->carry_site[k], site);
+                store_agent(&ctl->carry_part[k], particle);
+            }
+            kept += (uint32_t)__popcll(stay);
+            wait_for_stores();  // the next chunk's loads see them
+        }
+        if (lane == 0) {
             ctl->carry_count = kept;
             ctl->ovf_total += n;
             if (n > 0) ctl->ovf_steps += 1;
             ctl->ovf_count = 0;
-            ctl->timestep = t + 1;
         }
-        return;
+        return kept;
     }
 
-    const uint32_t X = p.X, Y = p.Y, Z = p.Z, lane = tid & 63, wave = tid >> 6;
     for (uint32_t e0 = 0; e0 < n;) {
         const uint32_t e = e0 + wave;
-        // room: empty slots in a row from f_slot on; 0: no candidate has one,
+        // room: empty slots in a row from sh.f_slot on; 0: no candidate has one,
         // kOut: the search leaves the lattice first.
         constexpr uint32_t kOut = 0xFFu;
-        if (lane == 0u) f_room[wave] = 0u;
+        if (lane == 0u) sh.f_room[wave] = 0u;
         if (e < n) {
             const uint32_t site = (uint32_t)((keys[e] >> 24) & 0xFFFFFFFFull);
             const uint32_t st0 = p.sites[site], xc = site % X, yc = (site / X) % Y, zc = site / p.XY;
@@ -222,29 +247,14 @@ __device__ inline void resolve_body(const Params &p, uint32_t *lat)
                                     !((ox && X - 1 >= R) || (oy && Y - 1 >= R) || (oz && Z - 1 >= R));
                 const bool out = listed && (ox || oy || oz), in = listed && !out;
                 const uint32_t s = in ? x + X * y + p.XY * z : site;
-                const uint32_t type = p.sites[s], slots = p.word_particles ? 1u : 4u;
-                uint32_t slot = 0, room = 0;
-#pragma unroll 1
-                for (uint32_t k0 = 0; k0 < p.W; k0 += 2u) {
-                    uint32_t word[2];
-#pragma unroll
-                    for (int k = 0; k < 2; k++)
-                        word[k] = in && k0 + k < p.W ? load_agent(lat + (size_t)(k0 + k) * p.N + s) : ~0u;
-#pragma unroll
-                    for (int k = 0; k < 2; k++)
-                        for (uint32_t b = 0; b < slots; b++) {
-                            const bool empty = slots == 1u ? word[k] == 0u : (word[k] >> (8u * b) & 0xFFu) == 0u;
-                            // (a taken slot after the first empty one ends the row)
-                            if (empty && slot + room == (k0 + k) * slots + b) room++;
-                            else if (!empty && room == 0u) slot++;
-                        }
-                }
+                const uint32_t type = p.sites[s];
+                const uint32_t seen = sites.look(in, s), slot = seen & 255u, room = seen >> 8;
                 const unsigned long long m = __ballot(out || (in && room != 0u && type == st0));
                 if (m == 0ull) continue;
                 if (lane == (uint32_t)__builtin_ctzll(m)) {
-                    f_site[wave] = s;
-                    f_slot[wave] = slot;
-                    f_room[wave] = out ? kOut : room;
+                    sh.f_site[wave] = s;
+                    sh.f_slot[wave] = slot;
+                    sh.f_room[wave] = out ? kOut : room;
                 }
                 break;
             }
@@ -254,13 +264,13 @@ __device__ inline void resolve_body(const Params &p, uint32_t *lat)
             const uint32_t count = n - e0 < (uint32_t)kRound ? n - e0 : (uint32_t)kRound;
             uint32_t sl = 0, se = 0, particle = 0, room = 1;
             if (lane < count) {
-                particle = n <= 64u ? parts[e0 + lane] : load_agent(&ctl->ovf_part[keys[e0 + lane] & 0x7FFull]);
-                se = f_site[lane];
-                sl = f_slot[lane];
-                room = f_room[lane];
+                particle = n <= 64u ? sh.parts[e0 + lane] : load_agent(&ctl->ovf_part[keys[e0 + lane] & 0x7FFull]);
+                se = sh.f_site[lane];
+                sl = sh.f_slot[lane];
+                room = sh.f_room[lane];
                 if (room != 0u && room != kOut)
                     for (uint32_t q = 0; q < lane; q++)
-                        if (f_site[q] == se) {
+                        if (sh.f_site[q] == se) {
                             sl++;
                             room--;
                             if (room == 0u) break;
@@ -270,36 +280,60 @@ __device__ inline void resolve_body(const Params &p, uint32_t *lat)
             // whose site the earlier ones of the round filled.
             const unsigned long long stop = __ballot(lane < count && (room == 0u || room == kOut));
             const uint32_t upto = stop ? (uint32_t)__builtin_ctzll(stop) : count;
-            if (lane < upto) {
-                clear_zero_flag(p, p.word_particles ? sl : sl >> 2, se);
-                if (p.word_particles) {
-                    store_agent(lat + (size_t)sl * p.N + se, particle);
-                } else {  // a byte: two entries may fill one word
-                    __hip_atomic_store(reinterpret_cast<uint8_t *>(lat + (size_t)(sl >> 2) * p.N + se) + (sl & 3u),
-                                       (uint8_t)particle, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    if ((sl >> 2) > 0) clear_chunk_flag(p, lat, sl >> 2, se >> 2);
-                }
-            }
+            if (lane < upto) sites.place(se, sl, particle);
             if (lane == upto || (upto == 64u && lane == 0u)) {
-                placed = upto;
-                const uint32_t r = upto < count ? f_room[upto] : 1u;
-                failure = r == 0u ? kErrUnplaceable : (r == kOut ? kErrOutOfRange : 0u);
+                sh.placed = upto;
+                const uint32_t r = upto < count ? sh.f_room[upto] : 1u;
+                sh.failure = r == 0u ? kErrUnplaceable : (r == kOut ? kErrOutOfRange : 0u);
             }
             wait_for_stores();  // the next round's loads see the stores
         }
         __syncthreads();
-        if (failure != 0u) {
-            if (tid == 0) set_error(ctl, failure, t);
+        if (sh.failure != 0u) {
+            if (tid == 0) set_error(ctl, sh.failure, t);
             break;
         }
-        e0 += placed;
+        e0 += sh.placed;
     }
     if (tid == 0) {
         atomicAdd(&ctl->ovf_total, (unsigned long long)n);
         atomicAdd(&ctl->ovf_steps, 1ull);
         ctl->ovf_count = 0;
-        ctl->timestep = t + 1;
     }
+    return 0;
+}
+
+// The overflow entries of a step on the lattice that it wrote, and the end of
+// the step: the reaction list's counters cleared, the step counter advanced.
+template <int kThreads>
+__device__ inline void resolve_body(const Params &p, uint32_t *lat)
+{
+    __shared__ unsigned long long keys[kMaxOverflows];
+    __shared__ ResolveLds<kThreads> sh;
+    __shared__ uint32_t s_t;
+    Control *ctl = p.ctl;
+    const int tid = threadIdx.x;
+    if (tid == 0) s_t = ctl->timestep;
+    // A few entries are read along with their number.
+    const uint32_t n = load_agent(&ctl->ovf_count);
+    const unsigned long long key0 =
+        __hip_atomic_load(&ctl->ovf_keys[tid & 63], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const uint32_t part0 = load_agent(&ctl->ovf_part[tid & 63]);
+    __syncthreads();
+    // The step's reaction phase has consumed the reaction list.
+    for (int k = tid; k < kListShards; k += kThreads) ctl->list_count[k] = 0u;
+    if (tid == 0) ctl->list_overflow = 0u;
+    const uint32_t t = s_t;
+    const uint32_t carried = p.relaxed ? ctl->carry_count : 0u;
+    if (n > kMaxOverflows || carried + n > kMaxOverflows) {
+        if (tid == 0) {
+            set_error(ctl, kErrOverflowCap, t);
+            ctl->ovf_count = 0;
+        }
+    } else if (n != 0 || carried != 0) {
+        resolve_entries<kThreads>(p, LatticeSites{p, lat}, keys, sh, n, carried, t, key0, part0);
+    }
+    if (tid == 0) ctl->timestep = t + 1;
 }
 
 }  // namespace lmx

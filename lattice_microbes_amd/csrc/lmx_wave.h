@@ -1,7 +1,9 @@
-// A reaction at one site, evaluated by a whole wave: a slot of the site per
+// Reactions of a wave's sites, shared by the boxed step's reaction launch and
+// the resident runs: a lane per site sums propensities (packed_propensity), and
+// a site that reacts is taken by the whole wave (wave_products), a slot per
 // lane to count and evaluate, a reaction per lane to select.  Loops over slots
 // are rolled, so that sites of 16 slots cost no more registers than those of
-// four.  Shared by the boxed step's reaction launch and the resident runs.
+// four.
 #pragma once
 
 #include "lmx_device.h"
@@ -13,6 +15,45 @@ __device__ inline uint32_t lane_id() { return __builtin_amdgcn_mbcnt_hi(~0u, __b
 __device__ inline uint32_t lane_of(uint32_t v, uint32_t src)
 {
     return (uint32_t)__builtin_amdgcn_readlane((int)v, (int)src);
+}
+
+// total_propensity's sum for a site of `count` particles in its first slots:
+// the same terms in the same order, a row of up to 8 pairs loaded at a time.
+// slots: the wave's copy of its sites' slots, slot-major, for this lane (a
+// slot's index is not known at compile time).
+template <uint32_t P, class Slot>
+__device__ inline float packed_propensity(const Params &p, uint32_t st, const Slot (*slots)[64], uint32_t lane,
+                                          uint32_t count)
+{
+    constexpr uint32_t kRow = P < 8u ? P : 8u;
+    float a = p.qp0[st];
+#pragma unroll 1
+    for (uint32_t m = 0; m < count; m++) {
+        const uint32_t row = st * p.nS + slots[m][lane] - 1u;
+        const float one = p.qp1[row];
+        const float *pairs = p.qp2 + (size_t)row * p.nS;
+        uint32_t n = m + 1u;
+        float v[kRow];
+        auto load = [&] {
+#pragma unroll
+            for (uint32_t k = 0; k < kRow; k++) {
+                const uint32_t q = n + k < count ? n + k : m;
+                v[k] = pairs[slots[q][lane] - 1u];
+            }
+        };
+        load();
+        a += one;
+#pragma unroll 1
+        for (;;) {
+#pragma unroll
+            for (uint32_t k = 0; k < kRow; k++)
+                if (n + k < count) a += v[k];
+            n += kRow;
+            if (n >= count) break;
+            load();
+        }
+    }
+    return a;
 }
 
 // Which reaction happens at site si (type sst, total propensity a) and the

@@ -637,45 +637,6 @@ __global__ __launch_bounds__(kBoxThreads, OCC) void box_jobs_kernel(const BoxJob
 // us, 256x256x128 uint32 lattice 21 -> 13.4, crowded P = 16 26 -> 15.4.
 // ---------------------------------------------------------------------------
 
-// total_propensity's sum for a site of `count` particles in its first slots:
-// the same terms in the same order, a row of up to 8 pairs loaded at a time.
-// slots: the wave's copy of its sites' slots, slot-major, for this lane (a
-// slot's index is not known at compile time).
-template <uint32_t P>
-__device__ inline float packed_propensity(const Params &p, uint32_t st, const uint32_t (*slots)[64], uint32_t lane,
-                                          uint32_t count)
-{
-    constexpr uint32_t kRow = P < 8u ? P : 8u;
-    float a = p.qp0[st];
-#pragma unroll 1
-    for (uint32_t m = 0; m < count; m++) {
-        const uint32_t row = st * p.nS + slots[m][lane] - 1u;
-        const float one = p.qp1[row];
-        const float *pairs = p.qp2 + (size_t)row * p.nS;
-        uint32_t n = m + 1u;
-        float v[kRow];
-        auto load = [&] {
-#pragma unroll
-            for (uint32_t k = 0; k < kRow; k++) {
-                const uint32_t q = n + k < count ? n + k : m;
-                v[k] = pairs[slots[q][lane] - 1u];
-            }
-        };
-        load();
-        a += one;
-#pragma unroll 1
-        for (;;) {
-#pragma unroll
-            for (uint32_t k = 0; k < kRow; k++)
-                if (n + k < count) a += v[k];
-            n += kRow;
-            if (n >= count) break;
-            load();
-        }
-    }
-    return a;
-}
-
 // A reaction at lane src's site i (propensity a, words w), by the whole wave.
 // Every lane of the wave calls it, with its own site's values.
 template <class L>

@@ -743,23 +743,12 @@ uint32_t resident_min_steps(const lmx_solver *s, bool alone)
     return alone && s->particles > 2u * lmx::kResidentThreads && s->N <= 1u << 21 ? 8u : 4u;
 }
 
-// Whether the sites of a lattice hold so many particles that its overflow
-// entries and sites of many particles, which a resident run takes one after
-// another, make it slower than the launches.  us a step, in one block against
-// sweeps: 4 slots 10^3 sites, 2000 particles 161/56, 16^3 3000 30/53;  8 slots
-// 10^3 2000 23/33, 3000 55/42, 8^3 3000 507/215;  16 slots 8^3 3000 68/195.
-bool crowded(const lmx_solver *s)
-{
-    const size_t most = s->P == 16 ? 6 : s->P / 4;  // particles a site
-    return s->particles > most * s->N;
-}
-
 // A solver of few particles runs in one block: the default options, no
 // zero-order reactions (they would need every empty site).  The bimolecular
 // 64^3 model (2000 particles) takes 16.5 us a step in boxes, 10.9 in one block.
 bool use_resident(const lmx_solver *s, uint32_t nsteps, bool alone)
 {
-    return nsteps >= resident_min_steps(s, alone) && s->resident_ok && s->particles <= lmx::kResidentMost && !crowded(s) && !s->any_qp0 &&
+    return nsteps >= resident_min_steps(s, alone) && s->resident_ok && s->particles <= lmx::kResidentMost && !s->any_qp0 &&
            s->boxes && s->path == LMX_PATH_SWEEPS && s->yz_kernel == 0 && s->fuse_reaction && !s->force_generic;
 }
 

@@ -28,6 +28,7 @@
 #include "lmx_device.h"
 #include "lmx_kernels.h"
 #include "lmx_resident.h"
+#include "lmx_resolve.h"
 #include "lmx_wave.h"
 
 namespace lmx {
@@ -39,7 +40,6 @@ constexpr uint32_t kChains = 8192u;      // two per record at least: most chains
 constexpr uint32_t kEnd = 0xFFFFu, kDead = 0xFFFFFFFFu;
 constexpr uint32_t kIdBits = 13u;        // of a chain head: the particle; the sweep's tag above
 constexpr uint32_t kTab = 2048u;         // floats of the model's tables kept in LDS
-constexpr uint32_t kBall = 729u;         // sites within distance 4 along each axis
 
 // key: x | y << 10 | z << 20.  ord: slot (4), class (2: stayed, from the minus,
 // from the plus neighbour), site type (8), species (16).
@@ -57,9 +57,8 @@ struct ResidentLds {
     uint16_t next[2][kCap];
     uint32_t head[2][kChains];
     float tab[kTab];
-    uint32_t occ[kBall];            // particles of the sites around an overflow entry
-    unsigned long long best;
-    uint32_t n[2], nc, ovf, spill, pick;  // records; sites to evaluate; ...
+    ResolveLds<(int)kNT> resolve;
+    uint32_t n[2], nc, ovf, spill;  // records; sites to evaluate; ...
 };
 
 __device__ inline uint32_t site_of(const Params &p, uint32_t key)
@@ -99,7 +98,7 @@ __device__ inline void chain_rank(const ResidentLds &s, int g, uint32_t e, uint3
 // One more particle at the end of generation 0; past the block's capacity it
 // goes into the (otherwise empty) lattice and the run ends after this step.
 template <class L>
-__device__ inline void append(const Params &p, uint32_t *lat, ResidentLds &s, uint32_t key, uint32_t ord)
+__device__ inline uint32_t append(const Params &p, uint32_t *lat, ResidentLds &s, uint32_t key, uint32_t ord)
 {
     const uint32_t k = atomicAdd(&s.n[0], 1u);
     if (k < kCap) {
@@ -109,6 +108,7 @@ __device__ inline void append(const Params &p, uint32_t *lat, ResidentLds &s, ui
         s.spill = 1u;
         put_particle<L>(p, lat, site_of(p, key), ord & 15u, ord_species(ord));
     }
+    return k;
 }
 
 // Whether a site of several particles with total propensity a reacts
@@ -122,13 +122,13 @@ __device__ inline bool reacts(float a, float u)
     return prob > 0.0f && u <= prob;
 }
 
-// The site of record e, by a wave: its total propensity a, or, if known is
-// set, its reaction.  The site's particles (the members of its chain in
-// generation 1 that fit) lie a slot per lane; a reaction's result goes back as
-// records of generation 0 -- in the members' places, further ones appended.
+// The reaction of record e's site (total propensity a), by a wave.  The site's
+// particles (the members of its chain in generation 1 that fit) lie a slot per
+// lane; the result goes back as records of generation 0 -- in the members'
+// places, further ones appended.
 template <class L>
-__device__ inline void react_site_wave(const Params &p, uint32_t *lat, ResidentLds &s, uint32_t e, bool known, float a,
-                                       uint32_t t, unsigned long long h3)
+__device__ inline void react_site_wave(const Params &p, uint32_t *lat, ResidentLds &s, uint32_t e, float a, uint32_t t,
+                                       unsigned long long h3)
 {
     constexpr uint32_t P = L::P;
     const uint32_t lane = lane_id(), key = s.key[1][e], type = ord_type(s.ord[1][e]);
@@ -141,25 +141,8 @@ __device__ inline void react_site_wave(const Params &p, uint32_t *lat, ResidentL
             rec = q;
         }
     }
-    const uint32_t i = site_of(p, key);
-    if (!known) {
-        // total_propensity's sum: the same terms in the same order, a
-        // particle's row of them a lane each.
-        const uint32_t count = (uint32_t)__popcll(__ballot(mine != 0u));
-        a = p.qp0[type];
-#pragma unroll 1
-        for (uint32_t m = 0; m < count; m++) {
-            const uint32_t row = type * p.nS + lane_of(mine, m) - 1u;
-            float v = 0.0f;
-            if (lane == m) v = p.qp1[row];
-            else if (lane > m && lane < count) v = p.qp2[(size_t)row * p.nS + (mine - 1u)];
-#pragma unroll 1
-            for (uint32_t n = m; n < count; n++) a += __uint_as_float(lane_of(__float_as_uint(v), n));
-        }
-        if (!reacts(a, uniform01(i, 1, 0, h3))) return;
-    }
     bool underflow;
-    const uint32_t now = wave_products<P>(p, i, type, mine, a, h3, underflow);
+    const uint32_t now = wave_products<P>(p, site_of(p, key), type, mine, a, h3, underflow);
     if (underflow && lane == 0u && atomicCAS(&p.ctl->error, 0u, kErrReactionUnderflow) == 0u) p.ctl->error_step = t;
     if (lane >= P) return;
     // products without a slot are overflow entries: only a full site has any
@@ -200,13 +183,15 @@ __device__ inline float few_propensity(const Params &p, uint32_t type, const uin
 }
 
 // The nc sites listed in s.next[0], whose particles are several or whose one
-// passed its test.  A lane per site sums the propensities of up to kFew
-// particles; the sites that react, and those of more particles, are taken by
-// the whole wave.  Latency bounds it where the sites are few, so that one wave
-// takes up to 32 of them (32^3, 2000 particles, 60 sites: 10.2 us a step, dealt
-// to sixteen waves 10.7), and issue where they are many (16^3, 2000 particles:
-// 12.0, in one wave 15.6).  kFew: 12^3, 2500 particles 14.7 us a step, with 4
-// of them 16.3.
+// passed its test.  A lane per site sums its propensities, and a site that
+// reacts is taken by the whole wave.  Latency bounds it where the sites are few,
+// so that one wave takes up to 32 of them (32^3, 2000 particles, 60 sites: 10.2
+// us a step, dealt to sixteen waves 10.7), and issue where they are many (16^3,
+// 2000 particles: 12.0, in one wave 15.6).  Sites of up to kFew particles keep
+// these in registers and their terms in flight together (8 slots: 64 crowded
+// sites in 32^3 19.7 us a step, with six in registers 25.5), fuller ones in LDS,
+// a row of terms at a time (16 slots, 100 sites of 14 particles: 73 us, by a
+// wave each 148).
 //
 // A thread per site for everything, with the site's slots in registers,
 // unrolls the evaluation over every slot: with 16 of them 40 VGPRs and 138
@@ -216,29 +201,35 @@ template <class L>
 __device__ inline void react_sites(const Params &p, uint32_t *lat, ResidentLds &s, uint32_t nc, uint32_t t,
                                    unsigned long long h3, const float2 *tab)
 {
-    constexpr uint32_t kFew = L::P < 6 ? L::P : 6;
+    constexpr uint32_t P = L::P, kFew = P <= 8 ? P : 6;
     const uint32_t waves = nc <= 32u ? 1u : (nc >= 512u ? 16u : (nc + 31u) / 32u);
-    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = lane_id();
     if (wave >= waves) return;
+    // Slots of the fuller sites: this wave's part of the chain heads of
+    // generation 0, free until the next y sweep, which finds them zero.
+    static_assert(sizeof(s.head[0]) >= kNT / 64u * P * 64u * sizeof(uint16_t), "room for the slots");
+    uint16_t (*slots)[64] = reinterpret_cast<uint16_t (*)[64]>(&s.head[0][0]) + wave * P;
 #pragma unroll 1
     for (uint32_t k0 = 0; k0 < nc; k0 += 64u * waves) {
-        const uint32_t k = k0 + lane_id() * waves + wave;
+        const uint32_t k = k0 + lane * waves + wave;
         uint32_t e = 0, count = 0, type = 0, sp[kFew] = {};
         float a = 0.0f, u = 1.0f;
         bool hit = false;
+        auto members = [&](auto &&with) {  // slot and species of each of the site's particles
+            const uint32_t key = s.key[1][e];
+            for (uint32_t q = s.head[1][chain_of(key)] & ((1u << kIdBits) - 1u); q != kEnd; q = s.next[1][q])
+                if (s.key[1][q] == key && s.key[0][q] != kDead) with(s.ord[0][q] & 15u, ord_species(s.ord[0][q]));
+        };
         if (k < nc) {
             e = s.next[0][k];
-            const uint32_t key = s.key[1][e];
             type = ord_type(s.ord[1][e]);
-            for (uint32_t q = s.head[1][chain_of(key)] & ((1u << kIdBits) - 1u); q != kEnd; q = s.next[1][q]) {
-                if (s.key[1][q] != key || s.key[0][q] == kDead) continue;
-                const uint32_t o = s.ord[0][q], j = o & 15u;
+            members([&](uint32_t j, uint32_t species) {
                 count++;
 #pragma unroll
                 for (uint32_t m = 0; m < kFew; m++)
-                    if (j == m) sp[m] = ord_species(o);
-            }
-            u = uniform01(site_of(p, key), 1, 0, h3);
+                    if (j == m) sp[m] = species;
+            });
+            u = uniform01(site_of(p, s.key[1][e]), 1, 0, h3);
         }
         const bool pairs = __ballot(count > 2u && count <= kFew) == 0ull;  // no site of three and more
         if (count == 1u) {
@@ -249,152 +240,102 @@ __device__ inline void react_sites(const Params &p, uint32_t *lat, ResidentLds &
             a = pairs ? few_propensity<2>(p, type, sp, count) : few_propensity<kFew>(p, type, sp, count);
             hit = reacts(a, u);
         }
+        if (kFew < P && __ballot(count > kFew) != 0ull) {
+            if (count > kFew) {
+                members([&](uint32_t j, uint32_t species) { slots[j][lane] = (uint16_t)species; });
+                a = packed_propensity<P>(p, type, slots, lane, count);
+                hit = reacts(a, u);
+            }
+            for (uint32_t m = lane; m < P * 32u; m += 64u) reinterpret_cast<uint32_t *>(slots)[m] = 0u;
+        }
 #pragma unroll 1
-        for (unsigned long long m = __ballot(hit || count > kFew); m; m &= m - 1) {
+        for (unsigned long long m = __ballot(hit); m; m &= m - 1) {
             const uint32_t src = (uint32_t)__builtin_ctzll(m);
-            react_site_wave<L>(p, lat, s, lane_of(e, src), lane_of(count, src) <= kFew,
-                               __uint_as_float(lane_of(__float_as_uint(a), src)), t, h3);
+            react_site_wave<L>(p, lat, s, lane_of(e, src), __uint_as_float(lane_of(__float_as_uint(a), src)), t, h3);
         }
     }
 }
 
-__device__ inline uint32_t agent_load(const uint32_t *q)
-{
-    return __hip_atomic_load(q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// The step's overflow entries into sites with room (resolve_kernel's rules,
-// on the records of generation 0): in canonical order, each entry scans the
-// candidate sites of growing radius.  All threads call it; rare.
+// What the resolver looks up and changes here: the particles on the chains of
+// generation 1 (sweep tag `tag`), those past the block's capacity in the
+// lattice.
 template <class L>
-__device__ void resolve_records(const Params &p, uint32_t *lat, ResidentLds &s, uint32_t t)
+struct ResidentSites {
+    const Params &p;
+    uint32_t *lat;
+    ResidentLds &s;
+    uint32_t tag;
+
+    __device__ inline uint32_t key_of(uint32_t i) const
+    {
+        const uint32_t r = i / p.X, z = r / p.Y;
+        return (i - r * p.X) | ((r - z * p.Y) << 10) | (z << 20);
+    }
+    // Record k of generation 0 joins its site's chain.
+    __device__ inline void link(uint32_t k) const
+    {
+        const uint32_t key = s.key[0][k], old = atomicExch(&s.head[1][chain_of(key)], k | (tag << kIdBits));
+        s.key[1][k] = key;
+        s.next[1][k] = (uint16_t)((old >> kIdBits) == tag ? old & ((1u << kIdBits) - 1u) : kEnd);
+    }
+    __device__ inline uint32_t occupancy(uint32_t i) const
+    {
+        const uint32_t key = key_of(i), hd = s.head[1][chain_of(key)];
+        uint32_t count = 0;
+        for (uint32_t q = (hd >> kIdBits) == tag ? hd & ((1u << kIdBits) - 1u) : kEnd; q != kEnd; q = s.next[1][q])
+            count += s.key[1][q] == key && s.key[0][q] != kDead ? 1u : 0u;
+        if (s.spill)
+            for (uint32_t k = 0; k < (uint32_t)L::W; k++) {
+                const uint32_t v = load_agent(lat + (size_t)k * p.N + i);
+                for (int b = 0; b < L::kPerWord; b++) count += L::part(v, b) != 0u ? 1u : 0u;
+            }
+        return count;
+    }
+    __device__ inline uint32_t look(bool in, uint32_t i) const
+    {
+        const uint32_t count = in ? occupancy(i) : (uint32_t)L::P;
+        return count | ((uint32_t)L::P - count) << 8;
+    }
+    __device__ inline void place(uint32_t i, uint32_t slot, uint32_t particle) const
+    {
+        const uint32_t k = append<L>(p, lat, s, key_of(i), make_ord(slot, 0u, p.nST > 1u ? p.sites[i] : 0u, particle));
+        if (k < kCap) link(k);
+        else __threadfence();
+    }
+};
+
+// The overflow entries of step t into sites with room; n: records before the
+// reactions.  All threads call it.
+template <class L>
+__device__ inline void resolve_records(const Params &p, uint32_t *lat, ResidentLds &s, uint32_t t, uint32_t n, uint32_t tag)
 {
-    constexpr uint32_t P = L::P;
     Control *ctl = p.ctl;
     const uint32_t tid = threadIdx.x;
-    __threadfence();
+    const ResidentSites<L> sites{p, lat, s, tag};
+    __threadfence();  // entries, and particles past the block's capacity
     __syncthreads();
-    const uint32_t n = agent_load(&ctl->ovf_count);
-    const uint32_t carried = p.relaxed ? agent_load(&ctl->carry_count) : 0u;
+    const uint32_t found = load_agent(&ctl->ovf_count), carried = p.relaxed ? load_agent(&ctl->carry_count) : 0u;
+    const unsigned long long key0 =
+        __hip_atomic_load(&ctl->ovf_keys[tid & 63], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const uint32_t part0 = load_agent(&ctl->ovf_part[tid & 63]);
+    for (uint32_t k = n + tid; k < s.n[0] && k < kCap; k += kNT) sites.link(k);  // (appended by the reactions)
     __syncthreads();
-    if (n > kMaxOverflows || carried + n > kMaxOverflows) {
+    uint32_t kept = carried;
+    if (found > kMaxOverflows || carried + found > kMaxOverflows) {
         if (tid == 0) {
-            if (atomicCAS(&ctl->error, 0u, kErrOverflowCap) == 0u) ctl->error_step = t;
+            set_error(ctl, kErrOverflowCap, t);
             ctl->ovf_count = 0u;
         }
-        __threadfence();
+    } else if (found != 0u || carried != 0u) {
+        // The keys take the chain heads of generation 0, free until the next
+        // y sweep, which finds them zero.
+        static_assert(sizeof(s.head[0]) >= kMaxOverflows * sizeof(unsigned long long), "room for the keys");
+        kept = resolve_entries<(int)kNT>(p, sites, reinterpret_cast<unsigned long long *>(&s.head[0][0]), s.resolve, found,
+                                         carried, t, key0, part0);
         __syncthreads();
-        return;
+        for (uint32_t k = tid; k < 2u * kMaxOverflows; k += kNT) s.head[0][k] = 0u;
     }
-    unsigned long long last = 0ull;
-    bool any = false, failed = false;
-    uint32_t kept = 0;
-    for (uint32_t e = 0; e < carried + n && !failed; e++) {
-        uint32_t site, particle;
-        if (e < carried) {
-            site = agent_load(&ctl->carry_site[e]);
-            particle = agent_load(&ctl->carry_part[e]);
-        } else {
-            // the smallest key above the last one
-            if (tid == 0) s.best = ~0ull;
-            __syncthreads();
-            for (uint32_t k = tid; k < n; k += kNT) {
-                const unsigned long long v = __hip_atomic_load(&ctl->ovf_keys[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                if (!any || v > last) atomicMin(&s.best, v);
-            }
-            __syncthreads();
-            last = s.best;
-            any = true;
-            __syncthreads();
-            site = (uint32_t)((last >> 24) & 0xFFFFFFFFull);
-            particle = agent_load(&ctl->ovf_part[last & 0x7FFull]);
-        }
-        const uint32_t xc = site % p.X, yc = (site / p.X) % p.Y, zc = site / p.XY;
-        // particles of every site within distance 4 of it
-        for (uint32_t k = tid; k < kBall; k += kNT) s.occ[k] = 0u;
-        __syncthreads();
-        const uint32_t m = s.n[0] < kCap ? s.n[0] : kCap;
-        for (uint32_t k = tid; k < m; k += kNT) {
-            const uint32_t key = s.key[0][k];
-            if (key == kDead) continue;
-            const uint32_t dx = (key & 1023u) + 4u - xc, dy = ((key >> 10) & 1023u) + 4u - yc, dz = (key >> 20) + 4u - zc;
-            if (dx <= 8u && dy <= 8u && dz <= 8u) atomicAdd(&s.occ[dx + 9u * (dy + 9u * dz)], 1u);
-        }
-        __syncthreads();
-        if (s.spill) {  // and those past the block's capacity
-            for (uint32_t k = tid; k < kBall; k += kNT) {
-                const uint32_t x = xc + k % 9u - 4u, y = yc + (k / 9u) % 9u - 4u, z = zc + k / 81u - 4u;
-                if (x >= p.X || y >= p.Y || z >= p.Z) continue;
-                for (uint32_t q = 0; q < p.W; q++) {
-                    const uint32_t v = agent_load(lat + (size_t)q * p.N + x + p.X * y + p.XY * z);
-                    for (uint32_t b = 0; b < 4u; b++)
-                        s.occ[k] += p.word_particles ? (b == 0u && v ? 1u : 0u) : (((v >> (8u * b)) & 0xFFu) ? 1u : 0u);
-                }
-            }
-            __syncthreads();
-        }
-        auto occupancy = [&](uint32_t x, uint32_t y, uint32_t z) {
-            return s.occ[(x + 4u - xc) + 9u * ((y + 4u - yc) + 9u * (z + 4u - zc))];
-        };
-        const uint32_t st0 = p.sites[site];
-        if (p.relaxed) {
-            // its own site, or it stays listed
-            const uint32_t occ = occupancy(xc, yc, zc);
-            __syncthreads();
-            if (tid == 0) {
-                if (occ < P) {
-                    append<L>(p, lat, s, xc | (yc << 10) | (zc << 20), make_ord(occ, 0u, st0, particle));
-                } else {
-                    __hip_atomic_store(&ctl->carry_site[kept], site, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    __hip_atomic_store(&ctl->carry_part[kept], particle, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                }
-            }
-            if (occ >= P) kept++;
-            __threadfence();
-            __syncthreads();
-            continue;
-        }
-        int found = 0x7fffffff;
-        for (uint32_t R = 0; R <= kMaxReplacementDist && found == 0x7fffffff; R++) {
-            const uint32_t minD = R > 0 ? R - 1 : 0, X = p.X, Y = p.Y, Z = p.Z;
-            const uint32_t x0 = xc >= R ? xc - R : 0, x1 = (xc <= X - 1 - R) ? xc + R : X - 1;
-            const uint32_t y0 = yc >= R ? yc - R : 0, y1 = (yc <= Y - 1 - R) ? yc + R : Y - 1;
-            const uint32_t z0 = zc >= R ? zc - R : 0, z1 = (zc <= Z - 1 - R) ? zc + R : Z - 1;
-            const uint32_t ny = y1 - y0 + 1, nz = z1 - z0 + 1, all = (x1 - x0 + 1) * ny * nz;  // at most 729
-            if (tid == 0) s.pick = 0x7fffffffu;
-            __syncthreads();
-            uint32_t x = 0, y = 0, z = 0;
-            if (tid < all) {
-                x = x0 + tid / (ny * nz);
-                const uint32_t rem = tid % (ny * nz);
-                y = y0 + rem / nz;
-                z = z0 + rem % nz;
-                const long long dx = (long long)x - xc, dy = (long long)y - yc, dz = (long long)z - zc;
-                const long long r2 = dx * dx + dy * dy + dz * dz;
-                if (r2 <= (long long)(R * R) && (r2 > (long long)(minD * minD) || R == 0)) {
-                    if (x >= X || y >= Y || z >= Z) atomicMin(&s.pick, 2u * tid + 1u);
-                    else if (p.sites[x + X * y + p.XY * z] == st0 && occupancy(x, y, z) < P) atomicMin(&s.pick, 2u * tid);
-                }
-            }
-            __syncthreads();
-            found = (int)s.pick;
-            if (found != 0x7fffffff && !(found & 1) && tid == (uint32_t)found >> 1)
-                append<L>(p, lat, s, x | (y << 10) | (z << 20), make_ord(occupancy(x, y, z), 0u, st0, particle));
-            __syncthreads();
-        }
-        if (found == 0x7fffffff || (found & 1)) {
-            if (tid == 0 && atomicCAS(&ctl->error, 0u, found & 1 && found != 0x7fffffff ? kErrOutOfRange : kErrUnplaceable) == 0u)
-                ctl->error_step = t;
-            failed = true;
-        }
-    }
-    if (tid == 0) {
-        if (p.relaxed) ctl->carry_count = kept;
-        ctl->ovf_total += n;
-        if (n > 0) ctl->ovf_steps += 1;
-        ctl->ovf_count = 0u;
-        s.ovf = p.relaxed && kept ? 1u : 0u;
-    }
+    if (tid == 0) s.ovf = p.relaxed && kept ? 1u : 0u;
     __threadfence();
     __syncthreads();
 }
@@ -409,7 +350,7 @@ __device__ inline void gather_body(const ResidentJob &job, uint32_t block, uint3
 {
     constexpr int W = L::W;
     const Params &p = job.p;
-    if (agent_load(&p.ctl->timestep) != job.start) return;
+    if (load_agent(&p.ctl->timestep) != job.start) return;
     uint32_t *lat = job.lat;
     const bool by4 = (p.N & 3u) == 0u;
     const uint32_t items = by4 ? p.N >> 2 : p.N;
@@ -505,8 +446,8 @@ __device__ __attribute__((always_inline)) inline void run_body(const ResidentJob
     Control *ctl = p.ctl;
     uint32_t *lat = job.lat;
     const uint32_t tid = threadIdx.x;
-    if (agent_load(&ctl->timestep) != job.start) return;
-    const uint32_t found = agent_load(job.count);
+    if (load_agent(&ctl->timestep) != job.start) return;
+    const uint32_t found = load_agent(job.count);
     const bool periodic = p.boundary == 0;
 
     for (uint32_t k = tid; k < 2u * kChains; k += kNT) (&s.head[0][0])[k] = 0u;
@@ -529,7 +470,7 @@ __device__ __attribute__((always_inline)) inline void run_body(const ResidentJob
     if (tid == 0) {
         s.n[0] = found < kCap ? found : kCap;
         s.n[1] = 0u;
-        s.ovf = p.relaxed && agent_load(&ctl->carry_count) ? 1u : 0u;
+        s.ovf = p.relaxed && load_agent(&ctl->carry_count) ? 1u : 0u;
         s.spill = s.nc = 0u;
     }
     for (uint32_t k = tid; k < found && k < kCap; k += kNT) {
@@ -663,7 +604,7 @@ __device__ __attribute__((always_inline)) inline void run_body(const ResidentJob
                 __syncthreads();
                 if (tid == 0) s.nc = 0u;
             }
-            if (s.ovf) resolve_records<L>(p, lat, s, t);
+            if (s.ovf) resolve_records<L>(p, lat, s, t, n, tag + 3u);
         }
     }
 

@@ -371,21 +371,6 @@ def test_crowded_lattices_step_in_what_is_faster(lib, shape, P, density, spot, w
     s.close()
 
 
-@pytest.mark.parametrize("P,n,resident", [(4, 1000, True), (4, 1001, False), (8, 2000, True), (8, 2001, False),
-                                          (16, 3000, True)])
-def test_crowded_lattices_are_not_run_in_one_block(lib, P, n, resident):
-    spec = models.random_model(shape=(10, 10, 10), P=P, nS=3, nST=1, R=0, density=0.0, seed=1)
-    spec.lattice = np.zeros(1000 * P, np.uint8)
-    spec.lattice[np.random.default_rng(1).permutation(1000 * P)[:n]] = 1
-    spec.lattice = spec.lattice.reshape(10, 10, 10, P)
-    s = lmx.MpdRdmeSolver(0)
-    spec.load_into(s, seed=1)
-    log(lib)
-    s.runTimesteps(8)
-    assert any(l.startswith("resident") for l in log(lib)) == resident
-    s.close()
-
-
 @pytest.mark.parametrize("edge,n,steps,resident", [(64, 2048, 3, False), (64, 2048, 4, True), (64, 2049, 7, False),
                                                    (64, 2049, 8, True), (160, 2049, 4, True)])
 def test_short_calls_of_more_particles_than_two_a_thread(lib, edge, n, steps, resident):
