@@ -1544,8 +1544,9 @@ __device__ inline void reaction_list_body(const Params &p, uint32_t *__restrict_
 
 // At most 128 VGPRs: four waves per SIMD to hide the table and lattice
 // latencies (measured 33 against 36 us with the compiler's 135).  P = 16 needs
-// 206 and takes two waves: held to 128 it spilled 121 VGPRs next to 387 SGPRs
-// and gave wrong sites.
+// 206 and takes two waves: held to 128 it spills 121 VGPRs next to 387 SGPRs
+// (320 bytes of scratch a lane), and an earlier text of react_apply gave wrong
+// sites that way.
 template <int W>
 __global__ __launch_bounds__(256, W == 4 ? 2 : 4) void reaction_list_kernel(Params p, uint32_t *__restrict__ lat, ReactionList rl,
                                                             uint32_t nshards)

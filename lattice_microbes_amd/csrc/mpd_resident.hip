@@ -21,10 +21,11 @@
 // ensemble runs a member per CU: 128 replicates on 32^3 to 128^3 sites take
 // 14.6 us a step against 970 us for the batched sweeps.
 //
-// What bounds it: a step is 28,000 cycles, 5,000 to 7,000 for each of the four
-// rounds (vector issue: two records per thread, about 200 instructions each
-// with the hash's quarter-rate multiplies, sixteen waves on four SIMDs) and
-// 5,000 for the sites to evaluate (latency of one wave's evaluation).
+// What bounds it (64^3, rocprofv3): a step is 26,250 cycles, at least 13,490 of them
+// vector issue (13,490 instructions on four SIMDs, four cycles and more each: two
+// records a thread in each of four rounds, with the hash's quarter-rate
+// multiplies), the rest latency of dependent LDS accesses between five
+// barriers.
 #include "lmx_device.h"
 #include "lmx_kernels.h"
 #include "lmx_resident.h"
