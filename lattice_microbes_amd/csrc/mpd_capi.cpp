@@ -277,7 +277,7 @@ lmx::Params make_params(const lmx_solver *s)
     return p;
 }
 
-int settle(lmx_solver *s);
+int settle(lmx_solver *s, bool *ran = nullptr);
 
 int require_built(lmx_solver *s)
 {
@@ -802,8 +802,8 @@ int enqueue_steps(lmx_solver *s, uint32_t nsteps, const lmx::ReactionList *rl = 
 // A resident run stops short when its block is full (the particles multiplied,
 // or a caller put more of them into the device's lattice); the runs enqueued
 // after it then did nothing.  The steps that are missing run here in the
-// ordinary way, before anything else looks at the state.
-int settle(lmx_solver *s)
+// ordinary way, before anything else looks at the state; ran: there were some.
+int settle(lmx_solver *s, bool *ran)
 {
     if (!s->res_pending) return LMX_OK;
     if (int rc = select_device(s)) return rc;
@@ -818,6 +818,7 @@ int settle(lmx_solver *s)
     const uint32_t missing = s->timestep - t;
     s->timestep = t;
     s->resident_ok = false;
+    if (ran) *ran = true;
     return enqueue_steps(s, missing);
 }
 
@@ -1678,6 +1679,13 @@ int lmx_time_steps(lmx_solver *s, uint32_t nsteps, double *total_ms, double *ker
         }
         LMX_HIP(hipEventRecord(t1, s->stream));
         LMX_HIP(hipEventSynchronize(t1));
+        // Steps that a resident run left out belong to the time.
+        bool more = false;
+        if ((rc = settle(s, &more))) return rc;
+        if (more) {
+            LMX_HIP(hipEventRecord(t1, s->stream));
+            LMX_HIP(hipEventSynchronize(t1));
+        }
         float ms = 0.0f;
         LMX_HIP(hipEventElapsedTime(&ms, t0, t1));
         if (total_ms) *total_ms = ms;
@@ -2110,6 +2118,22 @@ int batch_enqueue_step(lmx_batch *b)
     return LMX_OK;
 }
 
+// Records the end of a timed run once it has ended; steps that members'
+// resident runs left out belong to the time.
+int batch_timed(lmx_batch *b, hipEvent_t end)
+{
+    LMX_HIP(hipEventRecord(end, b->stream));
+    LMX_HIP(hipEventSynchronize(end));
+    bool more = false;
+    for (lmx_solver *s : b->members)
+        if (int rc = settle(s, &more)) return rc;
+    if (!more) return LMX_OK;
+    for (lmx_solver *s : b->members) LMX_HIP(hipStreamSynchronize(s->stream));
+    LMX_HIP(hipEventRecord(end, b->stream));
+    LMX_HIP(hipEventSynchronize(end));
+    return LMX_OK;
+}
+
 int batch_capture(lmx_batch *b)
 {
     if (b->exec && b->graph_members == b->stepped && std::memcmp(b->graph_total, b->total, sizeof(b->total)) == 0)
@@ -2426,8 +2450,7 @@ int lmx_batch_autotune(lmx_batch *b, uint32_t nsteps, double *best_ms, int *chos
                 if ((rc = lmx_batch_run_steps(b, 1))) break;  // untimed first step (captures the graph)
                 LMX_HIP(hipEventRecord(e0, b->stream));
                 if ((rc = lmx_batch_run_steps(b, timed))) break;
-                LMX_HIP(hipEventRecord(e1, b->stream));
-                LMX_HIP(hipEventSynchronize(e1));
+                if ((rc = batch_timed(b, e1))) break;
                 float ms = 0.0f;
                 LMX_HIP(hipEventElapsedTime(&ms, e0, e1));
                 const double per = (double)ms / timed;
@@ -2470,8 +2493,8 @@ int lmx_batch_time_steps(lmx_batch *b, uint32_t nsteps, double *total_ms)
             LMX_HIP(hipStreamSynchronize(b->stream));
             LMX_HIP(hipEventRecord(t0, b->stream));
             rc = lmx_batch_run_steps(b, nsteps);
-            LMX_HIP(hipEventRecord(t1, b->stream));
-            LMX_HIP(hipEventSynchronize(t1));
+            const int rc2 = batch_timed(b, t1);
+            if (!rc) rc = rc2;
             float ms = 0.0f;
             LMX_HIP(hipEventElapsedTime(&ms, t0, t1));
             *total_ms = ms;

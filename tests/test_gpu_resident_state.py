@@ -262,3 +262,23 @@ def test_overflow_entries_of_resident_runs(gpu, P, spot, density, handler, words
         assert s.getUnresolvedOverflows() == orc.unresolved
     assert orc.stats.overflow_entries > 20
     s.close()
+
+
+def test_timed_runs_that_outgrow_the_block(gpu):
+    """lmx_time_steps and the ensemble's, whose time includes the steps made up."""
+    spec = _splitting(2040, 3000.0)
+    pairs = []
+    for k in range(2):
+        s = lmx.MpdRdmeSolver(0)
+        spec.load_into(s, replicate=k, seed=3)
+        pairs.append((s, oracle.Oracle(spec, seed_top=3, replicate=k)))
+    assert pairs[0][0].timeSteps(9)[0] > 0
+    assert pairs[0][1].run(9) == 0
+    ens = lmx.Ensemble(0)
+    for s, _ in pairs:
+        ens.add(s)
+    assert ens.time_steps(8) > 0
+    for s, orc in pairs:
+        assert orc.run(8) == 0
+        assert np.array_equal(s.getLatticeNative(), orc.native()) and s.timestep == orc.timestep
+    ens.close()

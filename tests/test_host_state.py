@@ -440,3 +440,27 @@ def test_host_lattice_writes(lib, shape, P, words):
             with pytest.raises(lmx.InvalidArgException, match="invalid species"):
                 write(lattice)
     s.close()
+
+
+def test_timed_steps_include_those_a_resident_run_left_out(lib):
+    spec, s = small()
+    for kind, ms in dict(resident=1, box=16).items():
+        lib.standin_cost(kind.encode(), float(ms))
+    assert s.timeSteps(6)[0] == pytest.approx(6.0)
+    lib.standin_resident_limit(2)
+    assert s.timeSteps(6)[0] == pytest.approx(2 * 1.0 + 4 * 16.0)
+    assert s.timestep == 12
+    s.close()
+
+
+def test_timed_batch_steps_include_those_a_resident_run_left_out(lib):
+    ens = lmx.Ensemble(0, graph=False)
+    members = [small()[1] for _ in range(2)]
+    for s in members:
+        ens.add(s)
+    for kind, ms in dict(resident=1, box=16).items():
+        lib.standin_cost(kind.encode(), float(ms))
+    lib.standin_resident_limit(2)
+    assert ens.time_steps(6) == pytest.approx(2 * (2 * 1.0 + 4 * 16.0))
+    assert [s.timestep for s in members] == [6, 6]
+    ens.close()
