@@ -1,5 +1,6 @@
-// Overflow resolution on the device, shared by the resolver kernels and by the
-// boxed step's reaction launch, whose last block resolves.
+// Overflow resolution on the device, shared by the resolver kernels, the boxed
+// step's reaction launch, whose last block resolves, and the resident runs,
+// which resolve among a block's records.
 #pragma once
 
 #include "lmx_device.h"
@@ -16,10 +17,11 @@ namespace lmx {
 //
 // What it costs is the latency of the searches, so every wave searches for an
 // entry of its own, a lane per candidate in list order (the first 64
-// candidates, radius 2 and a third of radius 3, nearly always suffice).  They are committed in order: particles
-// only fill sites, so a search made before the earlier entries of its round
-// were placed is still right unless they filled the very site it found; from
-// the first such entry on the round is searched again.
+// candidates, radius 2 and a third of radius 3, nearly always suffice).  They
+// are committed in order: particles only fill sites, so a search made before
+// the earlier entries of its round were placed is still right unless they
+// filled the very site it found; from the first such entry on the round is
+// searched again.
 // ---------------------------------------------------------------------------
 __device__ inline uint32_t load_agent(const uint32_t *ptr)
 {
